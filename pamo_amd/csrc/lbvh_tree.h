@@ -148,13 +148,55 @@ static int tree_refit(Tree& t, int n, hipStream_t st) {
     return tree_boxes(t, n, true, st);
 }
 
+// Child-pair records for nearest-item walks: both children's boxes of internal
+// node i in one hop, the left child's in pre[2i], pre[2i + 1] and the right
+// child's in suf[2i], suf[2i + 1], with the child in the lo box's w: an
+// internal node's number, or ~item for a leaf.  A walk step is then one
+// round of independent loads; over the node records it is the children's
+// numbers first and their boxes after.  The records take the place of the
+// in-block prefix and suffix boxes, which only a (re)fit reads and rewrites.
+__global__ void __launch_bounds__(kB) child_pairs_k(const float4* __restrict__ box, const int* __restrict__ left,
+                                                    const int* __restrict__ right, const uint32_t* __restrict__ val,
+                                                    int n, float4* __restrict__ pre, float4* __restrict__ suf) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n - 1) return;
+    const int l = left[i], r = right[i];
+    float4 a = box[2 * (long long)l], c = box[2 * (long long)r];
+    a.w = __int_as_float(l >= n - 1 ? ~(int)val[l - (n - 1)] : l);
+    c.w = __int_as_float(r >= n - 1 ? ~(int)val[r - (n - 1)] : r);
+    pre[2 * (long long)i] = a;
+    pre[2 * (long long)i + 1] = box[2 * (long long)l + 1];
+    suf[2 * (long long)i] = c;
+    suf[2 * (long long)i + 1] = box[2 * (long long)r + 1];
+}
+
+// Writes the child-pair records of a built tree (again after each refit).
+static int tree_pairs(Tree& t, hipStream_t st) {
+    if (t.n < 2) return 0;
+    hipLaunchKernelGGL(child_pairs_k, dim3(grid_for(t.n - 1, kB)), dim3(kB), 0, st, (const float4*)t.box,
+                       (const int*)t.left, (const int*)t.right, (const uint32_t*)t.val, t.n, t.pre, t.suf);
+    PAMO_HIP(hipGetLastError());
+    return 0;
+}
+
+// Nearest-item walks keep the far children still to visit on a stack in LDS,
+// one column a lane (entry k of the wave's lanes at [k][lane]: no bank
+// conflicts).  kNearStack entries cover the trees of real meshes (one
+// entry a level at most: about log2 of the items, and a few more where the
+// mesh is graded); a lane that runs out finishes by the parent links.  One wave
+// a block: 12 KiB, so that 13 waves stay on a compute unit.
+constexpr int kNearStack = 24;
+
 struct TreeView {
     int n;
     const float4* box;
     const int *left, *right, *parent;
     const uint32_t* val;
+    const float4 *pre, *suf;  // child-pair records (tree_pairs)
 };
-static TreeView view(const Tree& t) { return TreeView{t.n, t.box, t.left, t.right, t.parent, t.val}; }
+static TreeView view(const Tree& t) {
+    return TreeView{t.n, t.box, t.left, t.right, t.parent, t.val, t.pre, t.suf};
+}
 
 __device__ __forceinline__ bool box_hit(V3 lo, V3 hi, float4 blo, float4 bhi) {
     return !(hi.x < blo.x || bhi.x < lo.x || hi.y < blo.y || bhi.y < lo.y || hi.z < blo.z || bhi.z < lo.z);

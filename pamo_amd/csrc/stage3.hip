@@ -294,11 +294,15 @@ __global__ void edge_items_k(const float4* __restrict__ x, const int2* __restric
 
 // ------------------------------------------------------------ closest point on the input surface (B4)
 // Nearest triangle by branch and bound over the GT tree: nearer child first,
-// subtrees whose box is no closer than the best distance so far skipped.
-__global__ void __launch_bounds__(kB) closest_point_k(const float4* __restrict__ x, int nV, TreeView T,
-                                                     const float4* __restrict__ gv, const int4* __restrict__ gf,
-                                                     float4* __restrict__ target, int* err) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
+// subtrees whose box is no closer than the best distance so far skipped, over
+// the tree's child-pair records with the far children on an LDS stack.
+__global__ void __launch_bounds__(kWave) closest_point_k(const float4* __restrict__ x, int nV, TreeView T,
+                                                        const float4* __restrict__ gv, const int4* __restrict__ gf,
+                                                        float4* __restrict__ target, int* err) {
+    __shared__ int stk_n[kNearStack][kWave];
+    __shared__ float stk_d[kNearStack][kWave];
+    const int lane = threadIdx.x;
+    const int i = blockIdx.x * kWave + lane;
     if (i >= nV) return;
     const V3 p = v3(x[i]);
     float best = 1e18f;  // squared; query radius 1e9
@@ -316,35 +320,77 @@ __global__ void __launch_bounds__(kB) closest_point_k(const float4* __restrict__
     if (n == 1) {
         leaf((int)T.val[0]);
     } else if (n > 1) {
-        int cur = 0, prev = -1;
-        const long long max_steps = 3LL * (2LL * n - 1) + 1;
-        for (long long steps = 0; cur >= 0; ++steps) {
-            if (steps >= max_steps || cur > 2 * n - 2) {
+        bool dropped = false;
+        int cur = 0, sp = 0;  // cur: internal node, ~face, or n when the stack is to be popped
+        for (long long steps = 0;; ++steps) {
+            if (steps >= 4LL * n) {  // every node at most once, every pop at most once
                 walk_overrun(err);
                 break;
             }
-            const int par = cur == 0 ? -1 : T.parent[cur];
-            int next;
-            if (prev == par) {
-                if (box_dist2(p, T.box[2 * (long long)cur], T.box[2 * (long long)cur + 1]) >= best) next = par;
-                else if (cur >= n - 1) {
-                    leaf((int)T.val[cur - (n - 1)]);
-                    next = par;
+            if (cur >= n - 1) {
+                if (sp == 0) break;
+                --sp;
+                cur = stk_d[sp][lane] >= best ? n : stk_n[sp][lane];
+                continue;
+            }
+            if (cur < 0) {
+                leaf(~cur);
+                cur = n;
+                continue;
+            }
+            const float4 la = T.pre[2 * (long long)cur], lb = T.pre[2 * (long long)cur + 1];
+            const float4 ra = T.suf[2 * (long long)cur], rb = T.suf[2 * (long long)cur + 1];
+            const float dl = box_dist2(p, la, lb), dr = box_dist2(p, ra, rb);
+            const bool left_first = dl <= dr;
+            const float dn = left_first ? dl : dr, df = left_first ? dr : dl;
+            const int cn = __float_as_int(left_first ? la.w : ra.w), cf = __float_as_int(left_first ? ra.w : la.w);
+            if (!(df >= best)) {
+                if (sp < kNearStack) {
+                    stk_d[sp][lane] = df;
+                    stk_n[sp][lane] = cf;
+                    ++sp;
+                } else {
+                    dropped = true;
+                }
+            }
+            cur = dn >= best ? n : cn;
+        }
+        if (dropped) {
+            // the stack ran out: the whole tree once more by parent links, from the start (so that among
+            // equally near points the first in the order of the visits is kept, as without the stack)
+            best = 1e18f;
+            bestp = mk(1e9f, 1e9f, 1e9f);
+            int prev = -1;
+            cur = 0;
+            const long long max_steps = 3LL * (2LL * n - 1) + 1;
+            for (long long steps = 0; cur >= 0; ++steps) {
+                if (steps >= max_steps || cur > 2 * n - 2) {
+                    walk_overrun(err);
+                    break;
+                }
+                const int par = cur == 0 ? -1 : T.parent[cur];
+                int next;
+                if (prev == par) {
+                    if (box_dist2(p, T.box[2 * (long long)cur], T.box[2 * (long long)cur + 1]) >= best) next = par;
+                    else if (cur >= n - 1) {
+                        leaf((int)T.val[cur - (n - 1)]);
+                        next = par;
+                    } else {
+                        int l = T.left[cur], r = T.right[cur];
+                        float dl = box_dist2(p, T.box[2 * (long long)l], T.box[2 * (long long)l + 1]);
+                        float dr = box_dist2(p, T.box[2 * (long long)r], T.box[2 * (long long)r + 1]);
+                        next = dl <= dr ? l : r;
+                    }
                 } else {
                     int l = T.left[cur], r = T.right[cur];
                     float dl = box_dist2(p, T.box[2 * (long long)l], T.box[2 * (long long)l + 1]);
                     float dr = box_dist2(p, T.box[2 * (long long)r], T.box[2 * (long long)r + 1]);
-                    next = dl <= dr ? l : r;
+                    int first = dl <= dr ? l : r, second = dl <= dr ? r : l;
+                    next = prev == first ? second : par;
                 }
-            } else {
-                int l = T.left[cur], r = T.right[cur];
-                float dl = box_dist2(p, T.box[2 * (long long)l], T.box[2 * (long long)l + 1]);
-                float dr = box_dist2(p, T.box[2 * (long long)r], T.box[2 * (long long)r + 1]);
-                int first = dl <= dr ? l : r, second = dl <= dr ? r : l;
-                next = prev == first ? second : par;
+                prev = cur;
+                cur = next;
             }
-            prev = cur;
-            cur = next;
         }
     }
     target[i] = f4(bestp);
@@ -1683,8 +1729,9 @@ static int detect_contacts(Ctx& c, int& nC) {
 
 static int update_target(Ctx& c) {
     if (c.P.mask & PAMO_S3_E_M2GT)
-        L3(closest_point_k, c.nV, (const float4*)c.q, c.nV, view(c.gt_tree), (const float4*)c.gt_v,
-           (const int4*)c.gt_f, c.target, c.ccount + 1);
+        hipLaunchKernelGGL(closest_point_k, dim3(grid_for(c.nV, kWave)), dim3(kWave), 0, c.stream, (const float4*)c.q,
+                           c.nV, view(c.gt_tree), (const float4*)c.gt_v, (const int4*)c.gt_f, c.target, c.ccount + 1);
+    PAMO_HIP(hipGetLastError());
     return 0;
 }
 
@@ -2217,6 +2264,7 @@ int pamo_s3_set_target(pamo_s3* s, const float* d_gt_v, int n_gt_v, const int* d
                        (const float4*)c.gt_v, (const int4*)c.gt_f, n_gt_f, 0.0f, c.gt_tree.item);
     PAMO_HIP(hipGetLastError());
     PAMO_TRY(pamo::s3::tree_build(c.gt_tree, n_gt_f, c.ws, c.stream));
+    PAMO_TRY(pamo::s3::tree_pairs(c.gt_tree, c.stream));
     PAMO_HIP(hipStreamSynchronize(c.stream));
     return 0;
 }
