@@ -653,13 +653,16 @@ def main():
         v3, f3 = pm.stage3_in
         Vs, Fs = float(len(v3)), float(len(f3))
         Es = 1.5 * Fs
-        n_nt, K, A = float(st3["newton"]), float(st3["contacts"]), float(pm.system.active_contacts())
+        # (the iterations that repeat a fixed point are counted by the statistics, not run and not priced)
+        n_nt = float(pm.system.newton_run())
+        K, A = (x * n_nt / max(st3["newton"], 1) for x in (float(st3["contacts"]), float(pm.system.active_contacts())))
         per_newton = (40 * (160 * Vs + 32 * Fs + 24 * Es) + 11 * (28 * Vs + 32 * Fs + 24 * Es)
                       + (52 * Vs + 32 * Fs + 24 * Es) + (12 * Vs + 24 * Fs + 24 * Es))
         B3 = n_nt * per_newton + K * (20 + 10 * 4 + 16) + A * (40 * 68 + 10 * 20 + 68) + 5 * 24 * Vs
     path_ach = (B2 + B3) / per_step / 1e9
     path_roofline = {"bound": "hbm", "achieved": round(path_ach, 2), "peak": 8000.0, "unit": "GB/s",
                      "frac": round(path_ach / 8000.0, 5), "stage2_bytes": round(B2), "stage3_bytes": round(B3),
+                     "stage3_newton_run": int(n_nt) if use_s3 else 0,
                      "model": "stage 2: sum_r 231 F_r + 128 V_r (V_r = F_r / 2; the 80 C_r guard-pair term not "
                               "counted); stage 3 per Newton iteration: 40 CG passes over the active contacts A, "
                               "one full and ten line-search energy passes, the gradient pass and the detection "

@@ -279,7 +279,10 @@ int pamo_s3_merge_vertices(pamo_s3* s3, const float* d_v, int n_v, int* d_f, int
 
 /* n_steps calls of Stage3System.step (system.py:411-470): closest-point
  * targets, then n_newton_iters of {contacts, gradient, Jacobi PCG, clamp,
- * ACCD, halving line search}. */
+ * ACCD, halving line search}.  An iteration that leaves every vertex where it
+ * was, bit for bit, is a fixed point: the iterations that would repeat it are
+ * counted and not run (pamo_s3_step_eval runs them all; the positions are the
+ * same). */
 int pamo_s3_step(pamo_s3* s3, int n_steps);
 /* Replaces Stage3System.step(eval=True, ...) (system.py:411-470): one step,
  * calling on_newton(newton_iter, user) after each Newton iteration once its
@@ -330,6 +333,10 @@ int pamo_s3_stats(pamo_s3* s3, double* out8);
  * gradient pass and the CG products touch (measurement; no counterpart in
  * the reference). */
 int pamo_s3_active_contacts(pamo_s3* s3, long long* total);
+/* Newton iterations run since the mesh was set; the statistics above count
+ * the ones that repeat a fixed point too (measurement; no counterpart in the
+ * reference). */
+int pamo_s3_newton_run(pamo_s3* s3, long long* total);
 
 /* Run-time options (no counterpart in the reference's interface, which
  * fixes its CUDA-graph capture of the PCG loop in config.py:21).

@@ -332,6 +332,13 @@ class Stage3System:
         _hip.check(_hip.lib().pamo_s3_active_contacts(self.ptr, ctypes.byref(n)), "pamo_s3_active_contacts")
         return int(n.value)
 
+    def newton_run(self) -> int:
+        """Newton iterations run since set_mesh; stats() also counts those
+        that repeat a fixed point (measurement)."""
+        n = ctypes.c_longlong(0)
+        _hip.check(_hip.lib().pamo_s3_newton_run(self.ptr, ctypes.byref(n)), "pamo_s3_newton_run")
+        return int(n.value)
+
     def set_cg_graph(self, on: bool):
         """Replay the PCG loop from a captured HIP graph (default) or launch
         its kernels one by one; results do not change."""
