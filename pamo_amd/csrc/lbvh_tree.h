@@ -1,8 +1,7 @@
 // Generic LBVH over float boxes on gfx950, shared by stage 3 (contact and
 // closest-point trees) and the surface metrics: Morton codes of box centres,
-// the radix sort of prim.h, Karras's hierarchy and bottom-up node boxes
-// (the stage-2 tree kernels of stage2_kernels.h), escape links for
-// stackless walks.
+// the radix sort of prim.h, Karras's hierarchy and node boxes as child pairs
+// (the stage-2 tree kernels of stage2_kernels.h).
 #pragma once
 
 #include <algorithm>
@@ -23,7 +22,7 @@ struct Tree {
     int n = 0, cap = 0;
     float4* item = nullptr;  // 2 per item (lo, hi)
     uint32_t *key = nullptr, *val = nullptr, *key2 = nullptr, *val2 = nullptr;
-    int *left = nullptr, *right = nullptr, *parent = nullptr;
+    int *left = nullptr, *right = nullptr, *slot = nullptr;  // slot and box: see karras_k
     int2* range = nullptr;
     float4 *box = nullptr, *pre = nullptr, *suf = nullptr, *blk = nullptr, *blkpre = nullptr, *blksuf = nullptr,
            *sblk = nullptr, *blktab = nullptr;
@@ -51,7 +50,7 @@ static int tree_alloc(Tree& t, int n, hipStream_t st) {
     PAMO_TRY(dalloc(&t.item, 2 * a, st));
     PAMO_TRY(dalloc(&t.key, a, st)); PAMO_TRY(dalloc(&t.val, a, st));
     PAMO_TRY(dalloc(&t.key2, a, st)); PAMO_TRY(dalloc(&t.val2, a, st));
-    PAMO_TRY(dalloc(&t.left, a, st)); PAMO_TRY(dalloc(&t.right, a, st)); PAMO_TRY(dalloc(&t.parent, 2 * a, st));
+    PAMO_TRY(dalloc(&t.left, a, st)); PAMO_TRY(dalloc(&t.right, a, st)); PAMO_TRY(dalloc(&t.slot, 2 * a, st));
     PAMO_TRY(dalloc(&t.range, a, st));
     PAMO_TRY(dalloc(&t.box, 4 * a, st));
     PAMO_TRY(dalloc(&t.pre, 2 * a, st)); PAMO_TRY(dalloc(&t.suf, 2 * a, st));
@@ -66,7 +65,7 @@ static int tree_alloc(Tree& t, int n, hipStream_t st) {
 }
 
 static void tree_free(Tree& t) {
-    void* ptrs[] = {t.item, t.key, t.val, t.key2, t.val2, t.left, t.right, t.parent, t.range, t.box,
+    void* ptrs[] = {t.item, t.key, t.val, t.key2, t.val2, t.left, t.right, t.slot, t.range, t.box,
                     t.pre,  t.suf, t.blk, t.blkpre, t.blksuf, t.sblk, t.blktab, t.part, t.cnt};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
@@ -101,21 +100,24 @@ __global__ void items_morton_k(const float4* __restrict__ item, int n, const flo
     val[i] = (uint32_t)i;
 }
 
-// Leaf and node boxes of a built hierarchy (box_tab_k, node_box_k) and,
-// unless refitting a tree whose links are already written, its rope links.
-static int tree_boxes(Tree& t, int n, bool refit, hipStream_t st) {
+// Leaf and node boxes of a built hierarchy.
+static int tree_boxes(Tree& t, int n, hipStream_t st) {
     const unsigned nb = grid_for(n, kBlock), nb1 = grid_for(nb, kBlock);
     hipLaunchKernelGGL(box_tab_k, dim3(nb), dim3(kBlock), 0, st, (const float4*)t.item, (const uint32_t*)t.val,
-                       (const int*)t.cnt, 0, t.box, (const int2*)t.range, t.pre, t.suf, t.blk, (float4*)nullptr, 0LL);
-    hipLaunchKernelGGL(box_tab_k, dim3(nb1), dim3(kBlock), 0, st, (const float4*)t.blk, (const uint32_t*)nullptr,
-                       (const int*)t.cnt, 1, (float4*)nullptr, (const int2*)nullptr, t.blkpre, t.blksuf, t.sblk,
-                       t.blktab, t.tab_stride);
-    hipLaunchKernelGGL(node_box_k, dim3(nb), dim3(kBlock), 0, st, (const int2*)t.range, (const int*)t.cnt,
-                       (const float4*)t.pre, (const float4*)t.suf, (const float4*)t.blktab, t.tab_stride,
-                       (const float4*)t.blkpre, (const float4*)t.blksuf, (const float4*)t.sblk, t.box);
-    if (!refit)
-        hipLaunchKernelGGL(rope_k, dim3(grid_for(2LL * n, kBlock)), dim3(kBlock), 0, st, (const int*)t.left,
-                           (const int2*)t.range, (const int*)t.cnt, (const uint32_t*)t.val, t.box);
+                       (const int*)t.cnt, 0, t.box, (const int*)t.slot, (const int2*)t.range, t.pre, t.suf, t.blk,
+                       (float4*)nullptr, 0LL);
+    if (nb <= (unsigned)kBlock) {
+        hipLaunchKernelGGL(node_box_small_k, dim3(nb), dim3(kBlock), 0, st, (const int2*)t.range, (const int*)t.cnt,
+                           (const float4*)t.pre, (const float4*)t.suf, (const float4*)t.blk, (const int*)t.slot, t.box);
+    } else {
+        hipLaunchKernelGGL(box_tab_k, dim3(nb1), dim3(kBlock), 0, st, (const float4*)t.blk, (const uint32_t*)nullptr,
+                           (const int*)t.cnt, 1, (float4*)nullptr, (const int*)nullptr, (const int2*)nullptr, t.blkpre,
+                           t.blksuf, t.sblk, t.blktab, t.tab_stride);
+        hipLaunchKernelGGL(node_box_k, dim3(nb), dim3(kBlock), 0, st, (const int2*)t.range, (const int*)t.cnt,
+                           (const float4*)t.pre, (const float4*)t.suf, (const float4*)t.blktab, t.tab_stride,
+                           (const float4*)t.blkpre, (const float4*)t.blksuf, (const float4*)t.sblk,
+                           (const int*)t.slot, t.box);
+    }
     PAMO_HIP(hipGetLastError());
     return 0;
 }
@@ -133,50 +135,18 @@ static int tree_build(Tree& t, int n, int* ws, hipStream_t st) {
     PAMO_HIP(hipGetLastError());
     PAMO_TRY(radix_sort_pairs(t.key, t.val, t.key2, t.val2, n, 32, ws, st));
     hipLaunchKernelGGL(karras_k, dim3(nb), dim3(kBlock), 0, st, (const uint32_t*)t.key, (const uint32_t*)t.val,
-                       (const int*)t.cnt, t.left, t.right, t.parent, t.range);
-    return tree_boxes(t, n, false, st);
+                       (const int*)t.cnt, t.left, t.right, t.slot, t.range, t.box);
+    return tree_boxes(t, n, st);
 }
 
 // Recomputes every box of a tree built by tree_build over the same n items,
 // after the items' boxes changed: leaf boxes in the built leaf order, node
-// boxes over the built hierarchy; the rope links in the records' .w fields
-// stay as built.  The tree stays exact for any item boxes; its quality degrades
+// boxes over the built hierarchy; the links stay as built.  The tree stays exact for any item boxes; its quality degrades
 // only as far as the items moved since the build.
 static int tree_refit(Tree& t, int n, hipStream_t st) {
     PAMO_CHECK(n == t.n, "tree_refit: item count differs from the built tree");
     if (n <= 0) return 0;
-    return tree_boxes(t, n, true, st);
-}
-
-// Child-pair records for nearest-item walks: both children's boxes of internal
-// node i in one hop, the left child's in pre[2i], pre[2i + 1] and the right
-// child's in suf[2i], suf[2i + 1], with the child in the lo box's w: an
-// internal node's number, or ~item for a leaf.  A walk step is then one
-// round of independent loads; over the node records it is the children's
-// numbers first and their boxes after.  The records take the place of the
-// in-block prefix and suffix boxes, which only a (re)fit reads and rewrites.
-__global__ void __launch_bounds__(kB) child_pairs_k(const float4* __restrict__ box, const int* __restrict__ left,
-                                                    const int* __restrict__ right, const uint32_t* __restrict__ val,
-                                                    int n, float4* __restrict__ pre, float4* __restrict__ suf) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n - 1) return;
-    const int l = left[i], r = right[i];
-    float4 a = box[2 * (long long)l], c = box[2 * (long long)r];
-    a.w = __int_as_float(l >= n - 1 ? ~(int)val[l - (n - 1)] : l);
-    c.w = __int_as_float(r >= n - 1 ? ~(int)val[r - (n - 1)] : r);
-    pre[2 * (long long)i] = a;
-    pre[2 * (long long)i + 1] = box[2 * (long long)l + 1];
-    suf[2 * (long long)i] = c;
-    suf[2 * (long long)i + 1] = box[2 * (long long)r + 1];
-}
-
-// Writes the child-pair records of a built tree (again after each refit).
-static int tree_pairs(Tree& t, hipStream_t st) {
-    if (t.n < 2) return 0;
-    hipLaunchKernelGGL(child_pairs_k, dim3(grid_for(t.n - 1, kB)), dim3(kB), 0, st, (const float4*)t.box,
-                       (const int*)t.left, (const int*)t.right, (const uint32_t*)t.val, t.n, t.pre, t.suf);
-    PAMO_HIP(hipGetLastError());
-    return 0;
+    return tree_boxes(t, n, st);
 }
 
 // Nearest-item walks keep the far children still to visit on a stack in LDS,
@@ -189,14 +159,11 @@ constexpr int kNearStack = 24;
 
 struct TreeView {
     int n;
-    const float4* box;
-    const int *left, *right, *parent;
+    const float4* box;  // child pairs
+    const int *left, *right, *slot;
     const uint32_t* val;
-    const float4 *pre, *suf;  // child-pair records (tree_pairs)
 };
-static TreeView view(const Tree& t) {
-    return TreeView{t.n, t.box, t.left, t.right, t.parent, t.val, t.pre, t.suf};
-}
+static TreeView view(const Tree& t) { return TreeView{t.n, t.box, t.left, t.right, t.slot, t.val}; }
 
 __device__ __forceinline__ bool box_hit(V3 lo, V3 hi, float4 blo, float4 bhi) {
     return !(hi.x < blo.x || bhi.x < lo.x || hi.y < blo.y || bhi.y < lo.y || hi.z < blo.z || bhi.z < lo.z);

@@ -179,7 +179,10 @@ __device__ __forceinline__ float near_bound(double d) { return d > 1e-30 ? (floa
 __device__ inline void near_by_links(Near& q, TreeView T, const double* __restrict__ V, const int* __restrict__ F,
                                      int* err) {
     const int n = T.n;
-    auto bd = [&](int node) { return box_d2(q.p, T.box[2 * (long long)node], T.box[2 * (long long)node + 1]); };
+    auto bd = [&](int node) {  // (the root, which has no box, is entered)
+        if (node == 0) return 0.0;
+        return box_d2(q.p, T.box[2 * (long long)T.slot[node]], T.box[2 * (long long)T.slot[node] + 1]);
+    };
     int prev = -1, cur = 0;
     const long long max_steps = 3LL * (2LL * n - 1) + 1;
     for (long long steps = 0; cur >= 0; ++steps) {
@@ -187,7 +190,7 @@ __device__ inline void near_by_links(Near& q, TreeView T, const double* __restri
             walk_overrun(err);
             break;
         }
-        const int par = cur == 0 ? -1 : T.parent[cur];
+        const int par = cur == 0 ? -1 : T.slot[cur] >> 1;
         int next;
         if (prev == par) {
             if (bd(cur) > q.best) {
@@ -212,7 +215,7 @@ __device__ inline void near_by_links(Near& q, TreeView T, const double* __restri
 
 // Nearest face of each point, a point a lane (lane t takes point order[t], or
 // t without an order).  Bound by the latency of the node loads: a step reads
-// one child-pair record (both children's boxes in one round of loads) and
+// one child pair (both children's boxes in one round of loads) and
 // never climbs.  Near child first, subtrees farther than the best
 // skipped.  Writes sqd[i] and, when given, I[i] and the closest point C[i].
 // With `rest`, a query not finished after max_steps steps is left to
@@ -257,8 +260,8 @@ __global__ void __launch_bounds__(kWave) point_mesh_k(const double* __restrict__
                 cur = n;
                 continue;
             }
-            const float4 la = T.pre[2 * (long long)cur], lb = T.pre[2 * (long long)cur + 1];
-            const float4 ra = T.suf[2 * (long long)cur], rb = T.suf[2 * (long long)cur + 1];
+            const float4* pair = T.box + 4 * (long long)cur;
+            const float4 la = pair[0], lb = pair[1], ra = pair[2], rb = pair[3];
             const double dl = box_d2(q.p, la, lb), dr = box_d2(q.p, ra, rb);
             const bool left_first = dl <= dr;
             const double dn = left_first ? dl : dr, df = left_first ? dr : dl;
@@ -339,8 +342,8 @@ __global__ void __launch_bounds__(kWave) point_mesh_wave_k(const double* __restr
             int cl = -1, cr = -1, fl = -1, fr = -1;
             float bl = 0.0f, br = 0.0f;
             if (x >= 0) {
-                const float4 la = T.pre[2 * (long long)x], lb = T.pre[2 * (long long)x + 1];
-                const float4 ra = T.suf[2 * (long long)x], rb = T.suf[2 * (long long)x + 1];
+                const float4* pair = T.box + 4 * (long long)x;
+                const float4 la = pair[0], lb = pair[1], ra = pair[2], rb = pair[3];
                 const double dl = box_d2(q.p, la, lb), dr = box_d2(q.p, ra, rb);
                 if (!(dl > q.best)) {
                     cl = __float_as_int(la.w);
@@ -478,8 +481,7 @@ static int build_tree(Work& w, hipStream_t st, const double* V, int nV, const in
                std::string(who) + ": " + std::to_string(w.h_flags[0]) + " faces index outside the vertices");
     hipLaunchKernelGGL(face_box_d_k, dim3(grid_for(nF, kB)), dim3(kB), 0, st, V, F, nF, w.tree.item);
     PAMO_HIP(hipGetLastError());
-    PAMO_TRY(s3::tree_build(w.tree, nF, w.ws, st));
-    return s3::tree_pairs(w.tree, st);
+    return s3::tree_build(w.tree, nF, w.ws, st);
 }
 
 // Fewer points than this are walked in their own order.
@@ -594,7 +596,7 @@ static size_t noalloc_layout(unsigned char* base, int max_faces, Work& w) {
     Tree& t = w.tree;
     take(t.item, 2 * a);
     take(t.key, a); take(t.val, a); take(t.key2, a); take(t.val2, a);
-    take(t.left, a); take(t.right, a); take(t.parent, 2 * a);
+    take(t.left, a); take(t.right, a); take(t.slot, 2 * a);
     take(t.range, a);
     take(t.box, 4 * a);
     take(t.pre, 2 * a); take(t.suf, 2 * a);

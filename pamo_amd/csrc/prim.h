@@ -375,6 +375,19 @@ inline void lookback_free(LookbackScan& lb) {
     lb = LookbackScan{};
 }
 
+// A launch of `tiles` workgroups that uses lb_prefix: a new epoch before it,
+// the tickets it will have taken after it.
+inline int lookback_begin(LookbackScan& lb, long long tiles, hipStream_t st) {
+    PAMO_CHECK(lb.state && tiles <= lb.cap, "look-back scan: tile states not reserved for this size");
+    if (lb.epoch + 1 >= (1u << 30)) {  // epochs exhausted: clear the states and start again
+        PAMO_HIP(hipMemsetAsync(lb.state, 0, sizeof(unsigned long long) * lb.cap, st));
+        lb.epoch = 0;
+    }
+    ++lb.epoch;
+    return 0;
+}
+inline void lookback_end(LookbackScan& lb, long long tiles) { lb.base += (unsigned)tiles; }
+
 // One launch of scan_op_k over n >= 0 items (a single tile needs no waiting).
 template <class Op>
 inline int scan_op(const Op& op, long long n, LookbackScan& lb, hipStream_t st, int prof_id = K_SCAN_TILES,
@@ -382,18 +395,13 @@ inline int scan_op(const Op& op, long long n, LookbackScan& lb, hipStream_t st, 
     if (n < 0) return 0;
     constexpr long long kTile = (long long)kScanBlock * Op::kIpt;
     const long long nb = std::max(1LL, (n + kTile - 1) / kTile);  // n = 0 still runs Op::done(0)
-    PAMO_CHECK(lb.state && nb <= lb.cap, "look-back scan: tile states not reserved for this size");
-    if (lb.epoch + 1 >= (1u << 30)) {  // epochs exhausted: clear the states and start again
-        PAMO_HIP(hipMemsetAsync(lb.state, 0, sizeof(unsigned long long) * lb.cap, st));
-        lb.epoch = 0;
-    }
-    ++lb.epoch;
+    PAMO_TRY(lookback_begin(lb, nb, st));
     prof_begin(prof_id, bytes, st);
     hipLaunchKernelGGL(scan_op_k<Op>, dim3((unsigned)nb), dim3(kScanBlock), 0, st, op, n, lb.state, lb.ticket,
                        lb.err, lb.epoch, lb.base);
     prof_end(prof_id, st);
     PAMO_HIP(hipGetLastError());
-    lb.base += (unsigned)nb;
+    lookback_end(lb, nb);
     return 0;
 }
 

@@ -119,7 +119,7 @@ struct Ctx {
     int *face_scan = nullptr, *qlist = nullptr;
     // LBVH
     uint32_t *bkey = nullptr, *bval = nullptr, *bkey2 = nullptr, *bval2 = nullptr;
-    int *bleft = nullptr, *bright = nullptr, *bparent = nullptr;  // parent: 2n-1 nodes
+    int *bleft = nullptr, *bright = nullptr, *bslot = nullptr;  // slot: 2n-1 nodes (karras_k)
     int2* brange = nullptr;
     float4 *bbox = nullptr, *fbox = nullptr, *bpre = nullptr, *bsuf = nullptr;  // 2 float4 per box
     float4 *blk = nullptr, *blkpre = nullptr, *blksuf = nullptr, *sblk = nullptr, *blktab = nullptr;
@@ -149,6 +149,8 @@ struct Ctx {
     int tree_keep_pct = 80;     // 100: rebuild every round
     bool tree_valid = false;    // bval / hierarchy describe the current faces
     bool tree_fresh = false;    // the next round may refit instead of building
+    bool tree_carry = false;    // the leaves still hold the faces' numbers before the last compaction
+    int carry_old = 0;          // faces before that compaction
     int tree_n = 0;             // leaves of the last tree, as last read back
     // guard launch shape: meshes of at most guard_split_faces faces serve
     // each query group with 2^guard_split_log waves, one per subtree
@@ -303,7 +305,7 @@ static int grow_tris(Ctx& c, size_t n) {
     PAMO_TRY(dalloc(&c.bkey, a, c.stream)); PAMO_TRY(dalloc(&c.bval, a, c.stream));
     PAMO_TRY(dalloc(&c.bkey2, a, c.stream)); PAMO_TRY(dalloc(&c.bval2, a, c.stream));
     PAMO_TRY(dalloc(&c.bleft, a, c.stream)); PAMO_TRY(dalloc(&c.bright, a, c.stream));
-    PAMO_TRY(dalloc(&c.bparent, 2 * a, c.stream));
+    PAMO_TRY(dalloc(&c.bslot, 2 * a, c.stream));
     PAMO_TRY(dalloc(&c.brange, a, c.stream));
     PAMO_TRY(dalloc(&c.bbox, 4 * a, c.stream));  // 2n-1 nodes, 2 float4 each
     PAMO_TRY(dalloc(&c.fbox, 2 * a, c.stream));
@@ -340,7 +342,7 @@ static void free_all(Ctx& c) {
     void* ptrs[] = {c.p, c.op, c.np, c.Q, c.occ, c.pts_map, c.ring_off, c.ring_fill, c.eord_cnt, c.undo_list, c.tmp_undo,
                     c.undo_prev, c.invalid, c.ti, c.tj, c.tk, c.oi, c.oj, c.ok, c.ni, c.nj, c.nk, c.ring, c.ring_raw, c.ring_own, c.rv,
                     c.edge_off, c.vmin, c.changed, c.flagged, c.face_scan, c.qlist, c.bkey, c.bval, c.bkey2,
-                    c.bval2, c.bleft, c.bright, c.bparent, c.brange, c.bbox, c.fbox, c.bpre, c.bsuf, c.blk, c.blkpre,
+                    c.bval2, c.bleft, c.bright, c.bslot, c.brange, c.bbox, c.fbox, c.bpre, c.bsuf, c.blk, c.blkpre,
                     c.blksuf, c.sblk, c.blktab, c.box_part, c.eu, c.ev, c.edge_cost, c.esel, c.recs, c.pflag, c.pushed, c.eord, c.erank,
                     c.shuf, c.ws, c.dcnt, c.cent_out, c.ulist, c.cent_means};
     for (void* q : ptrs)
@@ -414,11 +416,11 @@ static int sync_counters(Ctx& c) {
 static int run_guard(Ctx& c, int nT, bool refit) {
     Mesh m = cur_mesh(c);
     const double nP = c.n_pts;
-    const int nparts = (int)grid_for(nT + 1, kBlock);  // face_box_k also writes the sentinel box at nT
-    int* leaf_part = (int*)(c.box_part + 6 * nparts + 6);
-    LAUNCHP(K_FACE_BOX, 12.0 * nT + 16.0 * nP + 32.0 * nT + 4.0 * nT, face_box_k, nT + 1, m, nT, c.fbox, c.box_part,
-            leaf_part, c.flagged, (const int*)c.oi);
     if (!refit) {
+        const int nparts = (int)grid_for(nT, kBlock);
+        int* leaf_part = (int*)(c.box_part + 6 * nparts + 6);
+        LAUNCHP(K_FACE_BOX, 12.0 * nT + 16.0 * nP + 32.0 * nT + 4.0 * nT, face_box_k, nT, m, nT, c.fbox, c.box_part,
+                leaf_part, (const int*)c.oi);
         hipLaunchKernelGGL(whole_box_k, dim3(1), dim3(kBlock), 0, c.stream, c.box_part, nparts,
                            (const int*)leaf_part, c.dcnt);
         PAMO_HIP(hipGetLastError());
@@ -426,39 +428,43 @@ static int run_guard(Ctx& c, int nT, bool refit) {
                 (const float*)(c.box_part + 6 * nparts), c.bkey, c.bval);
         PAMO_TRY(radix_sort_pairs(c.bkey, c.bval, c.bkey2, c.bval2, nT, 32, c.ws, c.stream));
         LAUNCHP(K_KARRAS, 8.0 * nT + 16.0 * nT + 8.0 * nT, karras_k, nT, c.bkey, c.bval, c.dcnt, c.bleft, c.bright,
-                c.bparent, c.brange);
+                c.bslot, c.brange, c.bbox);
+        c.tree_carry = false;
     }
     // leaves of the tree: at most nT for a tree built this round, the last
     // build's count for a tree carried across rounds
     const int nL = refit ? std::max(nT, c.tree_n) : nT;
     // node boxes from leaf ranges: no communication between workgroups
     const unsigned nb0 = grid_for(nL, kBlock), nb1 = grid_for(nb0, kBlock);
-    prof_begin(K_BVH_BOXES, 4.0 * nT + 32.0 * nT + 32.0 * nT + 64.0 * nT, c.stream);
-    hipLaunchKernelGGL(box_tab_k, dim3(nb0), dim3(kBlock), 0, c.stream, (const float4*)c.fbox,
-                       (const uint32_t*)c.bval, (const int*)c.dcnt, 0, c.bbox, (const int2*)c.brange, c.bpre, c.bsuf,
-                       c.blk, (float4*)nullptr, 0LL);
-    hipLaunchKernelGGL(box_tab_k, dim3(nb1), dim3(kBlock), 0, c.stream, (const float4*)c.blk,
-                       (const uint32_t*)nullptr, (const int*)c.dcnt, 1, (float4*)nullptr, (const int2*)nullptr,
-                       c.blkpre, c.blksuf, c.sblk, c.blktab, c.blktab_stride);
-    hipLaunchKernelGGL(node_box_k, dim3(grid_for(nL, kBlock)), dim3(kBlock), 0, c.stream, (const int2*)c.brange,
-                       (const int*)c.dcnt, (const float4*)c.bpre, (const float4*)c.bsuf, (const float4*)c.blktab,
-                       c.blktab_stride, (const float4*)c.blkpre, (const float4*)c.blksuf, (const float4*)c.sblk,
-                       c.bbox);
-    // a refit keeps the hierarchy, so the links in the records' .w fields
-    // stand (box_tab_k rewrites each leaf's face id, which a carry renumbers)
-    if (!refit)
-        hipLaunchKernelGGL(rope_k, dim3(grid_for(2LL * nL, kBlock)), dim3(kBlock), 0, c.stream, (const int*)c.bleft,
-                           (const int2*)c.brange, (const int*)c.dcnt, (const uint32_t*)c.bval, c.bbox);
+    PAMO_TRY(lookback_begin(c.lb, nb0, c.stream));
+    prof_begin(K_BVH_BOXES, 4.0 * nT + 12.0 * nT + 16.0 * nP + 32.0 * nT + 64.0 * nT, c.stream);
+    hipLaunchKernelGGL(guard_leaves_k, dim3(nb0), dim3(kBlock), 0, c.stream, m, nT, c.bval, c.tree_carry ? 1 : 0,
+                       (const int*)c.face_scan, c.carry_old, (const uint8_t*)c.changed, c.flagged, c.dcnt, c.bbox,
+                       (const int*)c.bslot, (const int2*)c.brange, c.bpre, c.bsuf, c.blk, c.qlist, c.lb.state,
+                       c.lb.ticket, c.lb.err, c.lb.epoch, c.lb.base);
+    lookback_end(c.lb, nb0);
+    c.tree_carry = false;  // the leaves now hold this round's faces
+    if (nb0 <= (unsigned)kBlock) {
+        hipLaunchKernelGGL(node_box_small_k, dim3(nb0), dim3(kBlock), 0, c.stream, (const int2*)c.brange,
+                           (const int*)c.dcnt, (const float4*)c.bpre, (const float4*)c.bsuf, (const float4*)c.blk,
+                           (const int*)c.bslot, c.bbox);
+    } else {
+        hipLaunchKernelGGL(box_tab_k, dim3(nb1), dim3(kBlock), 0, c.stream, (const float4*)c.blk,
+                           (const uint32_t*)nullptr, (const int*)c.dcnt, 1, (float4*)nullptr, (const int*)nullptr,
+                           (const int2*)nullptr, c.blkpre, c.blksuf, c.sblk, c.blktab, c.blktab_stride);
+        hipLaunchKernelGGL(node_box_k, dim3(nb0), dim3(kBlock), 0, c.stream, (const int2*)c.brange,
+                           (const int*)c.dcnt, (const float4*)c.bpre, (const float4*)c.bsuf, (const float4*)c.blktab,
+                           c.blktab_stride, (const float4*)c.blkpre, (const float4*)c.blksuf, (const float4*)c.sblk,
+                           (const int*)c.bslot, c.bbox);
+    }
     prof_end(K_BVH_BOXES, c.stream);
     PAMO_HIP(hipGetLastError());
-    // queries: changed live faces in Morton order
-    PAMO_TRY(scan_op(QueryListOp{c.bval, c.changed, c.ti, nT, c.qlist, c.dcnt}, nL, c.lb, c.stream));
     // meshes up to 256k faces split every query group over 8 subtrees: late
     // rounds hold few queries, and one query with a large box would otherwise
     // hold a whole launch in one wave
     const int part_log = nT <= c.guard_split_faces ? c.guard_split_log : 0;
     const long long guard_threads = ((((long long)nT + kGuardQ - 1) / kGuardQ) << part_log) * kWave;
-    const double guard_bytes = 4.0 * nT + 12.0 * nT + 16.0 * nP + 32.0 * nT + 64.0 * nT + 8.0 * nT + 4.0 * nT + 1.0 * nT;
+    const double guard_bytes = 4.0 * nT + 12.0 * nT + 16.0 * nP + 64.0 * nT + 1.0 * nT + 1.0 * nT;
     Undecided u{nullptr, c.dcnt + C_UNDECIDED, 0, c.exact_guard == 2 ? 1 : 0};
     if (c.exact_guard) {
         // list capacity: undecided pairs are near-degenerate ones (a few per
@@ -472,19 +478,19 @@ static int run_guard(Ctx& c, int nT, bool refit) {
         u.cap = (int)std::min<size_t>(c.alloc_ulist, 0x7fffffff);
         PAMO_HIP(hipMemsetAsync(c.dcnt + C_UNDECIDED, 0, sizeof(int), c.stream));
         LAUNCHP(K_GUARD_QUERY, guard_bytes, (guard_query_k<kGuardStack, true>), guard_threads, m, c.qlist, c.dcnt,
-                c.changed, c.fbox, (const float4*)c.bbox, c.bright, 1e-3f, c.flagged, u, part_log, c.dcnt + C_WALK_ERR, c.walk_cap);
+                c.changed, (const float4*)c.bbox, (const int*)c.bslot, 1e-3f, c.flagged, u, part_log, c.dcnt + C_WALK_ERR, c.walk_cap);
         hipLaunchKernelGGL(exact_pairs_k, dim3(1024), dim3(kBlock), 0, c.stream, m, (const int2*)c.ulist,
                            (const int*)(c.dcnt + C_UNDECIDED), u.cap, c.flagged);
         PAMO_HIP(hipGetLastError());
     } else if (c.guard_small_stack) {
         LAUNCHP(K_GUARD_QUERY, guard_bytes, (guard_query_k<kGuardStackSmall, false>), guard_threads, m, c.qlist,
-                c.dcnt, c.changed, c.fbox, (const float4*)c.bbox, c.bright, 1e-3f, c.flagged, u, part_log, c.dcnt + C_WALK_ERR, c.walk_cap);
+                c.dcnt, c.changed, (const float4*)c.bbox, (const int*)c.bslot, 1e-3f, c.flagged, u, part_log, c.dcnt + C_WALK_ERR, c.walk_cap);
     } else if (c.guard_waves == 4) {
-        LAUNCHP(K_GUARD_QUERY, guard_bytes, guard_query_w4_k, guard_threads, m, c.qlist, c.dcnt, c.changed, c.fbox,
-                (const float4*)c.bbox, c.bright, 1e-3f, c.flagged, u, part_log, c.dcnt + C_WALK_ERR, c.walk_cap);
+        LAUNCHP(K_GUARD_QUERY, guard_bytes, guard_query_w4_k, guard_threads, m, c.qlist, c.dcnt, c.changed,
+                (const float4*)c.bbox, (const int*)c.bslot, 1e-3f, c.flagged, u, part_log, c.dcnt + C_WALK_ERR, c.walk_cap);
     } else {
         LAUNCHP(K_GUARD_QUERY, guard_bytes, (guard_query_k<kGuardStack, false>), guard_threads, m, c.qlist, c.dcnt,
-                c.changed, c.fbox, (const float4*)c.bbox, c.bright, 1e-3f, c.flagged, u, part_log, c.dcnt + C_WALK_ERR, c.walk_cap);
+                c.changed, (const float4*)c.bbox, (const int*)c.bslot, 1e-3f, c.flagged, u, part_log, c.dcnt + C_WALK_ERR, c.walk_cap);
     }
     return 0;
 }
@@ -708,28 +714,25 @@ static int prologue(Ctx& c, const int* undo_in, int n_undo_in, bool is_stuck) {
 
 // Drop removed vertices and faces and renumber (pamo/__init__.py:163-167):
 // stable compaction by pts_map and by a scan of live faces.
-// With carry, the guard tree's leaves are renumbered to the compacted
-// faces (carry_leaves_k) and the next round refits it unless fewer than
-// tree_keep_pct % of its leaves are still live.
+// With carry, the next round refits the guard tree, renumbering its leaves to
+// the compacted faces (guard_leaves_k), unless fewer than tree_keep_pct % of
+// its leaves are still live.
 static int compact_round(Ctx& c, int nP, int nT, bool carry = false) {
     Mesh m = cur_mesh(c);
     PAMO_TRY(scan_op(CompactMeshOp{m, nP, nT, c.occ, c.pts_map, c.face_scan, c.np, c.ni, c.nj, c.nk, c.dcnt},
                      (long long)std::max(nP, nT) + 1, c.lb, c.stream, K_COMPACT_MESH,
                      4.0 * nP + 4.0 * nP + 16.0 * nP + 16.0 * nP + 12.0 * nT + 4.0 * nT + 12.0 * nT));
     carry = carry && c.tree_valid && c.tree_keep_pct < 100;
-    if (carry) {
-        // over every leaf (CompactMeshOp has zeroed the live-leaf count): a carried tree can have more leaves than faces
-        LAUNCH(carry_leaves_k, std::max(nT, c.tree_n), c.bval, (const int*)c.ti, (const int*)c.face_scan, nT,
-               c.dcnt);
-    }
     PAMO_TRY(sync_counters(c));
     c.tree_n = c.hcnt[C_NLIVE];
     if (carry) {
-        const long long leaves = c.hcnt[C_NLIVE], live = c.hcnt[C_LIVE_LEAVES];
+        // every live face holds one leaf
+        const long long leaves = c.hcnt[C_NLIVE], live = c.hcnt[C_NF];
         c.tree_fresh = live > 1 && live * 100 >= leaves * (long long)c.tree_keep_pct;
-        c.tree_valid = c.tree_fresh;
+        c.tree_valid = c.tree_carry = c.tree_fresh;
+        c.carry_old = nT;
     } else {
-        c.tree_valid = c.tree_fresh = false;
+        c.tree_valid = c.tree_fresh = c.tree_carry = false;
     }
     std::swap(c.p, c.np);
     std::swap(c.ti, c.ni);
@@ -1071,7 +1074,19 @@ int pamo_round_debug(pamo_ctx* ctx, int what, void* d_out, long long cap, long l
             else if (what == PAMO_DBG_BVH_FACES) { n = h; src = c.bval; }
             else if (what == PAMO_DBG_BVH_LEFT) { n = h > 0 ? h - 1 : 0; src = c.bleft; }
             else if (what == PAMO_DBG_BVH_RIGHT) { n = h > 0 ? h - 1 : 0; src = c.bright; }
-            else { n = h > 0 ? 8LL * (2 * h - 1) : 0; src = c.bbox; }  // (2n-1) nodes x (lo4, hi4)
+            else {  // (2n-1) nodes x (lo4, hi4), gathered from the child pairs
+                n = h > 0 ? 8LL * (2 * h - 1) : 0;
+                PAMO_CHECK(n <= cap, "pamo_round_debug: cap too small");
+                if (h > 1)
+                    hipLaunchKernelGGL(pamo::node_records_k, dim3(pamo::grid_for(2LL * h, pamo::kBlock)),
+                                       dim3(pamo::kBlock), 0, c.stream, (const int*)c.bleft, (const int2*)c.brange,
+                                       (const int*)c.dcnt, (const uint32_t*)c.bval, (const int*)c.bslot,
+                                       (const float4*)c.bbox, (float4*)d_out);
+                PAMO_HIP(hipGetLastError());
+                PAMO_HIP(hipStreamSynchronize(c.stream));
+                if (n_out) *n_out = n;
+                return 0;
+            }
             break;
         }
         case PAMO_DBG_UNDO_ITERS: if (n_out) *n_out = c.undo_iters; return 0;

@@ -11,6 +11,7 @@
 #include "exact_guard.h"
 #include "guard_ref.h"
 #include "hip_common.h"
+#include "prim.h"
 
 namespace pamo {
 // Internal linkage: every translation unit that includes this header gets
@@ -69,7 +70,6 @@ enum Counter {
     C_UNDECIDED = 8,  // exact guard: pairs the filtered predicates left undecided
     C_WALK_ERR = 9,   // a guard tree walk exceeded its bound (walk_overrun)
     C_BAD_UNDO = 10,  // an incoming undo entry outside the context's points
-    C_LIVE_LEAVES = 11,  // guard tree leaves still live after a compaction
     C_COUNT = 16
 };
 
@@ -1100,45 +1100,42 @@ __device__ __forceinline__ void block_minmax6(float lo[3], float hi[3], float (*
     }
 }
 
-// Face boxes (an empty box, lo = +inf and hi = -inf, for a removed face),
-// per-block partial bounding boxes of the live faces, per-block counts of
-// the guard tree's leaves, and the guard's flags cleared (flagged[f] = 0).
+// Box of face f (empty, lo = +inf and hi = -inf, for a removed one).
+__device__ __forceinline__ void face_box(const Mesh& m, int f, float4& lo, float4& hi) {
+    const float inf = __builtin_huge_valf();
+    lo = make_float4(inf, inf, inf, 0.0f);
+    hi = make_float4(-inf, -inf, -inf, 0.0f);
+    const int a = m.i[f];
+    if (a == -1) return;
+    const float4 p = m.p[a], q = m.p[m.j[f]], r = m.p[m.k[f]];
+    lo = make_float4(fminf(p.x, fminf(q.x, r.x)), fminf(p.y, fminf(q.y, r.y)), fminf(p.z, fminf(q.z, r.z)), 0.0f);
+    hi = make_float4(fmaxf(p.x, fmaxf(q.x, r.x)), fmaxf(p.y, fmaxf(q.y, r.y)), fmaxf(p.z, fmaxf(q.z, r.z)), 0.0f);
+}
+
+// For a tree to be built: face boxes, per-block partial bounding boxes of the
+// live faces, and per-block counts of the guard tree's leaves.
 // The leaves are the faces live at the start of the round (snap_i[f] != -1):
 // every face live after the collapse, and every face an undo can restore.
 __global__ void __launch_bounds__(kBlock) face_box_k(Mesh m, int nT, float4* __restrict__ fbox,
                                                      float* __restrict__ part, int* __restrict__ leaf_part,
-                                                     uint8_t* __restrict__ flagged, const int* __restrict__ snap_i) {
+                                                     const int* __restrict__ snap_i) {
     __shared__ float red[6][kBlock];
     __shared__ int nleaf;
     const int f = blockIdx.x * blockDim.x + threadIdx.x;
     const float inf = __builtin_huge_valf();
-    float lo[3] = {inf, inf, inf}, hi[3] = {-inf, -inf, -inf};
+    float4 a = make_float4(inf, inf, inf, 0.0f), b = make_float4(-inf, -inf, -inf, 0.0f);
     bool leaf = false;
     if (threadIdx.x == 0) nleaf = 0;
     __syncthreads();
-    if (f == nT) {
-        // the box of a carried tree's dead leaves (face id nT): empty
-        fbox[2 * (long long)f] = make_float4(inf, inf, inf, 0.0f);
-        fbox[2 * (long long)f + 1] = make_float4(-inf, -inf, -inf, 0.0f);
-    }
     if (f < nT) {
-        flagged[f] = 0;
-        int a = m.i[f];
-        if (a != -1) {
-            F3 p = ld(m, a), q = ld(m, m.j[f]), r = ld(m, m.k[f]);
-            lo[0] = fminf(p.x, fminf(q.x, r.x));
-            lo[1] = fminf(p.y, fminf(q.y, r.y));
-            lo[2] = fminf(p.z, fminf(q.z, r.z));
-            hi[0] = fmaxf(p.x, fmaxf(q.x, r.x));
-            hi[1] = fmaxf(p.y, fmaxf(q.y, r.y));
-            hi[2] = fmaxf(p.z, fmaxf(q.z, r.z));
-        }
-        leaf = a != -1 || snap_i[f] != -1;
-        fbox[2 * (long long)f] = make_float4(lo[0], lo[1], lo[2], 0.0f);
-        fbox[2 * (long long)f + 1] = make_float4(hi[0], hi[1], hi[2], 0.0f);
+        face_box(m, f, a, b);
+        leaf = m.i[f] != -1 || snap_i[f] != -1;
+        fbox[2 * (long long)f] = a;
+        fbox[2 * (long long)f + 1] = b;
     }
     uint64_t lm = __ballot(leaf);
     if ((threadIdx.x & 63) == 0 && lm) atomicAdd(&nleaf, (int)__popcll(lm));
+    float lo[3] = {a.x, a.y, a.z}, hi[3] = {b.x, b.y, b.z};
     block_minmax6(lo, hi, red);
     __syncthreads();
     if (threadIdx.x < 6) part[6 * blockIdx.x + threadIdx.x] = red[threadIdx.x][0];
@@ -1261,9 +1258,16 @@ __device__ __forceinline__ int delta_at(const uint32_t* key, const uint32_t* val
 
 // Karras 2012 radix tree over the sorted keys (code << 32 | face); also
 // records each internal node's leaf range for the box pass.
+//
+// Boxes are stored as child pairs: node x (internal: its number, leaf s: n - 1
+// + s) has slot[x] = 2 parent + (0 left, 1 right) and its box at box[2 slot]
+// (lo, hi), so both children of internal node i lie in the four float4 at 4 i
+// and a walk's step reads them in one round of independent loads.  lo.w links
+// to the child: an internal node's number, or ~item for a leaf.  The root has
+// no slot: a walk starts at pair 0.
 __global__ void karras_k(const uint32_t* __restrict__ key, const uint32_t* __restrict__ val,
                          const int* __restrict__ cnt, int* __restrict__ left, int* __restrict__ right,
-                         int* __restrict__ parent, int2* __restrict__ range) {
+                         int* __restrict__ slot, int2* __restrict__ range, float4* __restrict__ box) {
     const int n = cnt[C_NLIVE];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n - 1) return;
@@ -1303,9 +1307,12 @@ __global__ void karras_k(const uint32_t* __restrict__ key, const uint32_t* __res
     const int r = (last == split + 1) ? split + 1 + (n - 1) : split + 1;
     left[i] = l;
     right[i] = r;
-    parent[l] = i;
-    parent[r] = i;
+    slot[l] = 2 * i;
+    slot[r] = 2 * i + 1;
     range[i] = make_int2(first, last);
+    // (a leaf's link is written with its box)
+    if (l < n - 1) box[4 * (long long)i].w = __int_as_float(l);
+    if (r < n - 1) box[4 * (long long)i + 2].w = __int_as_float(r);
 }
 
 // Box unions inside aligned blocks of 256 leaves, from a sparse table in
@@ -1344,9 +1351,60 @@ __device__ __forceinline__ void store_xyz(float4* q, const float* v) {
     f[2] = v[2];
 }
 
+// Builds the table of one block's boxes (a, b; empty past the end) in T.
+__device__ __forceinline__ void tab_build(BoxTab& T, int t, float4 a, float4 b) {
+    T.v[0][0][t] = a.x; T.v[0][1][t] = a.y; T.v[0][2][t] = a.z;
+    T.v[0][3][t] = b.x; T.v[0][4][t] = b.y; T.v[0][5][t] = b.z;
+    for (int k = 1; k < kTabLevels; ++k) {
+        __syncthreads();
+        const int h = 1 << (k - 1);
+        const int u = t + h < kBlock ? t + h : t;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            T.v[k][c][t] = fminf(T.v[k - 1][c][t], T.v[k - 1][c][u]);
+            T.v[k][3 + c][t] = fmaxf(T.v[k - 1][3 + c][t], T.v[k - 1][3 + c][u]);
+        }
+    }
+    __syncthreads();
+}
+
+__device__ __forceinline__ void put_box(float4* __restrict__ dst, long long q, const float* lo, const float* hi) {
+    dst[2 * q] = make_float4(lo[0], lo[1], lo[2], 0.0f);
+    dst[2 * q + 1] = make_float4(hi[0], hi[1], hi[2], 0.0f);
+}
+
+// From block b's table (entries s = 256 b + t < n): the prefix and suffix
+// boxes, the block's box, and (with range) the boxes of the internal nodes
+// numbered and contained in the block.
+__device__ __forceinline__ void tab_store(const BoxTab& T, int b, int t, int n, float4* __restrict__ pre,
+                                          float4* __restrict__ suf, float4* __restrict__ blk, int n_leaves,
+                                          const int2* __restrict__ range, const int* __restrict__ slot,
+                                          float4* __restrict__ box) {
+    const int base = b * kBlock, s = base + t;
+    float lo[3], hi[3];
+    if (s < n) {
+        tab_union(T, 0, t, lo, hi);
+        put_box(pre, s, lo, hi);
+        tab_union(T, t, kBlock - 1, lo, hi);
+        put_box(suf, s, lo, hi);
+        if (t == 0) put_box(blk, b, lo, hi);
+    }
+    if (range && s > 0 && s < n_leaves - 1) {
+        const int2 r = range[s];
+        if ((r.x >> 8) == (r.y >> 8)) {
+            tab_union(T, r.x - base, r.y - base, lo, hi);
+            float4* q = box + 2 * (long long)slot[s];
+            store_xyz(q, lo);
+            store_xyz(q + 1, hi);
+        }
+    }
+}
+
+// Level 0: the leaves' boxes from src (gathered by item) and what follows from
+// them; level 1: the same over the block boxes, with the table stored.
 __global__ void __launch_bounds__(kBlock) box_tab_k(const float4* __restrict__ src, const uint32_t* __restrict__ gather,
-                                                    const int* __restrict__ cnt, int level,
-                                                    float4* __restrict__ node, const int2* __restrict__ range,
+                                                    const int* __restrict__ cnt, int level, float4* __restrict__ box,
+                                                    const int* __restrict__ slot, const int2* __restrict__ range,
                                                     float4* __restrict__ pre, float4* __restrict__ suf,
                                                     float4* __restrict__ blk, float4* __restrict__ tab,
                                                     long long tab_stride) {
@@ -1362,47 +1420,15 @@ __global__ void __launch_bounds__(kBlock) box_tab_k(const float4* __restrict__ s
         const long long g = gather ? (long long)gather[s] : s;
         a = src[2 * g];
         b = src[2 * g + 1];
-        if (node) {
-            float4* q = node + 2 * ((long long)nl - 1 + s);
-            q[0] = make_float4(a.x, a.y, a.z, __int_as_float((int)g));
+        if (box && nl > 1) {
+            float4* q = box + 2 * (long long)slot[nl - 1 + s];
+            q[0] = make_float4(a.x, a.y, a.z, __int_as_float(~(int)g));
             const float hv[3] = {b.x, b.y, b.z};
             store_xyz(q + 1, hv);
         }
     }
-    T.v[0][0][t] = a.x; T.v[0][1][t] = a.y; T.v[0][2][t] = a.z;
-    T.v[0][3][t] = b.x; T.v[0][4][t] = b.y; T.v[0][5][t] = b.z;
-    for (int k = 1; k < kTabLevels; ++k) {
-        __syncthreads();
-        const int h = 1 << (k - 1);
-        const int u = t + h < kBlock ? t + h : t;
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            T.v[k][c][t] = fminf(T.v[k - 1][c][t], T.v[k - 1][c][u]);
-            T.v[k][3 + c][t] = fmaxf(T.v[k - 1][3 + c][t], T.v[k - 1][3 + c][u]);
-        }
-    }
-    __syncthreads();
-    float lo[3], hi[3];
-    if (s < n) {
-        tab_union(T, 0, t, lo, hi);
-        pre[2 * (long long)s] = make_float4(lo[0], lo[1], lo[2], 0.0f);
-        pre[2 * (long long)s + 1] = make_float4(hi[0], hi[1], hi[2], 0.0f);
-        tab_union(T, t, kBlock - 1, lo, hi);
-        suf[2 * (long long)s] = make_float4(lo[0], lo[1], lo[2], 0.0f);
-        suf[2 * (long long)s + 1] = make_float4(hi[0], hi[1], hi[2], 0.0f);
-        if (t == 0) {
-            blk[2 * (long long)blockIdx.x] = make_float4(lo[0], lo[1], lo[2], 0.0f);
-            blk[2 * (long long)blockIdx.x + 1] = make_float4(hi[0], hi[1], hi[2], 0.0f);
-        }
-    }
-    if (range && s < nl - 1) {
-        const int2 r = range[s];
-        if ((r.x >> 8) == (r.y >> 8)) {
-            tab_union(T, r.x - base, r.y - base, lo, hi);
-            store_xyz(node + 2 * (long long)s, lo);
-            store_xyz(node + 2 * (long long)s + 1, hi);
-        }
-    }
+    tab_build(T, t, a, b);
+    tab_store(T, blockIdx.x, t, n, pre, suf, blk, nl, box ? range : nullptr, slot, box);
     if (tab && s < n) {
         for (int k = 0; k < kTabLevels; ++k) {
             float4* q = tab + 2 * (k * tab_stride + s);
@@ -1449,10 +1475,11 @@ __global__ void __launch_bounds__(kBlock) node_box_k(const int2* __restrict__ ra
                                                      const float4* __restrict__ tab, long long tab_stride,
                                                      const float4* __restrict__ bpre,
                                                      const float4* __restrict__ bsuf,
-                                                     const float4* __restrict__ sblk, float4* __restrict__ box) {
+                                                     const float4* __restrict__ sblk, const int* __restrict__ slot,
+                                                    float4* __restrict__ box) {
     const int n = cnt[C_NLIVE];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n - 1) return;
+    if (i == 0 || i >= n - 1) return;
     const int2 r = range[i];
     const int A = r.x >> 8, B = r.y >> 8;
     if (A == B) return;
@@ -1474,23 +1501,67 @@ __global__ void __launch_bounds__(kBlock) node_box_k(const int2* __restrict__ ra
         }
     }
     const float l3[3] = {lo.x, lo.y, lo.z}, h3[3] = {hi.x, hi.y, hi.z};
-    store_xyz(box + 2 * (long long)i, l3);
-    store_xyz(box + 2 * (long long)i + 1, h3);
+    store_xyz(box + 2 * (long long)slot[i], l3);
+    store_xyz(box + 2 * (long long)slot[i] + 1, h3);
+}
+
+// The level-1 table and node_box_k in one launch, for trees of at most 256
+// blocks (65,536 leaves): every block builds the table of the block boxes
+// itself (8 KiB of loads) instead of waiting for a launch of one block.
+__global__ void __launch_bounds__(kBlock) node_box_small_k(const int2* __restrict__ range, const int* __restrict__ cnt,
+                                                           const float4* __restrict__ pre,
+                                                           const float4* __restrict__ suf,
+                                                           const float4* __restrict__ blk,
+                                                           const int* __restrict__ slot, float4* __restrict__ box) {
+    __shared__ BoxTab T;
+    const int n = cnt[C_NLIVE];
+    const int t = threadIdx.x, i = blockIdx.x * kBlock + t;
+    int A = 0, B = 0;
+    int2 r = make_int2(0, 0);
+    if (i > 0 && i < n - 1) {
+        r = range[i];
+        A = r.x >> 8;
+        B = r.y >> 8;
+    }
+    if (!__syncthreads_or(A != B)) return;
+    const int nb = (n + kBlock - 1) / kBlock;
+    const float inf = __builtin_huge_valf();
+    float4 a = make_float4(inf, inf, inf, 0.0f), b = make_float4(-inf, -inf, -inf, 0.0f);
+    if (t < nb) {
+        a = blk[2 * t];
+        b = blk[2 * t + 1];
+    }
+    tab_build(T, t, a, b);
+    if (A == B) return;
+    float4 lo = make_float4(inf, inf, inf, 0.0f), hi = make_float4(-inf, -inf, -inf, 0.0f);
+    grow(lo, hi, suf, r.x);
+    grow(lo, hi, pre, r.y);
+    float l3[3] = {lo.x, lo.y, lo.z}, h3[3] = {hi.x, hi.y, hi.z};
+    if (A + 1 <= B - 1) {
+        float ml[3], mh[3];
+        tab_union(T, A + 1, B - 1, ml, mh);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            l3[c] = fminf(l3[c], ml[c]);
+            h3[c] = fmaxf(h3[c], mh[c]);
+        }
+    }
+    float4* q = box + 2 * (long long)slot[i];
+    store_xyz(q, l3);
+    store_xyz(q + 1, h3);
 }
 
 // ---------------------------------------------------------------- guard (A12, A13)
-// Escape ("rope") links: node records become two float4 (lo.xyz, left child
-// or, for a leaf, its item id in lo.w; hi.xyz, escape node in hi.w).  The
-// escape of x is the next node in depth-first order once x's subtree is
-// done: the right sibling of the first ancestor-or-self that is a left
-// child, -1 past the end.  Traversal then needs one 32-byte record per step
-// and no stack or parent walk.
-__global__ void __launch_bounds__(kBlock) rope_k(const int* __restrict__ left, const int2* __restrict__ range,
-                                                 const int* __restrict__ cnt, const uint32_t* __restrict__ val,
-                                                 float4* __restrict__ node) {
+// Node records for the tests' readback, in node order: lo.xyz with the left
+// child (a leaf: its item) in lo.w, hi.xyz with the escape node in hi.w (the
+// next node in depth-first order once the subtree is done, -1 past the end).
+__global__ void __launch_bounds__(kBlock) node_records_k(const int* __restrict__ left, const int2* __restrict__ range,
+                                                         const int* __restrict__ cnt, const uint32_t* __restrict__ val,
+                                                         const int* __restrict__ slot, const float4* __restrict__ box,
+                                                         float4* __restrict__ node) {
     const int n = cnt[C_NLIVE];
     const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n <= 0 || x >= 2 * n - 1) return;
+    if (n <= 1 || x >= 2 * n - 1) return;
     // x's subtree ends at leaf b; the next node in depth-first order is the
     // right child of the node that splits between leaves b and b+1.  That
     // child is internal node b+1 when that node's range starts at b+1 (an
@@ -1504,42 +1575,35 @@ __global__ void __launch_bounds__(kBlock) rope_k(const int* __restrict__ left, c
         const int c = b + 1;
         esc = (c <= n - 2 && range[c].x == c) ? c : c + (n - 1);
     }
-    const int lw = leaf ? (int)val[x - (n - 1)] : left[x];
-    float* r = reinterpret_cast<float*>(node + 2 * (long long)x);
-    r[3] = __int_as_float(lw);
-    r[7] = __int_as_float(esc);
-}
-
-// Splits a rope-linked tree into the 2^kLog subtrees under the root (fewer
-// where a leaf is reached early): lane k of a query walks subtree k, from the
-// returned node until *stop (that node's escape).  The right child of a node
-// is its left child's escape.  Returns -1 for lanes with no subtree.
-template <int kLog>
-__device__ __forceinline__ int subtree_start(const float4* __restrict__ node, int n_leaves, int k, int* stop) {
-    int cur = 0;
-    for (int d = kLog - 1; d >= 0; --d) {
-        if (cur >= n_leaves - 1) {
-            if ((k & ((2 << d) - 1)) != 0) return -1;
-            break;
-        }
-        const int left = __float_as_int(node[2 * (long long)cur].w);
-        cur = ((k >> d) & 1) ? __float_as_int(node[2 * (long long)left + 1].w) : left;
+    float4 lo, hi;
+    if (x == 0) {
+        const float4 a = box[0], c = box[1], d = box[2], e = box[3];
+        lo = make_float4(fminf(a.x, d.x), fminf(a.y, d.y), fminf(a.z, d.z), 0.0f);
+        hi = make_float4(fmaxf(c.x, e.x), fmaxf(c.y, e.y), fmaxf(c.z, e.z), 0.0f);
+    } else {
+        lo = box[2 * (long long)slot[x]];
+        hi = box[2 * (long long)slot[x] + 1];
     }
-    *stop = __float_as_int(node[2 * (long long)cur + 1].w);
-    return cur;
+    lo.w = __int_as_float(leaf ? (int)val[x - (n - 1)] : left[x]);
+    hi.w = __int_as_float(esc);
+    node[2 * (long long)x] = lo;
+    node[2 * (long long)x + 1] = hi;
 }
 
-// subtree_start with a run-time depth: the root of subtree k of 2^log (k's
-// bits choose left / right from the root down), -1 when that subtree does not
-// exist because a leaf is reached above depth log (the leaf then belongs to
-// the subtree whose remaining bits are zero).  The subtrees partition the
-// leaves.
-__device__ __forceinline__ int subtree_root(const float4* __restrict__ node, int n_leaves, int k, int log) {
+// The link to subtree k of the 2^log below the root (k's bits choose left /
+// right from the root down), with its box at *at (not for log = 0: the root
+// has none): an internal node, ~item of a leaf, or kNoNode when that subtree
+// does not exist because a leaf is reached above depth log (the leaf then
+// belongs to the subtree whose remaining bits are zero).  The subtrees
+// partition the leaves.
+constexpr int kNoNode = -0x7fffffff - 1;
+__device__ __forceinline__ int subtree_link(const float4* __restrict__ box, int k, int log, long long* at) {
     int cur = 0;
+    *at = 0;
     for (int d = log - 1; d >= 0; --d) {
-        if (cur >= n_leaves - 1) return (k & ((2 << d) - 1)) != 0 ? -1 : cur;
-        const int left = __float_as_int(node[2 * (long long)cur].w);
-        cur = ((k >> d) & 1) ? __float_as_int(node[2 * (long long)left + 1].w) : left;
+        if (cur < 0) return (k & ((2 << d) - 1)) != 0 ? kNoNode : cur;
+        *at = 4 * (long long)cur + 2 * ((k >> d) & 1);
+        cur = __float_as_int(box[*at].w);
     }
     return cur;
 }
@@ -1562,29 +1626,6 @@ __device__ __forceinline__ void load_tri9(Mesh m, int f, float T[3][3], int idx[
     }
 }
 
-// Carries the guard tree across a compaction: leaf s keeps its place in the
-// hierarchy and takes its face's new index, or nT_new (the empty sentinel
-// box) if the face was removed; counts the leaves still live.  Every face
-// live at the next round's start is live now, hence already a leaf.
-__global__ void carry_leaves_k(uint32_t* __restrict__ val, const int* __restrict__ ti, const int* __restrict__ fpos,
-                               int nT_old, int* __restrict__ cnt) {
-    __shared__ int nlive;
-    const int n = cnt[C_NLIVE], n_new = cnt[C_NF];
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (threadIdx.x == 0) nlive = 0;
-    __syncthreads();
-    bool live = false;
-    if (s < n) {
-        const int f = (int)val[s];  // nT_old: already dead
-        live = f >= 0 && f < nT_old && ti[f] != -1 && fpos[f] < n_new;
-        val[s] = live ? (uint32_t)fpos[f] : (uint32_t)n_new;
-    }
-    const uint64_t lm = __ballot(live);
-    if ((threadIdx.x & 63) == 0 && lm) atomicAdd(&nlive, (int)__popcll(lm));
-    __syncthreads();
-    if (threadIdx.x == 0 && nlive) atomicAdd(&cnt[C_LIVE_LEAVES], nlive);
-}
-
 // Wave-level ordering point for LDS traffic between lanes of one wave.
 __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -1605,7 +1646,7 @@ __device__ __forceinline__ void eval_pair(Mesh m, int a, int b, float epsilon, u
     }
 }
 
-constexpr int kQueue = 128;   // per-wave pair queue (< 64 pending + one append of <= 64)
+constexpr int kQueue = 192;   // per-wave pair queue (< 64 pending + one append of <= 128)
 constexpr int kGuardQ = 8;    // guard queries per wave
 constexpr int kGuardStack = 512;       // per-wave frontier entries
 constexpr int kGuardStackSmall = 32;   // test variant: forces the overflow walk
@@ -1691,33 +1732,42 @@ __global__ void __launch_bounds__(kBlock) exact_pairs_k(Mesh m, const int2* __re
     }
 }
 
-// Stackless walk of the subtree below internal node x: from its left child
-// until x's escape, evaluating candidates in this lane.  Inlined: as a
-// called function its register needs add to the caller's (242 registers,
-// 2 waves per SIMD, against 129 inlined).
+// Stackless walk of the subtree below internal node `top`, evaluating
+// candidates in this lane: a node's children in turn, back up by the slots.
+// Inlined: as a called function its register needs add to the caller's (242
+// registers, 2 waves per SIMD, against 129 inlined).
 template <bool kExact>
 __device__ __forceinline__ void guard_walk_subtree(Mesh m, const uint8_t* __restrict__ changed,
-                                                const float4* __restrict__ node, int n, int x, int stop,
-                                                float4 qlo, float4 qhi, int a, int ia0, int ia1, int ia2,
-                                                float epsilon, uint8_t* __restrict__ flagged, Undecided u,
-                                                int* err, long long max_visits) {
-    for (long long visits = 0; x != stop; ++visits) {
-        if (visits >= max_visits || x < 0) {
+                                                   const float4* __restrict__ box, const int* __restrict__ slot,
+                                                   int top, float4 qlo, float4 qhi, int a, int ia0, int ia1, int ia2,
+                                                   float epsilon, uint8_t* __restrict__ flagged, Undecided u,
+                                                   int* err, long long max_visits) {
+    int x = top, side = 0;
+    for (long long visits = 0;; ++visits) {
+        if (visits >= 3 * max_visits || x < 0) {
             walk_overrun(err);
             return;
         }
-        const float4 lo = node[2 * (long long)x], hi = node[2 * (long long)x + 1];
-        const int lw = __float_as_int(lo.w), esc = __float_as_int(hi.w);
-        if (overlap(qlo, qhi, lo, hi)) {
-            if (x >= n - 1) {
-                if (guard_candidate<kExact>(m, changed, a, ia0, ia1, ia2, lw))
-                    guard_eval<kExact>(m, a, lw, epsilon, flagged, u);
-                x = esc;
-            } else {
-                x = lw;
-            }
+        if (side == 2) {  // both children done
+            if (x == top) return;
+            const int up = slot[x];
+            x = up >> 1;
+            side = (up & 1) + 1;
+            continue;
+        }
+        const float4 lo = box[4 * (long long)x + 2 * side], hi = box[4 * (long long)x + 2 * side + 1];
+        if (!overlap(qlo, qhi, lo, hi)) {
+            ++side;
+            continue;
+        }
+        const int link = __float_as_int(lo.w);
+        if (link >= 0) {
+            x = link;
+            side = 0;
         } else {
-            x = esc;
+            if (guard_candidate<kExact>(m, changed, a, ia0, ia1, ia2, ~link))
+                guard_eval<kExact>(m, a, ~link, epsilon, flagged, u);
+            ++side;
         }
     }
 }
@@ -1726,21 +1776,22 @@ __device__ __forceinline__ void guard_walk_subtree(Mesh m, const uint8_t* __rest
 // every queried face a against every live face b whose box overlaps a's.
 //
 // A wave serves kGuardQ queries with one shared LIFO frontier of
-// (query, node) entries in LDS: each step pops up to 64 entries (one per
-// lane), tests their boxes, pushes both children of overlapping internal
-// nodes and appends overlapping leaves to a pair queue, which the wave
+// (query, internal node) entries in LDS: each step pops up to 64 entries (one
+// per lane), reads both children's boxes, pushes the overlapping internal
+// ones and appends the overlapping leaves to a pair queue, which the wave
 // evaluates 64 pairs at a time.  The critical path is then the wave's total
 // node count / 64 plus the tree depth, instead of the longest single walk.
-// When the frontier is full, a lane walks the rest of its subtree by escape
-// links (exact, only slower).  The flags are idempotent, so the visiting
-// order does not change the result.
+// (With node records and the children pushed untested, half of the pops found
+// no overlap: 60 us a launch on the 2M-face headline, GUARD_NOW now.)
+// When the frontier is full, a lane walks the rest of its subtree by itself
+// (exact, only slower).  The flags are idempotent, so the visiting order does
+// not change the result.
 template <int kStackCap, bool kExact>
 __device__ __forceinline__ void guard_query_body(Mesh m, const int* __restrict__ list, const int* __restrict__ cnt,
                                                  const uint8_t* __restrict__ changed,
-                                                 const float4* __restrict__ fbox, const float4* __restrict__ node,
-                                                 const int* __restrict__ right, float epsilon,
-                                                 uint8_t* __restrict__ flagged, Undecided u, int part_log, int* err,
-                                                 long long walk_cap) {
+                                                 const float4* __restrict__ box, const int* __restrict__ slot,
+                                                 float epsilon, uint8_t* __restrict__ flagged, Undecided u,
+                                                 int part_log, int* err, long long walk_cap) {
     constexpr int kW = kBlock / kWave;
     __shared__ int2 stk[kW][kStackCap];
     __shared__ int2 pq[kW][kQueue];
@@ -1755,18 +1806,33 @@ __device__ __forceinline__ void guard_query_body(Mesh m, const int* __restrict__
     const int nq = cnt[C_NQUERY];
     const int n = cnt[C_NLIVE];
     if (q0 >= nq || n <= 1) return;  // uniform per wave
-    const int root = subtree_root(node, n, part, part_log);
-    if (root < 0) return;
+    long long at;
+    const int root = subtree_link(box, part, part_log, &at);
+    if (root == kNoNode) return;
     const int nl = nq - q0 < kGuardQ ? (int)(nq - q0) : kGuardQ;
+    int size = nl, qn = 0;  // wave-uniform
+    bool at_leaf = false;
     if (lane < nl) {
         const int a = list[q0 + lane];
-        qid[w][lane] = make_int4(a, m.i[a], m.j[a], m.k[a]);
-        qbox[w][lane][0] = fbox[2 * (long long)a];
-        qbox[w][lane][1] = fbox[2 * (long long)a + 1];
-        stk[w][lane] = make_int2(lane, root);
+        const int i0 = m.i[a], i1 = m.j[a], i2 = m.k[a];
+        const float4 p = m.p[i0], q = m.p[i1], r = m.p[i2];
+        const float4 lo = make_float4(fminf(p.x, fminf(q.x, r.x)), fminf(p.y, fminf(q.y, r.y)),
+                                      fminf(p.z, fminf(q.z, r.z)), 0.0f);
+        const float4 hi = make_float4(fmaxf(p.x, fmaxf(q.x, r.x)), fmaxf(p.y, fmaxf(q.y, r.y)),
+                                      fmaxf(p.z, fmaxf(q.z, r.z)), 0.0f);
+        qid[w][lane] = make_int4(a, i0, i1, i2);
+        qbox[w][lane][0] = lo;
+        qbox[w][lane][1] = hi;
+        if (root >= 0) stk[w][lane] = make_int2(lane, root);
+        else at_leaf = overlap(lo, hi, box[at], box[at + 1]);
+    }
+    if (root < 0) {  // the whole part is one leaf
+        size = 0;
+        const uint64_t lm = __ballot(at_leaf);
+        if (at_leaf) pq[w][lanes_below(lm)] = make_int2(lane, ~root);
+        qn = (int)__popcll(lm);
     }
     wave_sync();
-    int size = nl, qn = 0;  // wave-uniform
     // bounds of a valid tree; walk_cap > 0 lowers them (tests of the error path)
     long long max_steps = (long long)nl * (2LL * n - 1), max_visits = 2LL * n;
     if (walk_cap > 0) {
@@ -1786,43 +1852,48 @@ __device__ __forceinline__ void guard_query_body(Mesh m, const int* __restrict__
             x = e.y;
         }
         size -= take;
-        int c0 = -1, c1 = -1, esc = -1, leaf = -1;
+        int c0 = -1, c1 = -1, f0 = -1, f1 = -1;
         float4 qlo = make_float4(0.f, 0.f, 0.f, 0.f), qhi = qlo;
         if (x >= 0) {
-            const float4 lo = node[2 * (long long)x], hi = node[2 * (long long)x + 1];
-            const int r = x < n - 1 ? right[x] : -1;
+            const float4* b = box + 4 * (long long)x;
+            const float4 llo = b[0], lhi = b[1], rlo = b[2], rhi = b[3];
             qlo = qbox[w][l][0];
             qhi = qbox[w][l][1];
-            if (overlap(qlo, qhi, lo, hi)) {
-                if (x >= n - 1) {
-                    leaf = __float_as_int(lo.w);
-                } else {
-                    c0 = __float_as_int(lo.w);
-                    c1 = r;
-                    esc = __float_as_int(hi.w);
-                }
+            if (overlap(qlo, qhi, llo, lhi)) {
+                const int k = __float_as_int(llo.w);
+                if (k >= 0) c0 = k;
+                else f0 = ~k;
+            }
+            if (overlap(qlo, qhi, rlo, rhi)) {
+                const int k = __float_as_int(rlo.w);
+                if (k >= 0) c1 = k;
+                else f1 = ~k;
             }
         }
         wave_sync();  // every pop has read its entry before pushes reuse the slots
-        const uint64_t lm = __ballot(leaf >= 0);
-        if (leaf >= 0) pq[w][qn + lanes_below(lm)] = make_int2(l, leaf);
-        qn += (int)__popcll(lm);
-        const uint64_t pm = __ballot(c0 >= 0);
-        const int below = lanes_below(pm);
-        const bool fits = size + 2 * (below + 1) <= kStackCap;  // pushes that fit form a prefix
-        if (c0 >= 0) {
-            if (fits) {
-                stk[w][size + 2 * below] = make_int2(l, c0);
-                stk[w][size + 2 * below + 1] = make_int2(l, c1);
-            } else {
-                const int4 id = qid[w][l];
-                guard_walk_subtree<kExact>(m, changed, node, n, c0, esc, qlo, qhi, id.x, id.y, id.z, id.w, epsilon,
-                                           flagged, u, err, max_visits);
+        const uint64_t l0 = __ballot(f0 >= 0), l1 = __ballot(f1 >= 0);
+        if (f0 >= 0) pq[w][qn + lanes_below(l0)] = make_int2(l, f0);
+        qn += (int)__popcll(l0);
+        if (f1 >= 0) pq[w][qn + lanes_below(l1)] = make_int2(l, f1);
+        qn += (int)__popcll(l1);
+        const uint64_t m0 = __ballot(c0 >= 0), m1 = __ballot(c1 >= 0);
+        const int p0 = size + lanes_below(m0), p1 = size + (int)__popcll(m0) + lanes_below(m1);
+        if (c0 >= 0 && p0 < kStackCap) stk[w][p0] = make_int2(l, c0);
+        if (c1 >= 0 && p1 < kStackCap) stk[w][p1] = make_int2(l, c1);
+        const int full = size + (int)__popcll(m0) + (int)__popcll(m1);
+        if (full > kStackCap) {  // wave-uniform: pushes that fit form a prefix
+            const bool o0 = c0 >= 0 && p0 >= kStackCap, o1 = c1 >= 0 && p1 >= kStackCap;
+            for (int k = 0; k < 2; ++k) {
+                if (k == 0 ? o0 : o1) {
+                    const int4 id = qid[w][l];
+                    guard_walk_subtree<kExact>(m, changed, box, slot, k == 0 ? c0 : c1, qlo, qhi, id.x, id.y, id.z,
+                                               id.w, epsilon, flagged, u, err, max_visits);
+                }
             }
         }
-        size += 2 * (int)__popcll(__ballot(c0 >= 0 && fits));
+        size = min(full, kStackCap);
         wave_sync();
-        if (qn >= kWave) {
+        while (qn >= kWave) {
             const int2 e = pq[w][qn - kWave + lane];
             const int4 id = qid[w][e.x];
             if (guard_candidate<kExact>(m, changed, id.x, id.y, id.z, id.w, e.y))
@@ -1841,9 +1912,8 @@ __device__ __forceinline__ void guard_query_body(Mesh m, const int* __restrict__
 
 #define PAMO_GUARD_PARAMS                                                                                  \
     Mesh m, const int* __restrict__ list, const int* __restrict__ cnt, const uint8_t* __restrict__ changed,   \
-        const float4* __restrict__ fbox, const float4* __restrict__ node, const int* __restrict__ right,       \
-        float epsilon, uint8_t* __restrict__ flagged, Undecided u, int part_log, int* err, long long walk_cap
-#define PAMO_GUARD_ARGS m, list, cnt, changed, fbox, node, right, epsilon, flagged, u, part_log, err, walk_cap
+        const float4* __restrict__ box, const int* __restrict__ slot, float epsilon, uint8_t* __restrict__ flagged, Undecided u, int part_log, int* err, long long walk_cap
+#define PAMO_GUARD_ARGS m, list, cnt, changed, box, slot, epsilon, flagged, u, part_log, err, walk_cap
 
 template <int kStackCap, bool kExact>
 __global__ void __launch_bounds__(kBlock) guard_query_k(PAMO_GUARD_PARAMS) {
@@ -2032,25 +2102,77 @@ __global__ void __launch_bounds__(kCentThreads) centroid_seq_k(const float* __re
 // look-back scan, and writes the compacted list and its count, where the
 // round used a flag kernel, a scan and a compaction kernel.
 
-// Guard queries: the changed live faces among the tree's leaves, in leaf
-// order (a carried tree's dead leaves hold the sentinel nT).
-struct QueryListOp {
-    static constexpr int kIpt = 4;
-    const uint32_t* val;
-    const uint8_t* changed;
-    const int* ti;
-    int nT;
-    int* list;
-    int* cnt;
-    __device__ int count(long long s) const {
-        const int f = s < cnt[C_NLIVE] ? (int)val[s] : nT;
-        return (f < nT && changed[f] && ti[f] != -1) ? 1 : 0;
+// The leaves of the guard tree before a guard, one launch: the carried leaves'
+// faces renumbered (carry: fpos, the positions of the last compaction of nOld
+// faces; a removed face's leaf takes nT and stays empty), the faces' boxes,
+// the flags cleared, the in-block node boxes (see box_tab_k), and the
+// queries -- the changed live faces -- listed in leaf order by a look-back scan
+// over the blocks (which therefore take their numbers from its ticket).
+// Every face live at the round's start was live at the previous one's, hence is
+// a leaf; a face that no leaf holds is in no ring, and its flag is not read.
+__global__ void __launch_bounds__(kBlock) guard_leaves_k(Mesh m, int nT, uint32_t* __restrict__ val, int carry,
+                                                         const int* __restrict__ fpos, int nOld,
+                                                         const uint8_t* __restrict__ changed,
+                                                         uint8_t* __restrict__ flagged, int* __restrict__ cnt,
+                                                         float4* __restrict__ box, const int* __restrict__ slot,
+                                                         const int2* __restrict__ range, float4* __restrict__ pre,
+                                                         float4* __restrict__ suf, float4* __restrict__ blk,
+                                                         int* __restrict__ list, unsigned long long* __restrict__ state,
+                                                         unsigned* __restrict__ ticket, int* __restrict__ err,
+                                                         unsigned epoch, unsigned tick0) {
+    __shared__ BoxTab T;
+    __shared__ int lds[4];
+    __shared__ int sh[2];
+    if (threadIdx.x == 0) sh[0] = (int)(atomicAdd(ticket, 1u) - tick0);
+    __syncthreads();
+    const int tile = sh[0];
+    if ((unsigned)tile >= gridDim.x) {  // ticket out of step with the host's count
+        if (threadIdx.x == 0) atomicOr(err, 2);
+        return;
     }
-    __device__ void emit(long long s, int v, int pos) const {
-        if (v) list[pos] = (int)val[s];
+    const int n = cnt[C_NLIVE];
+    const int t = threadIdx.x, s = tile * kBlock + t;
+    const float inf = __builtin_huge_valf();
+    float4 a = make_float4(inf, inf, inf, 0.0f), b = make_float4(-inf, -inf, -inf, 0.0f);
+    int f = nT, query = 0;
+    if (s < n) {
+        f = (int)val[s];
+        if (carry) {
+            const int old = f;
+            f = nT;
+            if (old < nOld) {
+                const int q = fpos[old];
+                if (fpos[old + 1] > q) f = q;
+            }
+            val[s] = (uint32_t)f;
+        }
+        if (f < nT) {
+            face_box(m, f, a, b);
+            flagged[f] = 0;
+            query = changed[f] && m.i[f] != -1 ? 1 : 0;
+        }
+        if (n > 1) {
+            float4* q = box + 2 * (long long)slot[n - 1 + s];
+            q[0] = make_float4(a.x, a.y, a.z, __int_as_float(~f));
+            const float hv[3] = {b.x, b.y, b.z};
+            store_xyz(q + 1, hv);
+        }
     }
-    __device__ void done(int total) const { cnt[C_NQUERY] = total; }
-};
+    int total;
+    const int ex = block_exclusive_scan(query, lds, total);
+    if (t < kWave) {
+        const int before = lb_prefix(tile, total, state, err, epoch);
+        if (t == 0) {
+            sh[1] = before;
+            if (tile == (int)gridDim.x - 1) cnt[C_NQUERY] = before + total;
+        }
+    }
+    __syncthreads();
+    if (query) list[sh[1] + ex] = f;
+    if (tile * kBlock >= n) return;
+    tab_build(T, t, a, b);
+    tab_store(T, tile, t, n, pre, suf, blk, n, range, slot, box);
+}
 
 // Regular collapse records in edge order (select_collapse_k's flags).
 struct CollapseListOp {
@@ -2141,7 +2263,7 @@ struct UndoListOp {
 // Compaction of the mesh (pamo/__init__.py:163-167): item t moves point t
 // to pts_map[t] if it is occupied, and face t to its position among the
 // live faces with renumbered corners; fpos[t] receives that position for
-// t <= nT (fpos[nT] = live faces), which the guard-tree carry reads.  Items
+// t <= nT (fpos[nT] = live faces), which the guard tree's carry reads.  Items
 // cover max(nP, nT) + 1.
 struct CompactMeshOp {
     static constexpr int kIpt = 2;
@@ -2157,7 +2279,6 @@ struct CompactMeshOp {
     int* cnt;
     __device__ int count(long long t) const { return (t < nT && m.i[t] >= 0) ? 1 : 0; }
     __device__ void emit(long long t, int v, int pos) const {
-        if (t == 0) cnt[C_LIVE_LEAVES] = 0;  // counted by carry_leaves_k next
         if (t < nP && occ[t]) np[pts_map[t]] = m.p[t];
         if (t == nP) cnt[C_NV] = pts_map[nP];
         if (t <= nT) fpos[t] = pos;

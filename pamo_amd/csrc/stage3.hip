@@ -299,7 +299,7 @@ __global__ void edge_items_k(const float4* __restrict__ x, const int2* __restric
 // ------------------------------------------------------------ closest point on the input surface (B4)
 // Nearest triangle by branch and bound over the GT tree: nearer child first,
 // subtrees whose box is no closer than the best distance so far skipped, over
-// the tree's child-pair records with the far children on an LDS stack.
+// the tree's child pairs with the far children on an LDS stack.
 __global__ void __launch_bounds__(kWave) closest_point_k(const float4* __restrict__ x, int nV, TreeView T,
                                                         const float4* __restrict__ gv, const int4* __restrict__ gf,
                                                         float4* __restrict__ target, int* err) {
@@ -342,8 +342,8 @@ __global__ void __launch_bounds__(kWave) closest_point_k(const float4* __restric
                 cur = n;
                 continue;
             }
-            const float4 la = T.pre[2 * (long long)cur], lb = T.pre[2 * (long long)cur + 1];
-            const float4 ra = T.suf[2 * (long long)cur], rb = T.suf[2 * (long long)cur + 1];
+            const float4* pair = T.box + 4 * (long long)cur;
+            const float4 la = pair[0], lb = pair[1], ra = pair[2], rb = pair[3];
             const float dl = box_dist2(p, la, lb), dr = box_dist2(p, ra, rb);
             const bool left_first = dl <= dr;
             const float dn = left_first ? dl : dr, df = left_first ? dr : dl;
@@ -364,6 +364,10 @@ __global__ void __launch_bounds__(kWave) closest_point_k(const float4* __restric
             // equally near points the first in the order of the visits is kept, as without the stack)
             best = 1e18f;
             bestp = mk(1e9f, 1e9f, 1e9f);
+            auto bd = [&](int node) {  // (the root, which has no box, is entered)
+                if (node == 0) return 0.0f;
+                return box_dist2(p, T.box[2 * (long long)T.slot[node]], T.box[2 * (long long)T.slot[node] + 1]);
+            };
             int prev = -1;
             cur = 0;
             const long long max_steps = 3LL * (2LL * n - 1) + 1;
@@ -372,24 +376,21 @@ __global__ void __launch_bounds__(kWave) closest_point_k(const float4* __restric
                     walk_overrun(err);
                     break;
                 }
-                const int par = cur == 0 ? -1 : T.parent[cur];
+                const int par = cur == 0 ? -1 : T.slot[cur] >> 1;
                 int next;
                 if (prev == par) {
-                    if (box_dist2(p, T.box[2 * (long long)cur], T.box[2 * (long long)cur + 1]) >= best) next = par;
+                    if (bd(cur) >= best) next = par;
                     else if (cur >= n - 1) {
                         leaf((int)T.val[cur - (n - 1)]);
                         next = par;
                     } else {
-                        int l = T.left[cur], r = T.right[cur];
-                        float dl = box_dist2(p, T.box[2 * (long long)l], T.box[2 * (long long)l + 1]);
-                        float dr = box_dist2(p, T.box[2 * (long long)r], T.box[2 * (long long)r + 1]);
-                        next = dl <= dr ? l : r;
+                        const int l = T.left[cur], r = T.right[cur];
+                        next = bd(l) <= bd(r) ? l : r;
                     }
                 } else {
-                    int l = T.left[cur], r = T.right[cur];
-                    float dl = box_dist2(p, T.box[2 * (long long)l], T.box[2 * (long long)l + 1]);
-                    float dr = box_dist2(p, T.box[2 * (long long)r], T.box[2 * (long long)r + 1]);
-                    int first = dl <= dr ? l : r, second = dl <= dr ? r : l;
+                    const int l = T.left[cur], r = T.right[cur];
+                    const bool left_first = bd(l) <= bd(r);
+                    const int first = left_first ? l : r, second = left_first ? r : l;
                     next = prev == first ? second : par;
                 }
                 prev = cur;
@@ -406,7 +407,7 @@ __global__ void __launch_bounds__(kWave) closest_point_k(const float4* __restric
 // holding it whose box overlaps x0 +- (2r + d_hat); EE = edge e0 against every
 // edge e1 > e0 sharing no vertex whose box overlaps e0's box grown by the same
 // amount; a pair is kept when its classified distance is <= 2r + d_hat.
-constexpr int kDetQ = 128;     // per-wave pair queue (< 64 pending + one append of <= 64)
+constexpr int kDetQ = 192;     // per-wave pair queue (< 64 pending + one append of <= 128)
 constexpr int kDetW = 4;       // queries per wave
 constexpr int kDetStack = 512; // frontier entries per wave
 
@@ -475,31 +476,41 @@ __device__ __forceinline__ void det_emit(bool keep, int4 ids, int type, const De
     }
 }
 
-// Stackless walk below internal node x (from its left child until x's
-// escape), classifying and appending in this lane.
+// Stackless walk below internal node `top`, classifying and appending in
+// this lane: a node's children in turn, back up by the slots.
 template <bool kPT>
 __device__ __forceinline__ void det_walk_subtree(const float4* __restrict__ x, const int4* __restrict__ tri,
-                                              const int2* __restrict__ edge, const float4* __restrict__ node,
-                                              int n_leaves, int cur, int stop, V3 lo, V3 hi, int q, float thr,
-                                              float ee_thres, const DetOut& o, int wid, int* wcnt, int* err) {
-    for (long long visits = 0; cur != stop; ++visits) {
-        if (visits >= 2LL * n_leaves || cur < 0) {
+                                                 const int2* __restrict__ edge, const float4* __restrict__ box,
+                                                 const int* __restrict__ slot, int n_leaves, int top, V3 lo, V3 hi,
+                                                 int q, float thr, float ee_thres, const DetOut& o, int wid, int* wcnt,
+                                                 int* err) {
+    int cur = top, side = 0;
+    for (long long visits = 0;; ++visits) {
+        if (visits >= 6LL * n_leaves || cur < 0) {
             walk_overrun(err);
             return;
         }
-        const float4 blo = node[2 * (long long)cur], bhi = node[2 * (long long)cur + 1];
-        const int lw = __float_as_int(blo.w), esc = __float_as_int(bhi.w);
-        if (box_hit(lo, hi, blo, bhi)) {
-            if (cur >= n_leaves - 1) {
-                int4 ids = make_int4(0, 0, 0, 0);
-                const bool keep = (kPT || lw > q) && det_pair<kPT>(x, tri, edge, q, lw, thr, ee_thres, ids);
-                det_emit(keep, ids, kPT ? BLOCK_PT : BLOCK_EE, o, wid, wcnt);
-                cur = esc;
-            } else {
-                cur = lw;
-            }
+        if (side == 2) {  // both children done
+            if (cur == top) return;
+            const int up = slot[cur];
+            cur = up >> 1;
+            side = (up & 1) + 1;
+            continue;
+        }
+        const float4 blo = box[4 * (long long)cur + 2 * side], bhi = box[4 * (long long)cur + 2 * side + 1];
+        if (!box_hit(lo, hi, blo, bhi)) {
+            ++side;
+            continue;
+        }
+        const int link = __float_as_int(blo.w);
+        if (link >= 0) {
+            cur = link;
+            side = 0;
         } else {
-            cur = esc;
+            int4 ids = make_int4(0, 0, 0, 0);
+            const bool keep = (kPT || ~link > q) && det_pair<kPT>(x, tri, edge, q, ~link, thr, ee_thres, ids);
+            det_emit(keep, ids, kPT ? BLOCK_PT : BLOCK_EE, o, wid, wcnt);
+            ++side;
         }
     }
 }
@@ -510,16 +521,17 @@ __device__ __forceinline__ void det_walk_subtree(const float4* __restrict__ x, c
 // counter (contact_detection.py:120-214).
 //
 // A wave serves kDetW queries with one shared LIFO frontier of
-// (query, node) entries in LDS: each step pops up to 64 entries, one per
-// lane, pushes both children of overlapping internal nodes and queues
-// overlapping leaves; the queue is classified 64 pairs at a time, and output
-// slots are reserved with one atomic per wave.  When the frontier is full, a
-// lane walks the rest of its subtree by escape links.
+// (query, internal node) entries in LDS: each step pops up to 64 entries, one
+// per lane, reads both children's boxes, pushes the overlapping internal ones
+// and queues the overlapping leaves; the queue is classified 64 pairs at a
+// time, and output slots are reserved with one atomic per wave.  When the
+// frontier is full, a lane walks the rest of its subtree by itself.
 template <bool kPT>
 __global__ void __launch_bounds__(kB) detect_k(const float4* __restrict__ x, int nq, const int4* __restrict__ tri,
-                                               const int2* __restrict__ edge, const float4* __restrict__ node,
-                                               const int* __restrict__ right, int n_leaves, float d_hat,
-                                               float radius, float ee_thres, DetOut o, int* err) {
+                                               const int2* __restrict__ edge, const float4* __restrict__ box,
+                                               const int* __restrict__ slot, const uint32_t* __restrict__ val,
+                                               int n_leaves, float d_hat, float radius, float ee_thres, DetOut o,
+                                               int* err) {
     constexpr int kW = kB / kWave;
     __shared__ int2 stk[kW][kDetStack];
     __shared__ int2 pq[kW][kDetQ];
@@ -533,6 +545,8 @@ __global__ void __launch_bounds__(kB) detect_k(const float4* __restrict__ x, int
     if (lane == 0) wcnt[w] = 0;
     const int nl = nq - q0 < kDetW ? (int)(nq - q0) : kDetW;
     const float thr = 2.0f * radius + d_hat;
+    int size = nl, qn = 0;  // wave-uniform
+    bool one = false;
     if (lane < nl) {
         const int q = (int)q0 + lane;
         V3 lo, hi;
@@ -549,6 +563,14 @@ __global__ void __launch_bounds__(kB) detect_k(const float4* __restrict__ x, int
         qbox[w][lane][0] = make_float4(lo.x, lo.y, lo.z, 0.0f);
         qbox[w][lane][1] = make_float4(hi.x, hi.y, hi.z, 0.0f);
         stk[w][lane] = make_int2(lane, 0);  // root
+        // a tree of one leaf has no pairs: the distance test alone decides
+        one = n_leaves == 1 && (kPT || (int)val[0] > q);
+    }
+    if (n_leaves == 1) {
+        size = 0;
+        const uint64_t lm = __ballot(one);
+        if (one) pq[w][lanes_below(lm)] = make_int2(lane, (int)val[0]);
+        qn = (int)__popcll(lm);
     }
     wave_sync();
     // emits the classified pairs of pq[w][qn - take, qn) with one atomic per wave
@@ -561,7 +583,6 @@ __global__ void __launch_bounds__(kB) detect_k(const float4* __restrict__ x, int
         }
         det_emit(keep, ids, kPT ? BLOCK_PT : BLOCK_EE, o, wid, &wcnt[w]);
     };
-    int size = nl, qn = 0;  // wave-uniform
     const long long max_steps = (long long)nl * (2LL * n_leaves - 1);
     for (long long steps = 0; size > 0; ++steps) {
         if (steps >= max_steps) {  // wave-uniform
@@ -577,44 +598,46 @@ __global__ void __launch_bounds__(kB) detect_k(const float4* __restrict__ x, int
             cur = e.y;
         }
         size -= take;
-        int c0 = -1, c1 = -1, esc = -1, leaf = -1;
+        int c0 = -1, c1 = -1, f0 = -1, f1 = -1;
         V3 lo = mk(0.f, 0.f, 0.f), hi = lo;
         if (cur >= 0) {
-            const float4 blo = node[2 * (long long)cur], bhi = node[2 * (long long)cur + 1];
-            const int r = cur < n_leaves - 1 ? right[cur] : -1;
+            const float4* b = box + 4 * (long long)cur;
+            const float4 llo = b[0], lhi = b[1], rlo = b[2], rhi = b[3];
             const float4 ql = qbox[w][l][0], qh = qbox[w][l][1];
             lo = mk(ql.x, ql.y, ql.z);
             hi = mk(qh.x, qh.y, qh.z);
-            if (box_hit(lo, hi, blo, bhi)) {
-                const int lw = __float_as_int(blo.w);
-                if (cur >= n_leaves - 1) {
-                    if (kPT || lw > (int)q0 + l) leaf = lw;
-                } else {
-                    c0 = lw;
-                    c1 = r;
-                    esc = __float_as_int(bhi.w);
-                }
+            if (box_hit(lo, hi, llo, lhi)) {
+                const int k = __float_as_int(llo.w);
+                if (k >= 0) c0 = k;
+                else if (kPT || ~k > (int)q0 + l) f0 = ~k;
+            }
+            if (box_hit(lo, hi, rlo, rhi)) {
+                const int k = __float_as_int(rlo.w);
+                if (k >= 0) c1 = k;
+                else if (kPT || ~k > (int)q0 + l) f1 = ~k;
             }
         }
         wave_sync();  // every pop has read its entry before pushes reuse the slots
-        const uint64_t lm = __ballot(leaf >= 0);
-        if (leaf >= 0) pq[w][qn + lanes_below(lm)] = make_int2(l, leaf);
-        qn += (int)__popcll(lm);
-        const uint64_t pm = __ballot(c0 >= 0);
-        const int below = lanes_below(pm);
-        const bool fits = size + 2 * (below + 1) <= kDetStack;  // pushes that fit form a prefix
-        if (c0 >= 0) {
-            if (fits) {
-                stk[w][size + 2 * below] = make_int2(l, c0);
-                stk[w][size + 2 * below + 1] = make_int2(l, c1);
-            } else {
-                det_walk_subtree<kPT>(x, tri, edge, node, n_leaves, c0, esc, lo, hi, (int)q0 + l, thr, ee_thres,
-                                      o, wid, &wcnt[w], err);
-            }
+        const uint64_t l0 = __ballot(f0 >= 0), l1 = __ballot(f1 >= 0);
+        if (f0 >= 0) pq[w][qn + lanes_below(l0)] = make_int2(l, f0);
+        qn += (int)__popcll(l0);
+        if (f1 >= 0) pq[w][qn + lanes_below(l1)] = make_int2(l, f1);
+        qn += (int)__popcll(l1);
+        const uint64_t m0 = __ballot(c0 >= 0), m1 = __ballot(c1 >= 0);
+        const int p0 = size + lanes_below(m0), p1 = size + (int)__popcll(m0) + lanes_below(m1);
+        if (c0 >= 0 && p0 < kDetStack) stk[w][p0] = make_int2(l, c0);
+        if (c1 >= 0 && p1 < kDetStack) stk[w][p1] = make_int2(l, c1);
+        const int full = size + (int)__popcll(m0) + (int)__popcll(m1);
+        if (full > kDetStack) {  // wave-uniform: pushes that fit form a prefix
+            const bool o0 = c0 >= 0 && p0 >= kDetStack, o1 = c1 >= 0 && p1 >= kDetStack;
+            for (int k = 0; k < 2; ++k)
+                if (k == 0 ? o0 : o1)
+                    det_walk_subtree<kPT>(x, tri, edge, box, slot, n_leaves, k == 0 ? c0 : c1, lo, hi, (int)q0 + l, thr,
+                                          ee_thres, o, wid, &wcnt[w], err);
         }
-        size += 2 * (int)__popcll(__ballot(c0 >= 0 && fits));
+        size = min(full, kDetStack);
         wave_sync();
-        if (qn >= kWave) {
+        while (qn >= kWave) {
             classify(qn, kWave);
             qn -= kWave;
             wave_sync();
@@ -1720,11 +1743,11 @@ static int detect_contacts(Ctx& c, int& nC) {
             PAMO_TRY(fill(c.wave_count, 0, n_waves + 1, c.stream));
             DetOut o{c.ccount, cap, c.cidx, c.ctype1, c.ctag, c.wave_count, 0};
             L3(detect_k<true>, pt_blocks * kB, (const float4*)c.q, c.nV, (const int4*)c.tri, (const int2*)c.edge,
-               (const float4*)c.tri_tree.box, (const int*)c.tri_tree.right, c.nF, c.P.d_hat, c.radius, c.P.ee_thres,
+               (const float4*)c.tri_tree.box, (const int*)c.tri_tree.slot, (const uint32_t*)c.tri_tree.val, c.nF, c.P.d_hat, c.radius, c.P.ee_thres,
                o, c.ccount + 1);
             o.wave0 = pt_waves;
             L3(detect_k<false>, ee_blocks * kB, (const float4*)c.q, c.nE, (const int4*)c.tri, (const int2*)c.edge,
-               (const float4*)c.edge_tree.box, (const int*)c.edge_tree.right, c.nE, c.P.d_hat, c.radius,
+               (const float4*)c.edge_tree.box, (const int*)c.edge_tree.slot, (const uint32_t*)c.edge_tree.val, c.nE, c.P.d_hat, c.radius,
                c.P.ee_thres, o, c.ccount + 1);
             PAMO_HIP(hipMemcpyAsync(c.hcount, c.ccount, 3 * sizeof(int), hipMemcpyDeviceToHost, c.stream));
             PAMO_HIP(hipStreamSynchronize(c.stream));
@@ -2324,7 +2347,6 @@ int pamo_s3_set_target(pamo_s3* s, const float* d_gt_v, int n_gt_v, const int* d
                        (const float4*)c.gt_v, (const int4*)c.gt_f, n_gt_f, 0.0f, c.gt_tree.item);
     PAMO_HIP(hipGetLastError());
     PAMO_TRY(pamo::s3::tree_build(c.gt_tree, n_gt_f, c.ws, c.stream));
-    PAMO_TRY(pamo::s3::tree_pairs(c.gt_tree, c.stream));
     PAMO_HIP(hipStreamSynchronize(c.stream));
     return 0;
 }
