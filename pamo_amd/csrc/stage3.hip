@@ -407,7 +407,7 @@ __global__ void __launch_bounds__(kWave) closest_point_k(const float4* __restric
 // holding it whose box overlaps x0 +- (2r + d_hat); EE = edge e0 against every
 // edge e1 > e0 sharing no vertex whose box overlaps e0's box grown by the same
 // amount; a pair is kept when its classified distance is <= 2r + d_hat.
-constexpr int kDetQ = 192;     // per-wave pair queue (< 64 pending + one append of <= 128)
+constexpr int kDetQ = 128;     // per-wave pair queue (< 64 pending + one append of <= 64)
 constexpr int kDetW = 4;       // queries per wave
 constexpr int kDetStack = 512; // frontier entries per wave
 
@@ -476,42 +476,41 @@ __device__ __forceinline__ void det_emit(bool keep, int4 ids, int type, const De
     }
 }
 
-// Stackless walk below internal node `top`, classifying and appending in
-// this lane: a node's children in turn, back up by the slots.
+// Stackless walk below internal node `top`, classifying and appending in this
+// lane: one node a step in depth-first order, left child first; past a
+// subtree's end the way up is the slots.
 template <bool kPT>
 __device__ __forceinline__ void det_walk_subtree(const float4* __restrict__ x, const int4* __restrict__ tri,
                                                  const int2* __restrict__ edge, const float4* __restrict__ box,
                                                  const int* __restrict__ slot, int n_leaves, int top, V3 lo, V3 hi,
                                                  int q, float thr, float ee_thres, const DetOut& o, int wid, int* wcnt,
                                                  int* err) {
-    int cur = top, side = 0;
+    int at = 2 * top;  // a node by its slot
     for (long long visits = 0;; ++visits) {
-        if (visits >= 6LL * n_leaves || cur < 0) {
+        if (visits >= 2LL * n_leaves) {
             walk_overrun(err);
             return;
         }
-        if (side == 2) {  // both children done
-            if (cur == top) return;
-            const int up = slot[cur];
-            cur = up >> 1;
-            side = (up & 1) + 1;
-            continue;
-        }
-        const float4 blo = box[4 * (long long)cur + 2 * side], bhi = box[4 * (long long)cur + 2 * side + 1];
-        if (!box_hit(lo, hi, blo, bhi)) {
-            ++side;
-            continue;
-        }
-        const int link = __float_as_int(blo.w);
-        if (link >= 0) {
-            cur = link;
-            side = 0;
-        } else {
+        const float4 blo = box[2 * (long long)at], bhi = box[2 * (long long)at + 1];
+        if (box_hit(lo, hi, blo, bhi)) {
+            const int link = __float_as_int(blo.w);
+            if (link >= 0) {
+                at = 2 * link;
+                continue;
+            }
             int4 ids = make_int4(0, 0, 0, 0);
             const bool keep = (kPT || ~link > q) && det_pair<kPT>(x, tri, edge, q, ~link, thr, ee_thres, ids);
             det_emit(keep, ids, kPT ? BLOCK_PT : BLOCK_EE, o, wid, wcnt);
-            ++side;
         }
+        for (int up = 0; at & 1; ++up) {  // to the next node that is not below a finished one
+            if ((at >> 1) == top) return;
+            if (up >= n_leaves) {
+                walk_overrun(err);
+                return;
+            }
+            at = slot[at >> 1];
+        }
+        ++at;
     }
 }
 
@@ -520,12 +519,18 @@ __device__ __forceinline__ void det_walk_subtree(const float4* __restrict__ x, c
 // thr = 2 r + d_hat of the query's box; classified contacts are appended at
 // counter (contact_detection.py:120-214).
 //
-// A wave serves kDetW queries with one shared LIFO frontier of
-// (query, internal node) entries in LDS: each step pops up to 64 entries, one
-// per lane, reads both children's boxes, pushes the overlapping internal ones
-// and queues the overlapping leaves; the queue is classified 64 pairs at a
-// time, and output slots are reserved with one atomic per wave.  When the
-// frontier is full, a lane walks the rest of its subtree by itself.
+// A wave serves kDetW queries with one shared LIFO frontier of (query, node)
+// entries in LDS, a node being its slot (-1: the root, which is entered
+// untested): each step pops up to 64 entries, one per lane, pushes both
+// children of overlapping internal nodes and queues overlapping leaves; the
+// queue is classified 64 pairs at a time, and output slots are reserved with
+// one atomic per wave.  When the frontier is full, a lane walks the rest of
+// its subtree by itself.
+//
+// The order of the visits is the order of the contacts, and so of the sums
+// over a vertex's contacts: testing both children at the pop of their parent
+// saves a step a level but lists them in another order, which a long solve
+// with many contacts turns into another surface (0.8 % at 300 ms of it).
 template <bool kPT>
 __global__ void __launch_bounds__(kB) detect_k(const float4* __restrict__ x, int nq, const int4* __restrict__ tri,
                                                const int2* __restrict__ edge, const float4* __restrict__ box,
@@ -562,7 +567,7 @@ __global__ void __launch_bounds__(kB) detect_k(const float4* __restrict__ x, int
         }
         qbox[w][lane][0] = make_float4(lo.x, lo.y, lo.z, 0.0f);
         qbox[w][lane][1] = make_float4(hi.x, hi.y, hi.z, 0.0f);
-        stk[w][lane] = make_int2(lane, 0);  // root
+        stk[w][lane] = make_int2(lane, -1);  // root
         // a tree of one leaf has no pairs: the distance test alone decides
         one = n_leaves == 1 && (kPT || (int)val[0] > q);
     }
@@ -591,53 +596,47 @@ __global__ void __launch_bounds__(kB) detect_k(const float4* __restrict__ x, int
             return;
         }
         const int take = size < kWave ? size : kWave;
-        int l = 0, cur = -1;
+        int l = 0, at = -2;
         if (lane < take) {
             const int2 e = stk[w][size - take + lane];
             l = e.x;
-            cur = e.y;
+            at = e.y;
         }
         size -= take;
-        int c0 = -1, c1 = -1, f0 = -1, f1 = -1;
+        int node = -1, leaf = -1;  // the internal node to open, or the face or edge to test
         V3 lo = mk(0.f, 0.f, 0.f), hi = lo;
-        if (cur >= 0) {
-            const float4* b = box + 4 * (long long)cur;
-            const float4 llo = b[0], lhi = b[1], rlo = b[2], rhi = b[3];
+        if (at >= 0) {
+            const float4 blo = box[2 * (long long)at], bhi = box[2 * (long long)at + 1];
             const float4 ql = qbox[w][l][0], qh = qbox[w][l][1];
             lo = mk(ql.x, ql.y, ql.z);
             hi = mk(qh.x, qh.y, qh.z);
-            if (box_hit(lo, hi, llo, lhi)) {
-                const int k = __float_as_int(llo.w);
-                if (k >= 0) c0 = k;
-                else if (kPT || ~k > (int)q0 + l) f0 = ~k;
+            if (box_hit(lo, hi, blo, bhi)) {
+                const int link = __float_as_int(blo.w);
+                if (link >= 0) node = link;
+                else if (kPT || ~link > (int)q0 + l) leaf = ~link;
             }
-            if (box_hit(lo, hi, rlo, rhi)) {
-                const int k = __float_as_int(rlo.w);
-                if (k >= 0) c1 = k;
-                else if (kPT || ~k > (int)q0 + l) f1 = ~k;
-            }
+        } else if (at == -1) {
+            node = 0;
         }
         wave_sync();  // every pop has read its entry before pushes reuse the slots
-        const uint64_t l0 = __ballot(f0 >= 0), l1 = __ballot(f1 >= 0);
-        if (f0 >= 0) pq[w][qn + lanes_below(l0)] = make_int2(l, f0);
-        qn += (int)__popcll(l0);
-        if (f1 >= 0) pq[w][qn + lanes_below(l1)] = make_int2(l, f1);
-        qn += (int)__popcll(l1);
-        const uint64_t m0 = __ballot(c0 >= 0), m1 = __ballot(c1 >= 0);
-        const int p0 = size + lanes_below(m0), p1 = size + (int)__popcll(m0) + lanes_below(m1);
-        if (c0 >= 0 && p0 < kDetStack) stk[w][p0] = make_int2(l, c0);
-        if (c1 >= 0 && p1 < kDetStack) stk[w][p1] = make_int2(l, c1);
-        const int full = size + (int)__popcll(m0) + (int)__popcll(m1);
-        if (full > kDetStack) {  // wave-uniform: pushes that fit form a prefix
-            const bool o0 = c0 >= 0 && p0 >= kDetStack, o1 = c1 >= 0 && p1 >= kDetStack;
-            for (int k = 0; k < 2; ++k)
-                if (k == 0 ? o0 : o1)
-                    det_walk_subtree<kPT>(x, tri, edge, box, slot, n_leaves, k == 0 ? c0 : c1, lo, hi, (int)q0 + l, thr,
-                                          ee_thres, o, wid, &wcnt[w], err);
+        const uint64_t lm = __ballot(leaf >= 0);
+        if (leaf >= 0) pq[w][qn + lanes_below(lm)] = make_int2(l, leaf);
+        qn += (int)__popcll(lm);
+        const uint64_t pm = __ballot(node >= 0);
+        const int below = lanes_below(pm);
+        const bool fits = size + 2 * (below + 1) <= kDetStack;  // pushes that fit form a prefix
+        if (node >= 0) {
+            if (fits) {
+                stk[w][size + 2 * below] = make_int2(l, 2 * node);
+                stk[w][size + 2 * below + 1] = make_int2(l, 2 * node + 1);
+            } else {
+                det_walk_subtree<kPT>(x, tri, edge, box, slot, n_leaves, node, lo, hi, (int)q0 + l, thr, ee_thres, o,
+                                      wid, &wcnt[w], err);
+            }
         }
-        size = min(full, kDetStack);
+        size += 2 * (int)__popcll(__ballot(node >= 0 && fits));
         wave_sync();
-        while (qn >= kWave) {
+        if (qn >= kWave) {
             classify(qn, kWave);
             qn -= kWave;
             wave_sync();
