@@ -255,20 +255,12 @@ __device__ __forceinline__ int lb_prefix(int tile, int total, unsigned long long
     return excl;
 }
 
+// Tile `tile` of `tiles` of operation op over n items (whole workgroup).
 template <class Op>
-__global__ void __launch_bounds__(kScanBlock) scan_op_k(Op op, long long n, unsigned long long* __restrict__ state,
-                                                        unsigned* __restrict__ ticket, int* __restrict__ err,
-                                                        unsigned epoch, unsigned base) {
+__device__ __forceinline__ void scan_tile(const Op& op, long long n, int tile, int tiles,
+                                          unsigned long long* __restrict__ state, int* __restrict__ err, unsigned epoch,
+                                          int* lds /*[4]*/, int* sh /*[2]*/) {
     constexpr int kIpt = Op::kIpt;
-    __shared__ int lds[4];
-    __shared__ int sh[2];
-    if (threadIdx.x == 0) sh[0] = (int)(atomicAdd(ticket, 1u) - base);
-    __syncthreads();
-    const int tile = sh[0];
-    if ((unsigned)tile >= gridDim.x) {  // ticket out of step with the host's count
-        if (threadIdx.x == 0) atomicOr(err, 2);
-        return;
-    }
     const long long first = ((long long)tile * kScanBlock + threadIdx.x) * kIpt;
     int v[kIpt];
     int s = 0;
@@ -284,7 +276,7 @@ __global__ void __launch_bounds__(kScanBlock) scan_op_k(Op op, long long n, unsi
         const int excl = lb_prefix(tile, total, state, err, epoch);
         if (threadIdx.x == 0) {
             sh[1] = excl;
-            if (tile == (int)gridDim.x - 1) op.done(excl + total);
+            if (tile == tiles - 1) op.done(excl + total);
         }
     }
     __syncthreads();
@@ -297,6 +289,22 @@ __global__ void __launch_bounds__(kScanBlock) scan_op_k(Op op, long long n, unsi
     }
 }
 
+template <class Op>
+__global__ void __launch_bounds__(kScanBlock) scan_op_k(Op op, long long n, unsigned long long* __restrict__ state,
+                                                        unsigned* __restrict__ ticket, int* __restrict__ err,
+                                                        unsigned epoch, unsigned base) {
+    __shared__ int lds[4];
+    __shared__ int sh[2];
+    if (threadIdx.x == 0) sh[0] = (int)(atomicAdd(ticket, 1u) - base);
+    __syncthreads();
+    const int tile = sh[0];
+    if ((unsigned)tile >= gridDim.x) {  // ticket out of step with the host's count
+        if (threadIdx.x == 0) atomicOr(err, 2);
+        return;
+    }
+    scan_tile(op, n, tile, (int)gridDim.x, state, err, epoch, lds, sh);
+}
+
 // out[i] = sum_{j<i} in[j] (in may alias out: a tile reads all its items
 // before writing any).
 struct ScanOp {
@@ -307,6 +315,74 @@ struct ScanOp {
     __device__ void emit(long long i, int, int pos) const { out[i] = pos; }
     __device__ void done(int) const {}
 };
+
+// Up to three independent exclusive scans, in place, in one launch: the
+// tickets run through the first array's tiles, then the second's, then the
+// third's, each with states and a look-back of its own.
+struct ScanSet {
+    int* a[3];
+    long long n[3];
+    int first[4];  // first tile of each array; first[3] = all tiles
+};
+
+__global__ void __launch_bounds__(kScanBlock) scan_set_k(ScanSet q, unsigned long long* __restrict__ state,
+                                                         unsigned* __restrict__ ticket, int* __restrict__ err,
+                                                         unsigned epoch, unsigned base) {
+    __shared__ int lds[4];
+    __shared__ int sh[2];
+    if (threadIdx.x == 0) sh[0] = (int)(atomicAdd(ticket, 1u) - base);
+    __syncthreads();
+    const int all = sh[0];
+    if ((unsigned)all >= gridDim.x) {  // ticket out of step with the host's count
+        if (threadIdx.x == 0) atomicOr(err, 2);
+        return;
+    }
+    const int k = all < q.first[1] ? 0 : (all < q.first[2] ? 1 : 2);
+    int* __restrict__ x = k == 0 ? q.a[0] : (k == 1 ? q.a[1] : q.a[2]);
+    const long long n = k == 0 ? q.n[0] : (k == 1 ? q.n[1] : q.n[2]);
+    const int f = k == 0 ? q.first[0] : (k == 1 ? q.first[1] : q.first[2]);
+    const int tile = all - f;
+    const long long at = ((long long)tile * kScanBlock + threadIdx.x) * kScanIpt;
+    int v[kScanIpt];
+    int s = 0;
+#pragma unroll
+    for (int i = 0; i < kScanIpt; ++i) {
+        v[i] = at + i < n ? x[at + i] : 0;
+        s += v[i];
+    }
+    int total;
+    int ex = block_exclusive_scan(s, lds, total);
+    if (threadIdx.x < kWave) {
+        const int before = lb_prefix(tile, total, state + f, err, epoch);
+        if (threadIdx.x == 0) sh[1] = before;
+    }
+    __syncthreads();
+    ex += sh[1];
+#pragma unroll
+    for (int i = 0; i < kScanIpt; ++i) {
+        if (at + i < n) x[at + i] = ex;
+        ex += v[i];
+    }
+}
+
+// Two scan operations in one launch: A's tiles, then B's, independent.
+template <class A, class B>
+__global__ void __launch_bounds__(kScanBlock) scan_pair_k(A opa, long long na, int tiles_a, B opb, long long nb,
+                                                          unsigned long long* __restrict__ state,
+                                                          unsigned* __restrict__ ticket, int* __restrict__ err,
+                                                          unsigned epoch, unsigned base) {
+    __shared__ int lds[4];
+    __shared__ int sh[2];
+    if (threadIdx.x == 0) sh[0] = (int)(atomicAdd(ticket, 1u) - base);
+    __syncthreads();
+    const int tile = sh[0];
+    if ((unsigned)tile >= gridDim.x) {  // ticket out of step with the host's count
+        if (threadIdx.x == 0) atomicOr(err, 2);
+        return;
+    }
+    if (tile < tiles_a) scan_tile(opa, na, tile, tiles_a, state, err, epoch, lds, sh);
+    else scan_tile(opb, nb, tile - tiles_a, (int)gridDim.x - tiles_a, state + tiles_a, err, epoch, lds, sh);
+}
 
 // Workspace (ints) needed by scan_exclusive for n elements.
 inline long long scan_workspace(long long n) { return (n + kScanTile - 1) / kScanTile + 16; }
@@ -402,6 +478,36 @@ inline int scan_op(const Op& op, long long n, LookbackScan& lb, hipStream_t st, 
     prof_end(prof_id, st);
     PAMO_HIP(hipGetLastError());
     lookback_end(lb, nb);
+    return 0;
+}
+
+// scan_set_k over the arrays given (n items each, in place).
+inline int scan_set(int* a, long long na, int* b, long long nb, int* c, long long nc, LookbackScan& lb, hipStream_t st) {
+    ScanSet q{{a, b, c}, {na, nb, nc}, {0, 0, 0, 0}};
+    for (int k = 0; k < 3; ++k) q.first[k + 1] = q.first[k] + (int)((q.n[k] + kScanTile - 1) / kScanTile);
+    PAMO_TRY(lookback_begin(lb, q.first[3], st));
+    prof_begin(K_SCAN_TILES, 8.0 * (na + nb + nc), st);
+    hipLaunchKernelGGL(scan_set_k, dim3((unsigned)q.first[3]), dim3(kScanBlock), 0, st, q, lb.state, lb.ticket, lb.err,
+                       lb.epoch, lb.base);
+    prof_end(K_SCAN_TILES, st);
+    PAMO_HIP(hipGetLastError());
+    lookback_end(lb, q.first[3]);
+    return 0;
+}
+
+// scan_pair_k over na and nb items (either may be 0: its `done` still runs).
+template <class A, class B>
+inline int scan_pair(const A& opa, long long na, const B& opb, long long nb, LookbackScan& lb, hipStream_t st, int prof_id,
+                     double bytes) {
+    const long long ta = std::max(1LL, (na + kScanBlock * A::kIpt - 1) / (kScanBlock * A::kIpt));
+    const long long tb = std::max(1LL, (nb + kScanBlock * B::kIpt - 1) / (kScanBlock * B::kIpt));
+    PAMO_TRY(lookback_begin(lb, ta + tb, st));
+    prof_begin(prof_id, bytes, st);
+    hipLaunchKernelGGL((scan_pair_k<A, B>), dim3((unsigned)(ta + tb)), dim3(kScanBlock), 0, st, opa, na, (int)ta, opb, nb,
+                       lb.state, lb.ticket, lb.err, lb.epoch, lb.base);
+    prof_end(prof_id, st);
+    PAMO_HIP(hipGetLastError());
+    lookback_end(lb, ta + tb);
     return 0;
 }
 

@@ -102,7 +102,8 @@ struct Ctx {
     // point sized
     float4 *p = nullptr, *op = nullptr, *np = nullptr;
     float4* Q = nullptr;  // 3 per point
-    int *occ = nullptr, *pts_map = nullptr, *ring_off = nullptr, *ring_fill = nullptr;
+    int *occ = nullptr, *pts_map = nullptr, *ring_off = nullptr;
+    int* new_map = nullptr;  // the current round's map before it becomes pts_map
     int* eord_cnt = nullptr;  // edges per smaller endpoint, then the launch-order cursor
     int *undo_list = nullptr, *tmp_undo = nullptr, *undo_prev = nullptr;  // 4 * alloc_pts
     uint32_t* invalid = nullptr;  // epochs (invalid_set_k)
@@ -115,6 +116,8 @@ struct Ctx {
     int *ring_raw = nullptr, *ring_own = nullptr;  // unsorted ring slots and their vertex
     int4* rv = nullptr;   // 3 * alloc_tris
     int* edge_off = nullptr;
+    int4* frank = nullptr;   // per face: its slots among its vertices' rings
+    int2* ferank = nullptr;  // per face: its edges' places among their smaller endpoints'
     uint8_t *changed = nullptr, *flagged = nullptr;
     int *face_scan = nullptr, *qlist = nullptr;
     // LBVH
@@ -130,13 +133,14 @@ struct Ctx {
     uint32_t* edge_cost = nullptr;
     int *esel = nullptr, *recs = nullptr, *pflag = nullptr, *pushed = nullptr;
     int* eord = nullptr;  // edge ids grouped by smaller endpoint (edge-cost launch order)
-    int* erank = nullptr;  // each edge's rank among the edges of its smaller endpoint
+    int* lines = nullptr;  // line-collapse records
     int* shuf = nullptr;
     int* ws = nullptr;
     LookbackScan lb;  // single-launch scans of the round loop
     int* dcnt = nullptr;
     int* hcnt = nullptr;
     // last round, host view
+    int edge_bound = 0;  // edges that the round's launches cover
     int n_pts = 0, n_tris = 0, n_edges = 0, n_rec = 0, n_regular = 0, n_vertices_undo = 0;
     int n_cand = 0;  // records scanned for undo candidates
     int undo_iters = 0;
@@ -229,7 +233,7 @@ static int grow_pts(Ctx& c, size_t n) {
         PAMO_TRY(zero_async(c, c.p, a)); PAMO_TRY(zero_async(c, c.op, a)); PAMO_TRY(zero_async(c, c.np, a));
         PAMO_TRY(zero_async(c, c.Q, 3 * a));
         PAMO_TRY(zero_async(c, c.occ, a + 1)); PAMO_TRY(zero_async(c, c.pts_map, a + 1));
-        PAMO_TRY(zero_async(c, c.ring_off, a + 2)); PAMO_TRY(zero_async(c, c.ring_fill, a + 1));
+        PAMO_TRY(zero_async(c, c.ring_off, a + 2));
         PAMO_TRY(zero_async(c, c.eord_cnt, a + 1));
         PAMO_TRY(zero_async(c, c.undo_list, 4 * a)); PAMO_TRY(zero_async(c, c.tmp_undo, 4 * a));
         PAMO_TRY(zero_async(c, c.undo_prev, 4 * a));
@@ -244,7 +248,7 @@ static int grow_pts(Ctx& c, size_t n) {
     PAMO_TRY(dalloc(&c.occ, a + 1, c.stream));
     PAMO_TRY(dalloc(&c.pts_map, a + 1, c.stream));
     PAMO_TRY(dalloc(&c.ring_off, a + 2, c.stream));
-    PAMO_TRY(dalloc(&c.ring_fill, a + 1, c.stream));
+    PAMO_TRY(dalloc(&c.new_map, a + 1, c.stream));
     PAMO_TRY(dalloc(&c.eord_cnt, a + 1, c.stream));
     PAMO_TRY(dalloc(&c.undo_list, 4 * a, c.stream));
     PAMO_TRY(dalloc(&c.tmp_undo, 4 * a, c.stream));
@@ -265,7 +269,7 @@ static int alloc_edges(Ctx& c, size_t ae) {
     PAMO_TRY(dalloc(&c.pushed, ae + 1, c.stream));
     PAMO_TRY(dalloc(&c.edge_cost, ae + 1, c.stream));
     PAMO_TRY(dalloc(&c.eord, ae + 1, c.stream));
-    PAMO_TRY(dalloc(&c.erank, ae + 1, c.stream));
+    PAMO_TRY(dalloc(&c.lines, ae + 1, c.stream));
     return 0;
 }
 
@@ -298,6 +302,8 @@ static int grow_tris(Ctx& c, size_t n) {
     PAMO_TRY(dalloc(&c.ring_own, 3 * a, c.stream));
     PAMO_TRY(dalloc(&c.rv, 3 * a, c.stream));
     PAMO_TRY(dalloc(&c.edge_off, a + 1, c.stream));
+    PAMO_TRY(dalloc(&c.frank, a, c.stream));
+    PAMO_TRY(dalloc(&c.ferank, a, c.stream));
     PAMO_TRY(dalloc(&c.changed, a, c.stream));
     PAMO_TRY(dalloc(&c.flagged, a, c.stream));
     PAMO_TRY(dalloc(&c.face_scan, a + 1, c.stream));
@@ -339,11 +345,11 @@ static int grow_edges(Ctx& c, size_t n, bool* reallocated = nullptr) {
 }
 
 static void free_all(Ctx& c) {
-    void* ptrs[] = {c.p, c.op, c.np, c.Q, c.occ, c.pts_map, c.ring_off, c.ring_fill, c.eord_cnt, c.undo_list, c.tmp_undo,
+    void* ptrs[] = {c.p, c.op, c.np, c.Q, c.occ, c.pts_map, c.new_map, c.ring_off, c.eord_cnt, c.undo_list, c.tmp_undo,
                     c.undo_prev, c.invalid, c.ti, c.tj, c.tk, c.oi, c.oj, c.ok, c.ni, c.nj, c.nk, c.ring, c.ring_raw, c.ring_own, c.rv,
                     c.edge_off, c.vmin, c.changed, c.flagged, c.face_scan, c.qlist, c.bkey, c.bval, c.bkey2,
                     c.bval2, c.bleft, c.bright, c.bslot, c.brange, c.bbox, c.fbox, c.bpre, c.bsuf, c.blk, c.blkpre,
-                    c.blksuf, c.sblk, c.blktab, c.box_part, c.eu, c.ev, c.edge_cost, c.esel, c.recs, c.pflag, c.pushed, c.eord, c.erank,
+                    c.blksuf, c.sblk, c.blktab, c.box_part, c.eu, c.ev, c.edge_cost, c.esel, c.recs, c.pflag, c.pushed, c.eord, c.lines, c.frank, c.ferank,
                     c.shuf, c.ws, c.dcnt, c.cent_out, c.ulist, c.cent_means};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
@@ -499,10 +505,17 @@ static int run_guard(Ctx& c, int nT, bool refit) {
 // cusimp_free.cu:776-827, whose grid covers the regular-collapse count
 // rounded up to blocks of 512: line-collapse records past it are never
 // candidates).
+//
+// The new vertex ids (the scan of the occupancy) come with the same launch:
+// they stand unless an undo follows, which scans again.  They go to new_map,
+// since the undo reads the previous round's map.
+static int undo_scan(Ctx& c, long long n) {
+    return scan_pair(UndoListOp{c.recs, c.lines, c.ring_off, c.ring, c.eu, c.ev, c.flagged, c.pushed, c.dcnt}, n,
+                     ScanOp{c.occ, c.new_map}, c.n_pts + 1LL, c.lb, c.stream, K_UNDO_CAND, 16.0 * n + 1.0 * c.n_tris);
+}
+
 static int undo_candidates(Ctx& c, int& npushed) {
-    const int n = c.n_cand;
-    PAMO_TRY(scan_op(UndoListOp{c.recs, c.ring_off, c.ring, c.eu, c.ev, c.flagged, c.pushed, c.dcnt}, n, c.lb,
-                     c.stream, K_UNDO_CAND, 16.0 * n + 1.0 * c.n_tris));
+    PAMO_TRY(undo_scan(c, c.n_cand));
     PAMO_TRY(sync_counters(c));
     npushed = c.hcnt[C_PUSHED];
     c.tree_n = c.hcnt[C_NLIVE];  // leaves of the tree this guard used
@@ -515,23 +528,29 @@ static int undo_candidates(Ctx& c, int& npushed) {
 // (cusimp_free.cu:891-1048); the undo-list prologue has already run.
 // Vertex -> face rings in ascending face order (:276-304), the edge list
 // (:306-335), the quadrics (:337-366) and the edge-cost launch order; sets
-// c.n_edges.  Shared by the round and the legacy round.
-// ring_off, ring_fill and eord_cnt must hold zeros (round_init_k).
+// c.edge_bound.  Shared by the round and the legacy round.
+// ring_off and eord_cnt must hold zeros (round_init_k).
+//
+// The edge count stays on the device (cnt[C_NEDGE]): later launches cover the
+// bound c.edge_bound of two edges a face, which the edge buffers always hold.
+// The host reads it only where it may exceed the logical capacity, whose
+// growth restarts the stored costs (grow_edges): a round or two of a run.
 static int topology_and_quadrics(Ctx& c, Mesh m, int nP, int nT) {
-    // per-vertex ring counts and per-face edge counts in one pass
-    LAUNCHP(K_RING_COUNT, 12.0 * nT + 8.0 * nP + 4.0 * nT, topo_count_k, nT + 1, m, nT, c.ring_off, c.edge_off);
-    PAMO_TRY(scan_exclusive_lb(c.ring_off, c.ring_off, nP + 1, c.lb, c.stream));
-    LAUNCHP(K_RING_FILL, 12.0 * nT + 12.0 * nT + 32.0 * nT, ring_fill_k, nT, m, nT, c.ring_off, c.ring_fill,
-            c.ring_raw, c.ring_own);
+    // per-vertex ring counts, per-face edge counts and the order of the edges
+    // in one pass, the three scans in one launch, then everything placed
+    LAUNCHP(K_RING_COUNT, 12.0 * nT + 8.0 * nP + 28.0 * nT, topo_count_k, nT + 1, m, nT, c.ring_off, c.edge_off,
+            c.eord_cnt, c.frank, c.ferank);
+    PAMO_TRY(scan_set(c.ring_off, nP + 1, c.edge_off, nT + 1, c.eord_cnt, nP + 1, c.lb, c.stream));
+    PAMO_CHECK((size_t)2 * nT <= c.alloc_edges, "edge buffers smaller than two edges per face");
+    auto fill = [&]() -> int {
+        LAUNCHP(K_RING_FILL, 12.0 * nT + 12.0 * nT + 24.0 * nT + 24.0 * nT + 12.0 * 1.5 * nT, fill_topo_k, nT, m, nT,
+                (const int*)c.ring_off, (const int*)c.edge_off, (const int*)c.eord_cnt, (const int4*)c.frank,
+                (const int2*)c.ferank, c.ring_raw, c.ring_own, c.eu, c.ev, c.eord, c.dcnt);
+        return 0;
+    };
+    PAMO_TRY(fill());
     LAUNCHP(K_RING_SORT, 4.0 * nP + 24.0 * nT + 12.0 * nT + 60.0 * nT, ring_rank_k, 3LL * nT, m, c.ring_off,
             c.ring_raw, c.ring_own, 3 * nT, c.ring_off + nP, c.ring, c.rv);
-    // edges: at most two per face, which the edge buffers always hold, so the
-    // fill and the quadrics run before the host reads the count back (the
-    // read then waits on them instead of stalling the stream)
-    PAMO_TRY(scan_exclusive_lb(c.edge_off, c.edge_off, nT + 1, c.lb, c.stream));
-    PAMO_CHECK((size_t)2 * nT <= c.alloc_edges, "edge buffers smaller than two edges per face");
-    LAUNCHP(K_EDGE_FILL, 16.0 * nT + 12.0 * 1.5 * nT, edge_fill_k, nT, m, nT, c.edge_off, c.eu, c.ev, c.dcnt,
-            c.eord_cnt, c.erank);
     // quadrics
     const double quad_bytes = 4.0 * nP + 48.0 * nT + 16.0 * nP + 48.0 * nP;
     if (c.ring_lanes == 8)
@@ -540,20 +559,15 @@ static int topology_and_quadrics(Ctx& c, Mesh m, int nP, int nT) {
         LAUNCHP(K_QUADRIC, quad_bytes, quadric_group_k<4>, 4LL * nP, m, c.ring_off, c.rv, nP, c.Q);
     else
         LAUNCHP(K_QUADRIC, quad_bytes, quadric_k, nP, m, c.ring_off, c.rv, nP, c.Q);
-    PAMO_TRY(sync_counters(c));
-    const int nE = c.hcnt[C_NEDGE];
-    c.n_edges = nE;
-    bool realloc = false;
-    PAMO_TRY(grow_edges(c, (size_t)nE, &realloc));
-    if (realloc) {  // fresh edge buffers: fill and count them again
-        PAMO_HIP(hipMemsetAsync(c.eord_cnt, 0, sizeof(int) * (nP + 1), c.stream));
-        LAUNCHP(K_EDGE_FILL, 16.0 * nT + 12.0 * nE, edge_fill_k, nT, m, nT, c.edge_off, c.eu, c.ev, c.dcnt,
-                c.eord_cnt, c.erank);
+    c.edge_bound = 2 * nT;
+    if ((size_t)c.edge_bound > c.cap_edges) {
+        PAMO_TRY(sync_counters(c));
+        const int nE = c.hcnt[C_NEDGE];
+        c.edge_bound = nE;
+        bool realloc = false;
+        PAMO_TRY(grow_edges(c, (size_t)nE, &realloc));
+        if (realloc) PAMO_TRY(fill());  // fresh edge buffers
     }
-    // edge-cost launch order: edges grouped by smaller endpoint (counted by
-    // edge_fill_k)
-    PAMO_TRY(scan_exclusive_lb(c.eord_cnt, c.eord_cnt, nP + 1, c.lb, c.stream));
-    LAUNCH(edge_order_scatter_k, nE, c.eu, (const int*)c.erank, nE, (const int*)c.eord_cnt, c.eord);
     return 0;
 }
 
@@ -575,15 +589,16 @@ static int pasp_round_device(Ctx& c, int nP, int nT, float scale, float thr) {
     c.n_pts = nP;
     c.n_tris = nT;
     LAUNCH(round_init_k, std::max(nP + 1, nT), m, Mesh{nullptr, nullptr, nullptr, nullptr}, nP, nT, c.occ, c.ring_off,
-           c.ring_fill, c.eord_cnt, (unsigned long long*)c.vmin, (uint8_t*)nullptr);
+           c.eord_cnt, (unsigned long long*)c.vmin, (uint8_t*)nullptr);
     PAMO_TRY(topology_and_quadrics(c, m, nP, nT));
-    const int nE = c.n_edges;
+    const int nE = c.edge_bound;  // launches cover this bound
+    const int* cnt = c.dcnt;
     LAUNCHP(K_EDGE_COST, 12.0 * nE + 4.0 * nP + 48.0 * nT + 16.0 * nP + 48.0 * nP + 4.0 * nE, pasp_cost_k, nE, m,
-            c.ring_off, c.rv, c.eu, c.ev, c.eord, nE, c.Q, scale, thr, c.edge_cost);
-    LAUNCHP(K_PROPAGATE, 12.0 * nE + 16.0 * nP, propagate_k, nE, c.eu, c.ev, nE, c.edge_cost,
+            c.ring_off, c.rv, c.eu, c.ev, c.eord, cnt, c.Q, scale, thr, c.edge_cost);
+    LAUNCHP(K_PROPAGATE, 12.0 * nE + 16.0 * nP, propagate_k, nE, c.eu, c.ev, cnt, c.edge_cost,
             (unsigned long long*)c.vmin);
     LAUNCHP(K_SELECT_COLLAPSE, 16.0 * nE + 4.0 * nP + 48.0 * nT + 8.0 * nP, pasp_collapse_k, nE, m, c.occ,
-            c.ring_off, c.ring, (const int4*)c.rv, c.eu, c.ev, nE, c.edge_cost, (const unsigned long long*)c.vmin,
+            c.ring_off, c.ring, (const int4*)c.rv, c.eu, c.ev, cnt, c.edge_cost, (const unsigned long long*)c.vmin,
             collapse_t);
     PAMO_TRY(scan_exclusive_lb(c.occ, c.pts_map, nP + 1, c.lb, c.stream));
     return 0;
@@ -596,15 +611,16 @@ static int round_device(Ctx& c, int nP, int nT, float scale, float thr, bool is_
     c.n_pts = nP;
     c.n_tris = nT;
     // snapshot for undo, occupancy, ring counters, minimum keys, changed flags
-    LAUNCH(round_init_k, std::max(nP + 1, nT), m, Mesh{c.op, c.oi, c.oj, c.ok}, nP, nT, c.occ, c.ring_off, c.ring_fill,
+    LAUNCH(round_init_k, std::max(nP + 1, nT), m, Mesh{c.op, c.oi, c.oj, c.ok}, nP, nT, c.occ, c.ring_off,
            c.eord_cnt, (unsigned long long*)c.vmin, c.changed);
     PAMO_TRY(topology_and_quadrics(c, m, nP, nT));
-    const int nE = c.n_edges;
+    const int nE = c.edge_bound;  // launches cover this bound
+    const int* cnt = c.dcnt;
     CostParams cp{edge_s, tres, is_stuck ? 1 : 0, c.inv_epoch};
     // (+ 16 B per vertex: the minimum keys the fused propagation lowers)
     const double cost_bytes = 12.0 * nE + 4.0 * nP + 48.0 * nT + 16.0 * nP + 48.0 * nP + 1.0 * nP + 4.0 * nE + 16.0 * nP;
 #define PAMO_EDGE_COST(K, lanes)                                                                              \
-    LAUNCHP(K_EDGE_COST, cost_bytes, K, (long long)nE * (lanes), m, c.ring_off, c.rv, c.eu, c.ev, c.eord, nE,     \
+    LAUNCHP(K_EDGE_COST, cost_bytes, K, (long long)nE * (lanes), m, c.ring_off, c.rv, c.eu, c.ev, c.eord, cnt,    \
             c.invalid, c.Q, cp, c.edge_cost, (unsigned long long*)c.vmin)
     if (c.edge_lanes == 8) {
         if (c.placement) PAMO_EDGE_COST((edge_cost_group_k<true, 8>), 8);
@@ -621,8 +637,8 @@ static int round_device(Ctx& c, int nP, int nT, float scale, float thr, bool is_
     // per-vertex minimum keys)
     const double sel_bytes = 16.0 * nE + 4.0 * nP + 48.0 * nT + 8.0 * nP;
 #define PAMO_SELECT(K, lanes)                                                                                 \
-    LAUNCHP(K_SELECT_COLLAPSE, sel_bytes, K, (long long)(nE + 1) * (lanes), m, orig_mesh(c), c.occ, c.ring_off,   \
-            c.ring, (const int4*)c.rv, c.eu, c.ev, nE, c.edge_cost, (const unsigned long long*)c.vmin, collapse_t,  \
+    LAUNCHP(K_SELECT_COLLAPSE, sel_bytes, K, (long long)nE * (lanes), m, orig_mesh(c), c.occ, c.ring_off,         \
+            c.ring, (const int4*)c.rv, c.eu, c.ev, cnt, c.edge_cost, (const unsigned long long*)c.vmin, collapse_t,  \
             c.esel, (const float4*)c.Q, c.changed)
     if (c.ring_lanes == 8) {
         if (c.placement) PAMO_SELECT((select_collapse_group_k<true, 8>), 8);
@@ -635,12 +651,12 @@ static int round_device(Ctx& c, int nP, int nT, float scale, float thr, bool is_
         else PAMO_SELECT(select_collapse_k<false>, 1);
     }
 #undef PAMO_SELECT
-    PAMO_TRY(scan_op(CollapseListOp{c.esel, c.recs, c.dcnt}, nE, c.lb, c.stream));
-    // cleanup
-    PAMO_TRY(scan_op(CleanupOp{m, c.eu, c.ev, nE, nT, c.recs, c.dcnt}, (long long)std::max(nE, nT), c.lb, c.stream,
-                     K_LINE_FLAG, 8.0 * nE + 16.0 * nP + 4.0 * nE + 12.0 * nT));
+    // the records, and the cleanup with the line collapses, in one launch
+    PAMO_TRY(scan_pair(CollapseListOp{c.esel, c.recs, c.dcnt}, nE, CleanupOp{m, c.eu, c.ev, nT, c.lines, c.dcnt},
+                       (long long)std::max(nE, nT), c.lb, c.stream, K_LINE_FLAG,
+                       8.0 * nE + 16.0 * nP + 4.0 * nE + 12.0 * nT));
     hipLaunchKernelGGL(line_apply_k, dim3(1), dim3(1), 0, c.stream, m, c.occ, c.ring_off, c.ring, c.eu, c.ev,
-                       (const int*)c.recs, c.dcnt, c.changed);
+                       (const int*)c.lines, c.dcnt, c.changed);
     PAMO_HIP(hipGetLastError());
     // guard + undo loop (:1014-1040).  The guard is queued before the record
     // counts are read back, so the read waits on the guard's kernels instead
@@ -653,9 +669,9 @@ static int round_device(Ctx& c, int nP, int nT, float scale, float thr, bool is_
     // edge count and by half the points plus 512 (regular collapses share
     // no vertex)
     const long long cand_bound = std::min<long long>(nE, nP / 2 + 512);
-    PAMO_TRY(scan_op(UndoListOp{c.recs, c.ring_off, c.ring, c.eu, c.ev, c.flagged, c.pushed, c.dcnt}, cand_bound,
-                     c.lb, c.stream, K_UNDO_CAND, 16.0 * cand_bound + 1.0 * nT));
+    PAMO_TRY(undo_scan(c, cand_bound));
     PAMO_TRY(sync_counters(c));
+    c.n_edges = c.hcnt[C_NEDGE];
     c.n_regular = c.hcnt[C_NREG];
     c.n_rec = c.n_regular + c.hcnt[C_LINE];
     c.n_cand = std::min(c.n_rec, (c.n_regular + 511) / 512 * 512);
@@ -686,8 +702,9 @@ static int round_device(Ctx& c, int nP, int nT, float scale, float thr, bool is_
         c.n_vertices_undo += 2 * npushed;
         if (it == 5) break;
     }
-    // new vertex ids
-    PAMO_TRY(scan_exclusive_lb(c.occ, c.pts_map, nP + 1, c.lb, c.stream));
+    // the new vertex ids are those of the last undo_scan, in new_map: the
+    // caller makes them pts_map (entries past this round's points keep their
+    // older values, as in a map that is written in place)
     return 0;
 }
 
@@ -713,17 +730,19 @@ static int prologue(Ctx& c, const int* undo_in, int n_undo_in, bool is_stuck) {
 }
 
 // Drop removed vertices and faces and renumber (pamo/__init__.py:163-167):
-// stable compaction by pts_map and by a scan of live faces.
+// stable compaction by the point map (new_map after a round, which then
+// becomes pts_map; pts_map after a legacy round) and by a scan of live faces.
 // With carry, the next round refits the guard tree, renumbering its leaves to
 // the compacted faces (guard_leaves_k), unless fewer than tree_keep_pct % of
 // its leaves are still live.
-static int compact_round(Ctx& c, int nP, int nT, bool carry = false) {
+static int compact_round(Ctx& c, int nP, int nT, const int* map, bool carry = false) {
     Mesh m = cur_mesh(c);
-    PAMO_TRY(scan_op(CompactMeshOp{m, nP, nT, c.occ, c.pts_map, c.face_scan, c.np, c.ni, c.nj, c.nk, c.dcnt},
+    PAMO_TRY(scan_op(CompactMeshOp{m, nP, nT, c.occ, map, map == c.pts_map ? nullptr : c.pts_map, c.face_scan, c.np, c.ni, c.nj, c.nk, c.dcnt},
                      (long long)std::max(nP, nT) + 1, c.lb, c.stream, K_COMPACT_MESH,
                      4.0 * nP + 4.0 * nP + 16.0 * nP + 16.0 * nP + 12.0 * nT + 4.0 * nT + 12.0 * nT));
     carry = carry && c.tree_valid && c.tree_keep_pct < 100;
     PAMO_TRY(sync_counters(c));
+    c.n_edges = c.hcnt[C_NEDGE];
     c.tree_n = c.hcnt[C_NLIVE];
     if (carry) {
         // every live face holds one leaf
@@ -930,6 +949,7 @@ int pamo_round(pamo_ctx* ctx, const float* d_pts, int n_pts, const int* d_tris, 
     c.tree_n = 0;
     if (init) PAMO_TRY(pamo::shuffle_faces(c, n_tris));
     PAMO_TRY(pamo::round_device(c, n_pts, n_tris, scale, threshold, is_stuck != 0));
+    PAMO_HIP(hipMemcpyAsync(c.pts_map, c.new_map, sizeof(int) * ((size_t)n_pts + 1), hipMemcpyDeviceToDevice, c.stream));
     PAMO_CHECK(c.n_vertices_undo <= undo_cap, "pamo_round: undo_cap too small");
     pamo::Mesh m = pamo::cur_mesh(c);
     hipLaunchKernelGGL(pamo::store_points_k, dim3(pamo::grid_for(n_pts, pamo::kBlock)), dim3(pamo::kBlock), 0,
@@ -1033,7 +1053,19 @@ int pamo_round_debug(pamo_ctx* ctx, int what, void* d_out, long long cap, long l
             return 0;
         }
         case PAMO_DBG_EDGE_COST: n = c.n_edges; src = c.edge_cost; break;
-        case PAMO_DBG_RECORDS: n = c.n_rec; src = c.recs; break;
+        case PAMO_DBG_RECORDS: {  // the regular records, then the line collapses
+            n = c.n_rec;
+            PAMO_CHECK(n <= cap, "pamo_round_debug: cap too small");
+            const int nl = c.n_rec - c.n_regular;
+            if (c.n_regular > 0)
+                PAMO_HIP(hipMemcpyAsync(d_out, c.recs, 4 * (size_t)c.n_regular, hipMemcpyDeviceToDevice, c.stream));
+            if (nl > 0)
+                PAMO_HIP(hipMemcpyAsync((int*)d_out + c.n_regular, c.lines, 4 * (size_t)nl, hipMemcpyDeviceToDevice,
+                                        c.stream));
+            PAMO_HIP(hipStreamSynchronize(c.stream));
+            if (n_out) *n_out = n;
+            return 0;
+        }
         case PAMO_DBG_RING_OFF: n = c.n_pts + 1; src = c.ring_off; break;
         case PAMO_DBG_RING: {
             int tot = 0;
@@ -1153,7 +1185,7 @@ static int simplify_loop(Ctx& c, const float* d_verts, int n_verts, const int* d
         ++rounds;
         n_undo = c.n_vertices_undo;
         std::swap(c.undo_prev, c.undo_list);  // this round's list feeds the next prologue
-        PAMO_TRY(pamo::compact_round(c, nV, nF, true));
+        PAMO_TRY(pamo::compact_round(c, nV, nF, c.new_map, true));
         nV = c.hcnt[pamo::C_NV];
         nF = c.hcnt[pamo::C_NF];
         if (face_hist && rounds <= hist_cap) face_hist[rounds - 1] = nF;
@@ -1223,7 +1255,8 @@ int pamo_pasp_round(pamo_ctx* ctx, const float* d_pts, int n_pts, const int* d_t
     PAMO_HIP(hipGetLastError());
     PAMO_HIP(hipMemcpyAsync(d_out_occ, c.occ, sizeof(int) * n_pts, hipMemcpyDeviceToDevice, c.stream));
     PAMO_HIP(hipMemcpyAsync(d_out_map, c.pts_map, sizeof(int) * n_pts, hipMemcpyDeviceToDevice, c.stream));
-    PAMO_HIP(hipStreamSynchronize(c.stream));
+    PAMO_TRY(pamo::sync_counters(c));
+    c.n_edges = c.hcnt[pamo::C_NEDGE];
     return 0;
 }
 
@@ -1250,7 +1283,7 @@ int pamo_pasp_run(pamo_ctx* ctx, const float* d_verts, int n_verts, const int* d
         if (rounds == 0) PAMO_TRY(pamo::shuffle_faces(c, nF));
         PAMO_TRY(pamo::pasp_round_device(c, nV, nF, scale, threshold));
         ++rounds;
-        PAMO_TRY(pamo::compact_round(c, nV, nF));
+        PAMO_TRY(pamo::compact_round(c, nV, nF, c.pts_map));
         nV = c.hcnt[pamo::C_NV];
         nF = c.hcnt[pamo::C_NF];
         if (nF == prev) break;

@@ -164,21 +164,82 @@ __global__ void invalid_set_k(const int* __restrict__ undo_in, int n, uint32_t* 
 
 // ---------------------------------------------------------------- rings and edges (A4, A5)
 
-__global__ void ring_fill_k(Mesh m, int nT, const int* __restrict__ off, int* __restrict__ fill,
-                            int* __restrict__ raw, int* __restrict__ owner) {
+// One pass over the faces that counts, with the places that the counts leave:
+// each live face adds 1 to its three vertices' ring counters and keeps the old
+// values (rank.x, y, z: its slots among the vertex's), stores its emitted-edge
+// count, and for each emitted edge adds 1 to the smaller endpoint's counter
+// (erank: the edge's place in the edge-cost launch order).  fill_topo_k then
+// places everything without atomics of its own.  Bound by the atomics' round
+// trips over shuffled faces.  A run from 2M to 20k faces (573 rounds) spends
+// 19 + 12 ms in the two and 5 ms in the one launch that scans all three
+// arrays; counting without the places, two filling kernels with atomics, the
+// scatter of the order and three scans took 52 ms.
+__device__ __forceinline__ void count_topo(int f, int a, int b, int c, int* __restrict__ ring_cnt,
+                                           int* __restrict__ edge_cnt, int* __restrict__ order_cnt,
+                                           int4* __restrict__ rank, int2* __restrict__ erank) {
+    int4 r;
+    r.x = atomicAdd(&ring_cnt[a], 1);
+    r.y = atomicAdd(&ring_cnt[b], 1);
+    r.z = atomicAdd(&ring_cnt[c], 1);
+    r.w = 0;
+    // at most two of the three directed edges run from the larger end
+    int e0 = 0, e1 = 0, n = 0;
+    if (a > b) { e0 = atomicAdd(&order_cnt[b], 1); ++n; }
+    if (b > c) { const int q = atomicAdd(&order_cnt[c], 1); if (n++) e1 = q; else e0 = q; }
+    if (c > a) { const int q = atomicAdd(&order_cnt[a], 1); if (n++) e1 = q; else e0 = q; }
+    rank[f] = r;
+    erank[f] = make_int2(e0, e1);
+    edge_cnt[f] = n;
+}
+
+__global__ void topo_count_k(Mesh m, int nT, int* __restrict__ ring_cnt, int* __restrict__ edge_cnt,
+                             int* __restrict__ order_cnt, int4* __restrict__ rank, int2* __restrict__ erank) {
     int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= nT) return;
+    if (f > nT) return;
+    if (f == nT) {
+        edge_cnt[nT] = 0;
+        return;
+    }
     int a = m.i[f], b = m.j[f], c = m.k[f];
+    if (face_dead(a, b, c)) {
+        edge_cnt[f] = 0;
+        return;
+    }
+    count_topo(f, a, b, c, ring_cnt, edge_cnt, order_cnt, rank, erank);
+}
+
+// From the scanned counts: the ring slots (unordered; ring_rank_k sorts them),
+// the edge list, the edges grouped by smaller endpoint (order), and the edge
+// count in cnt[C_NEDGE].
+//
+// The order of the edge-cost lanes: edge ids follow the shuffled face order
+// while vertex ids are spatially coherent, so grouped by smaller endpoint the
+// lanes of a wave read neighbouring rings, positions and quadrics.  The order
+// inside a group depends on atomic timing; it changes only which lane
+// computes an edge, never a result.
+__global__ void fill_topo_k(Mesh m, int nT, const int* __restrict__ off, const int* __restrict__ edge_off,
+                            const int* __restrict__ order_off, const int4* __restrict__ rank,
+                            const int2* __restrict__ erank, int* __restrict__ raw, int* __restrict__ owner,
+                            int* __restrict__ eu, int* __restrict__ ev, int* __restrict__ order,
+                            int* __restrict__ cnt) {
+    int f = blockIdx.x * blockDim.x + threadIdx.x;
+    if (f == 0) cnt[C_NEDGE] = edge_off[nT];
+    if (f >= nT) return;
+    const int a = m.i[f], b = m.j[f], c = m.k[f];
     if (face_dead(a, b, c)) return;
-    int q = off[a] + atomicAdd(&fill[a], 1);
-    raw[q] = f;
-    owner[q] = a;
-    q = off[b] + atomicAdd(&fill[b], 1);
-    raw[q] = f;
-    owner[q] = b;
-    q = off[c] + atomicAdd(&fill[c], 1);
-    raw[q] = f;
-    owner[q] = c;
+    const int4 r = rank[f];
+    const int qa = off[a] + r.x, qb = off[b] + r.y, qc = off[c] + r.z;
+    raw[qa] = f;
+    owner[qa] = a;
+    raw[qb] = f;
+    owner[qb] = b;
+    raw[qc] = f;
+    owner[qc] = c;
+    const int2 er = erank[f];
+    int q = edge_off[f], n = 0;
+    if (a > b) { eu[q] = b; ev[q] = a; order[order_off[b] + er.x] = q; ++q; ++n; }
+    if (b > c) { eu[q] = c; ev[q] = b; order[order_off[c] + (n ? er.y : er.x)] = q; ++q; ++n; }
+    if (c > a) { eu[q] = a; ev[q] = c; order[order_off[a] + (n ? er.y : er.x)] = q; }
 }
 
 // Canonical ring order (ascending face index) with the packed int4 entries,
@@ -200,44 +261,6 @@ __global__ void __launch_bounds__(kBlock) ring_rank_k(Mesh m, const int* __restr
     }
     ring[b + r] = x;
     rv[b + r] = make_int4(m.i[x], m.j[x], m.k[x], x);
-}
-
-// Per-face counts in one pass: each live face adds 1 to its three vertices'
-// ring counters (ring_count_k) and stores its emitted-edge count (edge_count_k).
-__global__ void topo_count_k(Mesh m, int nT, int* __restrict__ ring_cnt, int* __restrict__ edge_cnt) {
-    int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f > nT) return;
-    if (f == nT) {
-        edge_cnt[nT] = 0;
-        return;
-    }
-    int a = m.i[f], b = m.j[f], c = m.k[f];
-    if (face_dead(a, b, c)) {
-        edge_cnt[f] = 0;
-        return;
-    }
-    atomicAdd(&ring_cnt[a], 1);
-    atomicAdd(&ring_cnt[b], 1);
-    atomicAdd(&ring_cnt[c], 1);
-    edge_cnt[f] = (int)(a > b) + (int)(b > c) + (int)(c > a);
-}
-
-// Also stores the edge count off[nT] to cnt[C_NEDGE].
-// Also counts the edges per smaller endpoint into order_cnt (zeroed by
-// round_init_k), the histogram of the edge-cost launch order.
-// also counts the edges per smaller endpoint (order_cnt) and keeps each
-// edge's rank among them (rank), for the edge-cost launch order
-__global__ void edge_fill_k(Mesh m, int nT, const int* __restrict__ off, int* __restrict__ eu, int* __restrict__ ev,
-                            int* __restrict__ cnt, int* __restrict__ order_cnt, int* __restrict__ rank) {
-    int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f == 0) cnt[C_NEDGE] = off[nT];
-    if (f >= nT) return;
-    int a = m.i[f], b = m.j[f], c = m.k[f];
-    if (face_dead(a, b, c)) return;
-    int q = off[f];
-    if (a > b) { eu[q] = b; ev[q] = a; rank[q] = atomicAdd(&order_cnt[b], 1); ++q; }
-    if (b > c) { eu[q] = c; ev[q] = b; rank[q] = atomicAdd(&order_cnt[c], 1); ++q; }
-    if (c > a) { eu[q] = a; ev[q] = c; rank[q] = atomicAdd(&order_cnt[a], 1); ++q; }
 }
 
 // ---------------------------------------------------------------- quadrics and costs (A6, A7)
@@ -429,19 +452,6 @@ __device__ __forceinline__ void edge_quadric(const float4* __restrict__ Q, int u
     M[8] = uc.x + vc.x; M[9] = uc.y + vc.y;
 }
 
-// Launch order of the edge-cost lanes: edge ids grouped by their smaller
-// endpoint (counting sort: histogram with ranks, exclusive scan, scatter).  Vertex ids of
-// a mesh are spatially coherent while edge ids follow the shuffled face
-// order, so in this order the lanes of a wave read neighbouring rings,
-// positions and quadrics.  The order inside one group (the ranks edge_fill_k
-// took) depends on atomic timing; it changes only which lane computes an
-// edge, never a result.
-__global__ void edge_order_scatter_k(const int* __restrict__ eu, const int* __restrict__ rank, int nE,
-                                     const int* __restrict__ start, int* __restrict__ order) {
-    int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e < nE) order[start[eu[e]] + rank[e]] = e;
-}
-
 __device__ __forceinline__ uint64_t edge_key(uint32_t c, int e) { return ((uint64_t)c << 32) | (uint32_t)e; }
 
 // propagate_edge_cost_kernel (:587-610) fused into the cost kernels: the
@@ -462,12 +472,12 @@ template <bool kOptimal>
 __global__ void __launch_bounds__(kBlock) edge_cost_k(Mesh m, const int* __restrict__ off,
                                                       const int4* __restrict__ rv, const int* __restrict__ eu,
                                                       const int* __restrict__ ev, const int* __restrict__ order,
-                                                      int nE, const uint32_t* __restrict__ invalid,
+                                                      const int* __restrict__ cnt, const uint32_t* __restrict__ invalid,
                                                       const float4* __restrict__ Q, CostParams cp,
                                                       uint32_t* __restrict__ cost,
                                                       unsigned long long* __restrict__ vmin) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nE) return;
+    if (t >= cnt[C_NEDGE]) return;  // the launch covers a bound
     const int e = order[t];
     const int u = eu[e], v = ev[e];
     if (invalid[u] == cp.inv_epoch && invalid[v] == cp.inv_epoch) {
@@ -580,7 +590,8 @@ template <bool kOptimal, int kG>
 __global__ void __launch_bounds__(kBlock) edge_cost_group_k(Mesh m, const int* __restrict__ off,
                                                             const int4* __restrict__ rv, const int* __restrict__ eu,
                                                             const int* __restrict__ ev, const int* __restrict__ order,
-                                                            int nE, const uint32_t* __restrict__ invalid,
+                                                            const int* __restrict__ cnt,
+                                                            const uint32_t* __restrict__ invalid,
                                                             const float4* __restrict__ Q, CostParams cp,
                                                             uint32_t* __restrict__ cost,
                                                             unsigned long long* __restrict__ vmin) {
@@ -588,7 +599,7 @@ __global__ void __launch_bounds__(kBlock) edge_cost_group_k(Mesh m, const int* _
     const long long gt = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const int g = (int)(threadIdx.x & (kG - 1));
     const long long t = gt / kG;
-    if (t >= nE) return;  // the whole group
+    if (t >= cnt[C_NEDGE]) return;  // the whole group (the launch covers a bound)
     const int e = order[t];
     const int u = eu[e], v = ev[e];
     if (invalid[u] == cp.inv_epoch && invalid[v] == cp.inv_epoch) {
@@ -699,11 +710,11 @@ __global__ void __launch_bounds__(kBlock) edge_cost_group_k(Mesh m, const int* _
 // exactly when x is one of its vertices, so tri_min[t] = min over t's three
 // vertices of vmin[x], vmin[x] = min key over edges incident to x: two
 // atomics per edge instead of one per ring face.
-__global__ void __launch_bounds__(kBlock) propagate_k(const int* __restrict__ eu, const int* __restrict__ ev, int nE,
+__global__ void __launch_bounds__(kBlock) propagate_k(const int* __restrict__ eu, const int* __restrict__ ev, const int* __restrict__ cnt,
                                                       const uint32_t* __restrict__ cost,
                                                       unsigned long long* __restrict__ vmin) {
     int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= nE) return;
+    if (e >= cnt[C_NEDGE]) return;
     const unsigned long long k = edge_key(cost[e], e);
     atomicMin(&vmin[eu[e]], k);
     atomicMin(&vmin[ev[e]], k);
@@ -769,17 +780,14 @@ template <bool kOptimal>
 __global__ void __launch_bounds__(kBlock) select_collapse_k(Mesh m, Orig o, int* occ, const int* __restrict__ off,
                                                             const int* __restrict__ ring, const int4* __restrict__ rv,
                                                             const int* __restrict__ eu, const int* __restrict__ ev,
-                                                            int nE, const uint32_t* __restrict__ cost,
+                                                            const int* __restrict__ cnt,
+                                                            const uint32_t* __restrict__ cost,
                                                             const unsigned long long* __restrict__ vmin,
                                                             uint32_t collapse_t, int* __restrict__ sel,
                                                             const float4* __restrict__ Q,
                                                             uint8_t* __restrict__ changed) {
     int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e > nE) return;
-    if (e == nE) {
-        sel[nE] = 0;
-        return;
-    }
+    if (e >= cnt[C_NEDGE]) return;  // the launch covers a bound
     const uint32_t c = cost[e];
     int s = 0;
     if (c <= collapse_t) {
@@ -843,7 +851,8 @@ __global__ void __launch_bounds__(kBlock) select_collapse_group_k(Mesh m, Orig o
                                                                   const int* __restrict__ ring,
                                                                   const int4* __restrict__ rv,
                                                                   const int* __restrict__ eu,
-                                                                  const int* __restrict__ ev, int nE,
+                                                                  const int* __restrict__ ev,
+                                                                  const int* __restrict__ cnt,
                                                                   const uint32_t* __restrict__ cost,
                                                                   const unsigned long long* __restrict__ vmin,
                                                                   uint32_t collapse_t, int* __restrict__ sel,
@@ -852,12 +861,8 @@ __global__ void __launch_bounds__(kBlock) select_collapse_group_k(Mesh m, Orig o
     const long long gt = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const int g = (int)(threadIdx.x & (kG - 1));
     const long long ee = gt / kG;
-    if (ee > nE) return;  // the whole group
+    if (ee >= cnt[C_NEDGE]) return;  // the whole group (the launch covers a bound)
     const int e = (int)ee;
-    if (e == nE) {
-        if (g == 0) sel[nE] = 0;
-        return;
-    }
     const uint32_t c = cost[e];
     if (c > collapse_t) {
         if (g == 0) sel[e] = 0;
@@ -944,11 +949,11 @@ __global__ void __launch_bounds__(kBlock) select_collapse_group_k(Mesh m, Orig o
 // / s * t`, cusimp.cu:378).  No invalid-vertex or stuck rules.
 __global__ void __launch_bounds__(kBlock) pasp_cost_k(Mesh m, const int* __restrict__ off, const int4* __restrict__ rv,
                                                       const int* __restrict__ eu, const int* __restrict__ ev,
-                                                      const int* __restrict__ order, int nE,
+                                                      const int* __restrict__ order, const int* __restrict__ cnt,
                                                       const float4* __restrict__ Q, float edge_s, float tres,
                                                       uint32_t* __restrict__ cost) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nE) return;
+    if (t >= cnt[C_NEDGE]) return;
     const int e = order[t];
     const int u = eu[e], v = ev[e];
     const int ub = off[u], ue = off[u + 1], vb = off[v], ve = off[v + 1];
@@ -1015,11 +1020,11 @@ __global__ void __launch_bounds__(kBlock) pasp_cost_k(Mesh m, const int* __restr
 __global__ void __launch_bounds__(kBlock) pasp_collapse_k(Mesh m, int* occ, const int* __restrict__ off,
                                                           const int* __restrict__ ring, const int4* __restrict__ rv,
                                                           const int* __restrict__ eu, const int* __restrict__ ev,
-                                                          int nE, const uint32_t* __restrict__ cost,
+                                                          const int* __restrict__ cnt, const uint32_t* __restrict__ cost,
                                                           const unsigned long long* __restrict__ vmin,
                                                           uint32_t collapse_t) {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= nE) return;
+    if (e >= cnt[C_NEDGE]) return;
     const uint32_t c = cost[e];
     if (c > collapse_t) return;
     const unsigned long long key = edge_key(c, e);
@@ -1047,13 +1052,12 @@ __global__ void __launch_bounds__(kBlock) pasp_collapse_k(Mesh m, int* occ, cons
 // the result deterministic where the reference races on shared faces.  The
 // lane walks the list CleanupOp built, not the whole edge array.
 __global__ void line_apply_k(Mesh m, int* occ, const int* __restrict__ off, const int* __restrict__ ring,
-                             const int* __restrict__ eu, const int* __restrict__ ev, const int* __restrict__ recs,
+                             const int* __restrict__ eu, const int* __restrict__ ev, const int* __restrict__ lines,
                              const int* cnt, uint8_t* __restrict__ changed) {
     if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    const int base = cnt[C_NREG];
     const int nl = cnt[C_LINE];
     for (int w = 0; w < nl; ++w) {
-        const int e = recs[base + w];
+        const int e = lines[w];
         const int u = eu[e], v = ev[e];
         // the record's one-ring faces are the guard's queries (the regular
         // records' are marked by the selection kernel)
@@ -1188,8 +1192,8 @@ __global__ void __launch_bounds__(kBlock) whole_box_k(float* __restrict__ part, 
 // (when snap.p is set), occupancy 1 (0 at nP), zeroed ring counters and
 // changed flags (when given), per-vertex minimum keys at the maximum.
 __global__ void round_init_k(Mesh m, Mesh snap, int nP, int nT, int* __restrict__ occ, int* __restrict__ ring_off,
-                             int* __restrict__ ring_fill, int* __restrict__ order_cnt,
-                             unsigned long long* __restrict__ vmin, uint8_t* __restrict__ changed) {
+                             int* __restrict__ order_cnt, unsigned long long* __restrict__ vmin,
+                             uint8_t* __restrict__ changed) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < nP) {
         if (snap.p) snap.p[i] = m.p[i];
@@ -1199,7 +1203,6 @@ __global__ void round_init_k(Mesh m, Mesh snap, int nP, int nT, int* __restrict_
     if (i == nP) occ[nP] = 0;
     if (i <= nP) {
         ring_off[i] = 0;
-        ring_fill[i] = 0;
         order_cnt[i] = 0;
     }
     if (i < nT) {
@@ -1782,7 +1785,9 @@ __device__ __forceinline__ void guard_walk_subtree(Mesh m, const uint8_t* __rest
 // evaluates 64 pairs at a time.  The critical path is then the wave's total
 // node count / 64 plus the tree depth, instead of the longest single walk.
 // (With node records and the children pushed untested, half of the pops found
-// no overlap: 60 us a launch on the 2M-face headline, GUARD_NOW now.)
+// no overlap; a launch still takes 60-64 us on average over a run from 2M to
+// 20k faces either way, and 37 us where it took 34-36 on 200k: what is gained
+// is the node records, which the box kernels no longer write.)
 // When the frontier is full, a lane walks the rest of its subtree by itself
 // (exact, only slower).  The flags are idempotent, so the visiting order does
 // not change the result.
@@ -2180,7 +2185,7 @@ struct CollapseListOp {
     const int* flag;
     int* recs;
     int* cnt;
-    __device__ int count(long long e) const { return flag[e]; }
+    __device__ int count(long long e) const { return e < cnt[C_NEDGE] ? flag[e] : 0; }
     __device__ void emit(long long e, int v, int pos) const {
         if (v) recs[pos] = (int)e;
     }
@@ -2188,16 +2193,16 @@ struct CollapseListOp {
 };
 
 // Cleanup (cusimp_free.cu:218-274): item t removes face t if two of its
-// corners coincide (t < nT) and flags edge t if its ends coincide (t < nE);
-// the line collapses go, in edge order, after the regular collapses in the
-// records.  Items cover max(nE, nT); the two parts touch disjoint data.
+// corners coincide (t < nT) and flags edge t if its ends coincide; the line
+// collapses are listed in edge order (lines).  Items cover the larger of the
+// faces and the bound of the edges; the two parts touch disjoint data.
 struct CleanupOp {
     static constexpr int kIpt = 2;
     Mesh m;
     const int* eu;
     const int* ev;
-    int nE, nT;
-    int* recs;
+    int nT;
+    int* lines;
     int* cnt;
     __device__ int count(long long t) const {
         if (t < nT) {
@@ -2208,12 +2213,12 @@ struct CleanupOp {
                 m.k[t] = -1;
             }
         }
-        if (t >= nE) return 0;
+        if (t >= cnt[C_NEDGE]) return 0;
         const F3 p = ld(m, eu[t]), q = ld(m, ev[t]);
         return (p.x == q.x && p.y == q.y && p.z == q.z) ? 1 : 0;
     }
     __device__ void emit(long long e, int v, int pos) const {
-        if (v) recs[cnt[C_NREG] + pos] = (int)e;
+        if (v) lines[pos] = (int)e;
     }
     __device__ void done(int total) const { cnt[C_LINE] = total; }
 };
@@ -2225,7 +2230,8 @@ struct CleanupOp {
 // vertex rings.
 struct UndoListOp {
     static constexpr int kIpt = 1;
-    const int* recs;
+    const int* recs;   // the regular records, then
+    const int* lines;  // the line collapses
     const int* off;
     const int* ring;
     const int* eu;
@@ -2238,7 +2244,7 @@ struct UndoListOp {
         // records (the reference's grid); the launch covers a bound
         const int nreg = cnt[C_NREG], nrec = nreg + cnt[C_LINE];
         if (r >= min(nrec, (nreg + 511) / 512 * 512)) return 0;
-        const int e = recs[r];
+        const int e = r < nreg ? recs[r] : lines[r - nreg];
         const int u = eu[e], v = ev[e];
         // four ring entries, then their four flags, per step
         for (int side = 0; side < 2; ++side) {
@@ -2255,22 +2261,24 @@ struct UndoListOp {
         return 0;
     }
     __device__ void emit(long long r, int v, int pos) const {
-        if (v) pushed[pos] = recs[r];
+        if (v) pushed[pos] = r < cnt[C_NREG] ? recs[r] : lines[r - cnt[C_NREG]];
     }
     __device__ void done(int total) const { cnt[C_PUSHED] = total; }
 };
 
 // Compaction of the mesh (pamo/__init__.py:163-167): item t moves point t
-// to pts_map[t] if it is occupied, and face t to its position among the
+// to map[t] if it is occupied, and face t to its position among the
 // live faces with renumbered corners; fpos[t] receives that position for
-// t <= nT (fpos[nT] = live faces), which the guard tree's carry reads.  Items
-// cover max(nP, nT) + 1.
+// t <= nT (fpos[nT] = live faces), which the guard tree's carry reads; keep[t]
+// receives map[t] unless keep is null (the map that the next round's undo
+// reads).  Items cover max(nP, nT) + 1.
 struct CompactMeshOp {
     static constexpr int kIpt = 2;
     Mesh m;
     int nP, nT;
     const int* occ;
-    const int* pts_map;
+    const int* map;
+    int* keep;
     int* fpos;
     float4* np;
     int* ni;
@@ -2279,13 +2287,17 @@ struct CompactMeshOp {
     int* cnt;
     __device__ int count(long long t) const { return (t < nT && m.i[t] >= 0) ? 1 : 0; }
     __device__ void emit(long long t, int v, int pos) const {
-        if (t < nP && occ[t]) np[pts_map[t]] = m.p[t];
-        if (t == nP) cnt[C_NV] = pts_map[nP];
+        if (t <= nP) {
+            const int to = map[t];
+            if (keep) keep[t] = to;
+            if (t == nP) cnt[C_NV] = to;
+            else if (occ[t]) np[to] = m.p[t];
+        }
         if (t <= nT) fpos[t] = pos;
         if (v) {
-            ni[pos] = pts_map[m.i[t]];
-            nj[pos] = pts_map[m.j[t]];
-            nk[pos] = pts_map[m.k[t]];
+            ni[pos] = map[m.i[t]];
+            nj[pos] = map[m.j[t]];
+            nk[pos] = map[m.k[t]];
         }
     }
     __device__ void done(int total) const { cnt[C_NF] = total; }
