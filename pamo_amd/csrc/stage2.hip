@@ -418,8 +418,11 @@ static int sync_counters(Ctx& c) {
 // over the same hierarchy (refit): the undo moves vertices and restores
 // faces, and every face it can restore is already a leaf, with an empty box
 // while it is removed.  Which pairs overlap does not depend on the tree's
-// shape, so the flags are those of a tree built afresh.
-static int run_guard(Ctx& c, int nT, bool refit) {
+// shape, so the flags are those of a tree built afresh.  again: the number of
+// the undo that this guard follows (0: the round's first guard), which then
+// asks only for the faces whose answer the undo can have changed
+// (guard_leaves_k).
+static int run_guard(Ctx& c, int nT, bool refit, int again = 0) {
     Mesh m = cur_mesh(c);
     const double nP = c.n_pts;
     if (!refit) {
@@ -445,7 +448,7 @@ static int run_guard(Ctx& c, int nT, bool refit) {
     PAMO_TRY(lookback_begin(c.lb, nb0, c.stream));
     prof_begin(K_BVH_BOXES, 4.0 * nT + 12.0 * nT + 16.0 * nP + 32.0 * nT + 64.0 * nT, c.stream);
     hipLaunchKernelGGL(guard_leaves_k, dim3(nb0), dim3(kBlock), 0, c.stream, m, nT, c.bval, c.tree_carry ? 1 : 0,
-                       (const int*)c.face_scan, c.carry_old, (const uint8_t*)c.changed, c.flagged, c.dcnt, c.bbox,
+                       (const int*)c.face_scan, c.carry_old, again, (const unsigned long long*)c.vmin, c.changed, c.flagged, c.dcnt, c.bbox,
                        (const int*)c.bslot, (const int2*)c.brange, c.bpre, c.bsuf, c.blk, c.qlist, c.lb.state,
                        c.lb.ticket, c.lb.err, c.lb.epoch, c.lb.base);
     lookback_end(c.lb, nb0);
@@ -689,15 +692,15 @@ static int round_device(Ctx& c, int nP, int nT, float scale, float thr, bool is_
         ++c.undo_iters;
         if (c.ring_lanes == 8)
             LAUNCH(undo_apply_group_k<8>, 8LL * npushed, m, orig_mesh(c), c.occ, c.ring_off, c.ring, c.eu, c.ev,
-                   c.pushed, npushed, (const int*)c.pts_map, c.undo_list, first);
+                   c.pushed, npushed, (const int*)c.pts_map, c.undo_list, first, (unsigned long long*)c.vmin, it);
         else if (c.ring_lanes == 4)
             LAUNCH(undo_apply_group_k<4>, 4LL * npushed, m, orig_mesh(c), c.occ, c.ring_off, c.ring, c.eu, c.ev,
-                   c.pushed, npushed, (const int*)c.pts_map, c.undo_list, first);
+                   c.pushed, npushed, (const int*)c.pts_map, c.undo_list, first, (unsigned long long*)c.vmin, it);
         else
             LAUNCH(undo_apply_k, npushed, m, orig_mesh(c), c.occ, c.ring_off, c.ring, c.eu, c.ev, c.pushed, npushed,
-                   (const int*)c.pts_map, c.undo_list, first);
+                   (const int*)c.pts_map, c.undo_list, first, (unsigned long long*)c.vmin, it);
         first += 2 * npushed;
-        PAMO_TRY(run_guard(c, nT, true));
+        PAMO_TRY(run_guard(c, nT, true, it));
         PAMO_TRY(undo_candidates(c, npushed));
         c.n_vertices_undo += 2 * npushed;
         if (it == 5) break;
