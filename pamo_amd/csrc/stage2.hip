@@ -410,6 +410,48 @@ static int sync_counters(Ctx& c) {
     return 0;
 }
 
+// The queries of guard_leaves_k's list over the current tree.
+static int guard_queries(Ctx& c, int nT) {
+    Mesh m = cur_mesh(c);
+    const double nP = c.n_pts;
+    // meshes up to 256k faces split every query group over 8 subtrees: late
+    // rounds hold few queries, and one query with a large box would otherwise
+    // hold a whole launch in one wave
+    const int part_log = nT <= c.guard_split_faces ? c.guard_split_log : 0;
+    const long long guard_threads = ((((long long)nT + kGuardQ - 1) / kGuardQ) << part_log) * kWave;
+    const double guard_bytes = 4.0 * nT + 12.0 * nT + 16.0 * nP + 64.0 * nT + 1.0 * nT + 1.0 * nT;
+    Undecided u{nullptr, c.dcnt + C_UNDECIDED, 0, c.exact_guard == 2 ? 1 : 0};
+    if (c.exact_guard) {
+        // list capacity: the pairs that filtered signs leave open are those
+        // whose planes both cross the other face, or touch it (a few per
+        // changed face at most; read_candidates grows it for more); the test
+        // setting lists every candidate pair
+        const size_t cap = c.exact_guard == 2 ? 48 * (size_t)c.alloc_tris : std::max<size_t>(1 << 16, 2 * c.alloc_tris);
+        if (cap > c.alloc_ulist) {
+            PAMO_TRY(dalloc(&c.ulist, cap, c.stream));
+            c.alloc_ulist = cap;
+        }
+        u.list = c.ulist;
+        u.cap = (int)std::min<size_t>(c.alloc_ulist, 0x7fffffff);
+        PAMO_HIP(hipMemsetAsync(c.dcnt + C_UNDECIDED, 0, sizeof(int), c.stream));
+        LAUNCHP(K_GUARD_QUERY, guard_bytes, (guard_query_k<kGuardStack, true>), guard_threads, m, c.qlist, c.dcnt,
+                c.changed, (const float4*)c.bbox, (const int*)c.bslot, 1e-3f, c.flagged, u, part_log, c.dcnt + C_WALK_ERR, c.walk_cap);
+        hipLaunchKernelGGL(exact_pairs_k, dim3(2048), dim3(kWave), 0, c.stream, m, (const int2*)c.ulist,
+                           (const int*)(c.dcnt + C_UNDECIDED), u.cap, c.flagged);
+        PAMO_HIP(hipGetLastError());
+    } else if (c.guard_small_stack) {
+        LAUNCHP(K_GUARD_QUERY, guard_bytes, (guard_query_k<kGuardStackSmall, false>), guard_threads, m, c.qlist,
+                c.dcnt, c.changed, (const float4*)c.bbox, (const int*)c.bslot, 1e-3f, c.flagged, u, part_log, c.dcnt + C_WALK_ERR, c.walk_cap);
+    } else if (c.guard_waves == 4) {
+        LAUNCHP(K_GUARD_QUERY, guard_bytes, guard_query_w4_k, guard_threads, m, c.qlist, c.dcnt, c.changed,
+                (const float4*)c.bbox, (const int*)c.bslot, 1e-3f, c.flagged, u, part_log, c.dcnt + C_WALK_ERR, c.walk_cap);
+    } else {
+        LAUNCHP(K_GUARD_QUERY, guard_bytes, (guard_query_k<kGuardStack, false>), guard_threads, m, c.qlist, c.dcnt,
+                c.changed, (const float4*)c.bbox, (const int*)c.bslot, 1e-3f, c.flagged, u, part_log, c.dcnt + C_WALK_ERR, c.walk_cap);
+    }
+    return 0;
+}
+
 // Flag the faces of intersecting pairs that involve a changed face
 // (self_intersect.cuh:151-392, restricted to the faces that can change an
 // undo decision), over an LBVH of the faces live at the start of the round.
@@ -468,40 +510,7 @@ static int run_guard(Ctx& c, int nT, bool refit, int again = 0) {
     }
     prof_end(K_BVH_BOXES, c.stream);
     PAMO_HIP(hipGetLastError());
-    // meshes up to 256k faces split every query group over 8 subtrees: late
-    // rounds hold few queries, and one query with a large box would otherwise
-    // hold a whole launch in one wave
-    const int part_log = nT <= c.guard_split_faces ? c.guard_split_log : 0;
-    const long long guard_threads = ((((long long)nT + kGuardQ - 1) / kGuardQ) << part_log) * kWave;
-    const double guard_bytes = 4.0 * nT + 12.0 * nT + 16.0 * nP + 64.0 * nT + 1.0 * nT + 1.0 * nT;
-    Undecided u{nullptr, c.dcnt + C_UNDECIDED, 0, c.exact_guard == 2 ? 1 : 0};
-    if (c.exact_guard) {
-        // list capacity: undecided pairs are near-degenerate ones (a few per
-        // changed face at most); the test setting lists every candidate pair
-        const size_t cap = c.exact_guard == 2 ? 48 * (size_t)c.alloc_tris : std::max<size_t>(1 << 16, 2 * c.alloc_tris);
-        if (cap > c.alloc_ulist) {
-            PAMO_TRY(dalloc(&c.ulist, cap, c.stream));
-            c.alloc_ulist = cap;
-        }
-        u.list = c.ulist;
-        u.cap = (int)std::min<size_t>(c.alloc_ulist, 0x7fffffff);
-        PAMO_HIP(hipMemsetAsync(c.dcnt + C_UNDECIDED, 0, sizeof(int), c.stream));
-        LAUNCHP(K_GUARD_QUERY, guard_bytes, (guard_query_k<kGuardStack, true>), guard_threads, m, c.qlist, c.dcnt,
-                c.changed, (const float4*)c.bbox, (const int*)c.bslot, 1e-3f, c.flagged, u, part_log, c.dcnt + C_WALK_ERR, c.walk_cap);
-        hipLaunchKernelGGL(exact_pairs_k, dim3(1024), dim3(kBlock), 0, c.stream, m, (const int2*)c.ulist,
-                           (const int*)(c.dcnt + C_UNDECIDED), u.cap, c.flagged);
-        PAMO_HIP(hipGetLastError());
-    } else if (c.guard_small_stack) {
-        LAUNCHP(K_GUARD_QUERY, guard_bytes, (guard_query_k<kGuardStackSmall, false>), guard_threads, m, c.qlist,
-                c.dcnt, c.changed, (const float4*)c.bbox, (const int*)c.bslot, 1e-3f, c.flagged, u, part_log, c.dcnt + C_WALK_ERR, c.walk_cap);
-    } else if (c.guard_waves == 4) {
-        LAUNCHP(K_GUARD_QUERY, guard_bytes, guard_query_w4_k, guard_threads, m, c.qlist, c.dcnt, c.changed,
-                (const float4*)c.bbox, (const int*)c.bslot, 1e-3f, c.flagged, u, part_log, c.dcnt + C_WALK_ERR, c.walk_cap);
-    } else {
-        LAUNCHP(K_GUARD_QUERY, guard_bytes, (guard_query_k<kGuardStack, false>), guard_threads, m, c.qlist, c.dcnt,
-                c.changed, (const float4*)c.bbox, (const int*)c.bslot, 1e-3f, c.flagged, u, part_log, c.dcnt + C_WALK_ERR, c.walk_cap);
-    }
-    return 0;
+    return guard_queries(c, nT);
 }
 
 // Undo candidates among the first n_cand records (get_undo_candidate_kernel,
@@ -517,13 +526,29 @@ static int undo_scan(Ctx& c, long long n) {
                      ScanOp{c.occ, c.new_map}, c.n_pts + 1LL, c.lb, c.stream, K_UNDO_CAND, 16.0 * n + 1.0 * c.n_tris);
 }
 
-static int undo_candidates(Ctx& c, int& npushed) {
-    PAMO_TRY(undo_scan(c, c.n_cand));
+//
+// Reads the counters back; with the exact guard and more open pairs than their
+// list holds, the list grows to their number and the queries are asked again.
+static int read_candidates(Ctx& c, long long n) {
+    PAMO_TRY(undo_scan(c, n));
     PAMO_TRY(sync_counters(c));
+    const long long open = c.exact_guard ? c.hcnt[C_UNDECIDED] : 0;
+    if (open <= (long long)std::min<size_t>(c.alloc_ulist, 0x7fffffff)) return 0;
+    const size_t cap = (size_t)open + (size_t)open / 4;
+    PAMO_TRY(dalloc(&c.ulist, cap, c.stream));
+    c.alloc_ulist = cap;
+    PAMO_TRY(guard_queries(c, c.n_tris));
+    PAMO_TRY(undo_scan(c, n));
+    PAMO_TRY(sync_counters(c));
+    PAMO_CHECK(c.hcnt[C_UNDECIDED] <= (long long)std::min<size_t>(c.alloc_ulist, 0x7fffffff),
+               "exact guard: more pairs left open than the list holds");
+    return 0;
+}
+
+static int undo_candidates(Ctx& c, int& npushed) {
+    PAMO_TRY(read_candidates(c, c.n_cand));
     npushed = c.hcnt[C_PUSHED];
     c.tree_n = c.hcnt[C_NLIVE];  // leaves of the tree this guard used
-    PAMO_CHECK(!c.exact_guard || c.hcnt[C_UNDECIDED] <= (long long)c.alloc_ulist,
-               "exact guard: more pairs left undecided than the list holds");
     return 0;
 }
 
@@ -672,16 +697,13 @@ static int round_device(Ctx& c, int nP, int nT, float scale, float thr, bool is_
     // edge count and by half the points plus 512 (regular collapses share
     // no vertex)
     const long long cand_bound = std::min<long long>(nE, nP / 2 + 512);
-    PAMO_TRY(undo_scan(c, cand_bound));
-    PAMO_TRY(sync_counters(c));
+    PAMO_TRY(read_candidates(c, cand_bound));
     c.n_edges = c.hcnt[C_NEDGE];
     c.n_regular = c.hcnt[C_NREG];
     c.n_rec = c.n_regular + c.hcnt[C_LINE];
     c.n_cand = std::min(c.n_rec, (c.n_regular + 511) / 512 * 512);
     c.tree_n = c.hcnt[C_NLIVE];
     PAMO_CHECK(c.n_cand <= cand_bound, "undo candidates beyond their launch bound");
-    PAMO_CHECK(!c.exact_guard || c.hcnt[C_UNDECIDED] <= (long long)c.alloc_ulist,
-               "exact guard: more pairs left undecided than the list holds");
     int first = c.n_vertices_undo;  // entries already placed by the prologue
     int npushed = c.hcnt[C_PUSHED];
     c.undo_iters = 0;

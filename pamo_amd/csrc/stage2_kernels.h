@@ -1687,23 +1687,22 @@ __device__ __forceinline__ void load_xtri(Mesh m, int f, XP3* p, int* idx) {
     }
 }
 
-// Exact mode, first pass: the decision with filtered predicates; a pair they
-// cannot decide is listed for exact_pairs_k.
-__device__ __noinline__ void eval_pair_filtered(Mesh m, int a, int b, uint8_t* __restrict__ flagged, Undecided u) {
+__device__ __forceinline__ XFace load_xface(Mesh m, int f) {
+    const int i = m.i[f], j = m.j[f], k = m.k[f];
+    const float4 p = m.p[i], q = m.p[j], r = m.p[k];
+    return XFace{XP3{p.x, p.y, p.z}, XP3{q.x, q.y, q.z}, XP3{r.x, r.y, r.z}, i, j, k};
+}
+
+// Exact mode, first pass: what filtered signs decide; the other pairs are
+// listed for exact_pairs_k.
+__device__ __forceinline__ void eval_pair_quick(Mesh m, int a, int b, uint8_t* __restrict__ flagged, Undecided u) {
     if (!u.force) {
-        XP3 pa[3], pb[3];
-        int ia[3], ib[3];
-        load_xtri(m, a, pa, ia);
-        load_xtri(m, b, pb, ib);
-        XPred<false> pr;
-        const bool hit = x_faces_intersect(pr, ia, pa, ib, pb);
-        if (!pr.undecided) {
-            if (hit) {
-                flagged[a] = 1;
-                flagged[b] = 1;
-            }
-            return;
+        const int r = x_faces_quick(load_xface(m, a), load_xface(m, b));
+        if (r == kMeet) {
+            flagged[a] = 1;
+            flagged[b] = 1;
         }
+        if (r != kUnsure) return;
     }
     const int k = atomicAdd(u.count, 1);
     if (k < u.cap) u.list[k] = make_int2(a, b);
@@ -1712,12 +1711,12 @@ __device__ __noinline__ void eval_pair_filtered(Mesh m, int a, int b, uint8_t* _
 template <bool kExact>
 __device__ __forceinline__ void guard_eval(Mesh m, int a, int b, float epsilon, uint8_t* __restrict__ flagged,
                                            Undecided u) {
-    if (kExact) eval_pair_filtered(m, a, b, flagged, u);
+    if (kExact) eval_pair_quick(m, a, b, flagged, u);
     else eval_pair(m, a, b, epsilon, flagged);
 }
 
 // Exact mode, second pass: the listed pairs with exact predicates.
-__global__ void __launch_bounds__(kBlock) exact_pairs_k(Mesh m, const int2* __restrict__ list,
+__global__ void __launch_bounds__(kWave) exact_pairs_k(Mesh m, const int2* __restrict__ list,
                                                         const int* __restrict__ count, int cap,
                                                         uint8_t* __restrict__ flagged) {
     const int n = min(*count, cap);
@@ -1727,8 +1726,7 @@ __global__ void __launch_bounds__(kBlock) exact_pairs_k(Mesh m, const int2* __re
         int ia[3], ib[3];
         load_xtri(m, e.x, pa, ia);
         load_xtri(m, e.y, pb, ib);
-        XPred<true> pr;
-        if (x_faces_intersect(pr, ia, pa, ib, pb)) {
+        if (x_faces_intersect(ia, pa, ib, pb)) {
             flagged[e.x] = 1;
             flagged[e.y] = 1;
         }
