@@ -78,7 +78,8 @@ int pamo_ctx_set_stream(pamo_ctx* ctx, void* stream, int own);
  * change): on meshes of at most PAMO_OPT_GUARD_SPLIT_FACES faces (default
  * 65536) each group of queries is served by 2^PAMO_OPT_GUARD_SPLIT_LOG
  * waves (default 3, at most 4), one per subtree under the root, so that one
- * query with a large box does not hold a late-round launch in one wave. */
+ * query with a large box does not hold a late-round launch in one wave; on
+ * any mesh waves without a query take finer subtrees. */
 #define PAMO_OPT_GUARD_SPLIT_FACES 6
 #define PAMO_OPT_GUARD_SPLIT_LOG 7
 /* Guard register budget (no counterpart in the reference; results do not

@@ -414,18 +414,18 @@ static int sync_counters(Ctx& c) {
 static int guard_queries(Ctx& c, int nT) {
     Mesh m = cur_mesh(c);
     const double nP = c.n_pts;
-    // meshes up to 256k faces split every query group over 8 subtrees: late
-    // rounds hold few queries, and one query with a large box would otherwise
-    // hold a whole launch in one wave
+    // meshes up to guard_split_faces split every query group over 8 subtrees at
+    // least (the kernel splits further where queries are few): one query with
+    // a large box would otherwise hold a whole launch in one wave
     const int part_log = nT <= c.guard_split_faces ? c.guard_split_log : 0;
     const long long guard_threads = ((((long long)nT + kGuardQ - 1) / kGuardQ) << part_log) * kWave;
     const double guard_bytes = 4.0 * nT + 12.0 * nT + 16.0 * nP + 64.0 * nT + 1.0 * nT + 1.0 * nT;
     Undecided u{nullptr, c.dcnt + C_UNDECIDED, 0, c.exact_guard == 2 ? 1 : 0};
     if (c.exact_guard) {
-        // list capacity: the pairs that filtered signs leave open are those
-        // whose planes both cross the other face, or touch it (a few per
-        // changed face at most; read_candidates grows it for more); the test
-        // setting lists every candidate pair
+        // list capacity: the pairs that filtered signs leave open, whose
+        // planes both cross or touch the other face, and those of waves with
+        // many pairs; a few per changed face (read_candidates grows it for
+        // more); the test setting lists every candidate pair
         const size_t cap = c.exact_guard == 2 ? 48 * (size_t)c.alloc_tris : std::max<size_t>(1 << 16, 2 * c.alloc_tris);
         if (cap > c.alloc_ulist) {
             PAMO_TRY(dalloc(&c.ulist, cap, c.stream));

@@ -1651,6 +1651,18 @@ __device__ __forceinline__ void eval_pair(Mesh m, int a, int b, float epsilon, u
 
 constexpr int kQueue = 192;   // per-wave pair queue (< 64 pending + one append of <= 128)
 constexpr int kGuardQ = 8;    // guard queries per wave
+// A launch covers a group of kGuardQ queries for every kGuardQ faces; where
+// few faces are queries, the idle waves take finer subtrees: the split is
+// doubled while all waves at work stay within kSplitWaves (half of the 16384
+// that can be resident), to at most 2^kMaxSplit subtrees.  A face that is long
+// and thin overlaps thousands of boxes, and such faces come in groups: 120k
+// faces with the exact guard 148 -> 122 ms a run, from 2M to 20k faces 304.5 ->
+// 301 (16384 waves: 307, to 2^6 subtrees: 133 and 303).
+constexpr int kMaxSplit = 8, kSplitWaves = 8192;
+// Exact mode: a wave decides its first kInWave batches of 64 pairs, and hands
+// further full batches to exact_pairs_k, which spreads them over the chip
+// (122 -> 106 ms a run; 4 batches: 109, 16: 111).
+constexpr int kInWave = 1;
 constexpr int kGuardStack = 512;       // per-wave frontier entries
 constexpr int kGuardStackSmall = 32;   // test variant: forces the overflow walk
 
@@ -1678,25 +1690,17 @@ struct Undecided {
     int force;  // test setting: every pair goes to the exact pass
 };
 
-__device__ __forceinline__ void load_xtri(Mesh m, int f, XP3* p, int* idx) {
-    idx[0] = m.i[f]; idx[1] = m.j[f]; idx[2] = m.k[f];
-#pragma unroll
-    for (int v = 0; v < 3; ++v) {
-        const float4 q = m.p[idx[v]];
-        p[v] = XP3{q.x, q.y, q.z};
-    }
-}
-
 __device__ __forceinline__ XFace load_xface(Mesh m, int f) {
     const int i = m.i[f], j = m.j[f], k = m.k[f];
     const float4 p = m.p[i], q = m.p[j], r = m.p[k];
     return XFace{XP3{p.x, p.y, p.z}, XP3{q.x, q.y, q.z}, XP3{r.x, r.y, r.z}, i, j, k};
 }
 
-// Exact mode, first pass: what filtered signs decide; the other pairs are
-// listed for exact_pairs_k.
-__device__ __forceinline__ void eval_pair_quick(Mesh m, int a, int b, uint8_t* __restrict__ flagged, Undecided u) {
-    if (!u.force) {
+// Exact mode, first pass: what filtered signs decide; the other pairs, and
+// those left for later, are listed for exact_pairs_k.
+__device__ __forceinline__ void eval_pair_quick(Mesh m, int a, int b, uint8_t* __restrict__ flagged, Undecided u,
+                                                bool later) {
+    if (!u.force && !later) {
         const int r = x_faces_quick(load_xface(m, a), load_xface(m, b));
         if (r == kMeet) {
             flagged[a] = 1;
@@ -1710,23 +1714,26 @@ __device__ __forceinline__ void eval_pair_quick(Mesh m, int a, int b, uint8_t* _
 
 template <bool kExact>
 __device__ __forceinline__ void guard_eval(Mesh m, int a, int b, float epsilon, uint8_t* __restrict__ flagged,
-                                           Undecided u) {
-    if (kExact) eval_pair_quick(m, a, b, flagged, u);
+                                           Undecided u, bool later = false) {
+    if (kExact) eval_pair_quick(m, a, b, flagged, u, later);
     else eval_pair(m, a, b, epsilon, flagged);
 }
 
-// Exact mode, second pass: the listed pairs with exact predicates.
+// Exact mode, second pass: the listed pairs, filtered and then exact.
 __global__ void __launch_bounds__(kWave) exact_pairs_k(Mesh m, const int2* __restrict__ list,
                                                         const int* __restrict__ count, int cap,
                                                         uint8_t* __restrict__ flagged) {
     const int n = min(*count, cap);
     for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
         const int2 e = list[k];
-        XP3 pa[3], pb[3];
-        int ia[3], ib[3];
-        load_xtri(m, e.x, pa, ia);
-        load_xtri(m, e.y, pb, ib);
-        if (x_faces_intersect(ia, pa, ib, pb)) {
+        const XFace A = load_xface(m, e.x), B = load_xface(m, e.y);
+        int r = x_faces_quick(A, B);
+        if (r == kUnsure) {
+            const XP3 pa[3] = {A.p0, A.p1, A.p2}, pb[3] = {B.p0, B.p1, B.p2};
+            const int ia[3] = {A.i0, A.i1, A.i2}, ib[3] = {B.i0, B.i1, B.i2};
+            r = x_faces_intersect(ia, pa, ib, pb) ? kMeet : kApart;
+        }
+        if (r == kMeet) {
             flagged[e.x] = 1;
             flagged[e.y] = 1;
         }
@@ -1801,13 +1808,16 @@ __device__ __forceinline__ void guard_query_body(Mesh m, const int* __restrict__
     __shared__ float4 qbox[kW][kGuardQ][2];
     __shared__ int4 qid[kW][kGuardQ];
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x >> 6;
-    // wave -> (query group, subtree): the 2^part_log waves of a group each
-    // walk one subtree, so one heavy query spreads over several waves
     const long long wid = (long long)blockIdx.x * kW + w;
-    const long long q0 = (wid >> part_log) * kGuardQ;
-    const int part = (int)(wid & ((1 << part_log) - 1));
     const int nq = cnt[C_NQUERY];
     const int n = cnt[C_NLIVE];
+    const long long groups = (nq + kGuardQ - 1) / kGuardQ, waves = (long long)gridDim.x * kW;
+    const long long room = waves < kSplitWaves ? waves : kSplitWaves;
+    while (part_log < kMaxSplit && (groups << (part_log + 1)) <= room) ++part_log;
+    // wave -> (query group, subtree): the 2^part_log waves of a group each
+    // walk one subtree, so one heavy query spreads over several waves
+    const long long q0 = (wid >> part_log) * kGuardQ;
+    const int part = (int)(wid & ((1 << part_log) - 1));
     if (q0 >= nq || n <= 1) return;  // uniform per wave
     long long at;
     const int root = subtree_link(box, part, part_log, &at);
@@ -1842,6 +1852,7 @@ __device__ __forceinline__ void guard_query_body(Mesh m, const int* __restrict__
         max_steps = min(max_steps, walk_cap);
         max_visits = min(max_visits, walk_cap);
     }
+    int batches = 0;
     for (long long steps = 0; size > 0; ++steps) {
         if (steps >= max_steps) {  // wave-uniform
             if (lane == 0) walk_overrun(err);
@@ -1900,7 +1911,8 @@ __device__ __forceinline__ void guard_query_body(Mesh m, const int* __restrict__
             const int2 e = pq[w][qn - kWave + lane];
             const int4 id = qid[w][e.x];
             if (guard_candidate<kExact>(m, changed, id.x, id.y, id.z, id.w, e.y))
-                guard_eval<kExact>(m, id.x, e.y, epsilon, flagged, u);
+                guard_eval<kExact>(m, id.x, e.y, epsilon, flagged, u, batches >= kInWave);
+            ++batches;
             qn -= kWave;
             wave_sync();
         }
