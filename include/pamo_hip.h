@@ -82,10 +82,9 @@ int pamo_ctx_set_stream(pamo_ctx* ctx, void* stream, int own);
  * any mesh waves without a query take finer subtrees. */
 #define PAMO_OPT_GUARD_SPLIT_FACES 6
 #define PAMO_OPT_GUARD_SPLIT_LOG 7
-/* Guard register budget (no counterpart in the reference; results do not
- * change): 0 runs the guard kernel as the compiler allocates its registers
- * (129 vector registers, 3 waves per SIMD), 4 (default) a variant capped at
- * 128 so that 4 waves fit per SIMD. */
+/* Guard register budget (no counterpart in the reference): 0 or 4 (default).
+ * Kept for callers that set it: the guard kernel has one variant, whose
+ * registers (112) let 4 waves run per SIMD. */
 #define PAMO_OPT_GUARD_WAVES 8
 /* Edge-cost launch shape (no counterpart in the reference; results do not
  * change): 1 lane per edge, or 4 (default) / 8 lanes sharing one edge's

@@ -374,7 +374,7 @@ __device__ bool x_faces_intersect(const int* ia, const XP3* pa, const int* ib, c
 // Most candidates share a vertex or an edge and end here after one to five
 // determinants, in 104 registers and no scratch memory; with the whole decision
 // in the query kernel it took 248 registers and 208 B of scratch a lane.  A run
-// on 120k faces with slivers: 118 us a query launch (336 before), 42 us for
+// on 200k faces with slivers: 118 us a query launch (336 before), 42 us for
 // the open pairs (115 before, with expansions in scratch memory).
 enum { kApart = 0, kMeet = 1, kUnsure = 2 };
 

@@ -160,7 +160,7 @@ struct Ctx {
     // each query group with 2^guard_split_log waves, one per subtree
     int guard_split_faces = 1 << 16;
     int guard_split_log = 3;
-    int guard_waves = 4;        // 0: the compiler's register allocation for the guard; 4: capped for 4 waves
+    int guard_waves = 4;        // accepted, no effect: the guard's own registers allow 4 waves per SIMD
     int edge_lanes = 4;         // lanes per edge in the edge-cost kernel (1, 4 or 8)
     int ring_lanes = 8;         // lanes per item in the quadric, selection and undo kernels (1, 4 or 8)
     float* cent_out = nullptr;  // pamo_centroid's result (3 floats)
@@ -435,19 +435,16 @@ static int guard_queries(Ctx& c, int nT) {
         u.cap = (int)std::min<size_t>(c.alloc_ulist, 0x7fffffff);
         PAMO_HIP(hipMemsetAsync(c.dcnt + C_UNDECIDED, 0, sizeof(int), c.stream));
         LAUNCHP(K_GUARD_QUERY, guard_bytes, (guard_query_k<kGuardStack, true>), guard_threads, m, c.qlist, c.dcnt,
-                c.changed, (const float4*)c.bbox, (const int*)c.bslot, 1e-3f, c.flagged, u, part_log, c.dcnt + C_WALK_ERR, c.walk_cap);
+                c.changed, (const float4*)c.bbox, 1e-3f, c.flagged, u, part_log, c.dcnt + C_WALK_ERR, c.walk_cap);
         hipLaunchKernelGGL(exact_pairs_k, dim3(2048), dim3(kWave), 0, c.stream, m, (const int2*)c.ulist,
                            (const int*)(c.dcnt + C_UNDECIDED), u.cap, c.flagged);
         PAMO_HIP(hipGetLastError());
     } else if (c.guard_small_stack) {
         LAUNCHP(K_GUARD_QUERY, guard_bytes, (guard_query_k<kGuardStackSmall, false>), guard_threads, m, c.qlist,
-                c.dcnt, c.changed, (const float4*)c.bbox, (const int*)c.bslot, 1e-3f, c.flagged, u, part_log, c.dcnt + C_WALK_ERR, c.walk_cap);
-    } else if (c.guard_waves == 4) {
-        LAUNCHP(K_GUARD_QUERY, guard_bytes, guard_query_w4_k, guard_threads, m, c.qlist, c.dcnt, c.changed,
-                (const float4*)c.bbox, (const int*)c.bslot, 1e-3f, c.flagged, u, part_log, c.dcnt + C_WALK_ERR, c.walk_cap);
+                c.dcnt, c.changed, (const float4*)c.bbox, 1e-3f, c.flagged, u, part_log, c.dcnt + C_WALK_ERR, c.walk_cap);
     } else {
         LAUNCHP(K_GUARD_QUERY, guard_bytes, (guard_query_k<kGuardStack, false>), guard_threads, m, c.qlist, c.dcnt,
-                c.changed, (const float4*)c.bbox, (const int*)c.bslot, 1e-3f, c.flagged, u, part_log, c.dcnt + C_WALK_ERR, c.walk_cap);
+                c.changed, (const float4*)c.bbox, 1e-3f, c.flagged, u, part_log, c.dcnt + C_WALK_ERR, c.walk_cap);
     }
     return 0;
 }

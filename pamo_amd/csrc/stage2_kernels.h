@@ -1655,7 +1655,7 @@ constexpr int kGuardQ = 8;    // guard queries per wave
 // few faces are queries, the idle waves take finer subtrees: the split is
 // doubled while all waves at work stay within kSplitWaves (half of the 16384
 // that can be resident), to at most 2^kMaxSplit subtrees.  A face that is long
-// and thin overlaps thousands of boxes, and such faces come in groups: 120k
+// and thin overlaps thousands of boxes, and such faces come in groups: 200k
 // faces with the exact guard 148 -> 122 ms a run, from 2M to 20k faces 304.5 ->
 // 301 (16384 waves: 307, to 2^6 subtrees: 133 and 303).
 constexpr int kMaxSplit = 8, kSplitWaves = 8192;
@@ -1664,7 +1664,8 @@ constexpr int kMaxSplit = 8, kSplitWaves = 8192;
 // (122 -> 106 ms a run; 4 batches: 109, 16: 111).
 constexpr int kInWave = 1;
 constexpr int kGuardStack = 512;       // per-wave frontier entries
-constexpr int kGuardStackSmall = 32;   // test variant: forces the overflow walk
+constexpr int kGuardStackSmall = 32;   // test variant: pops few entries a step
+constexpr int kTreeDepth = 66;         // 32 key bits, 32 index bits and the root
 
 // Candidate filter for queried face a (vertex ids ia0..ia2) and a live face b
 // whose box overlaps a's (closed intervals): b != a; a pair of queried faces
@@ -1740,46 +1741,6 @@ __global__ void __launch_bounds__(kWave) exact_pairs_k(Mesh m, const int2* __res
     }
 }
 
-// Stackless walk of the subtree below internal node `top`, evaluating
-// candidates in this lane: a node's children in turn, back up by the slots.
-// Inlined: as a called function its register needs add to the caller's (242
-// registers, 2 waves per SIMD, against 129 inlined).
-template <bool kExact>
-__device__ __forceinline__ void guard_walk_subtree(Mesh m, const uint8_t* __restrict__ changed,
-                                                   const float4* __restrict__ box, const int* __restrict__ slot,
-                                                   int top, float4 qlo, float4 qhi, int a, int ia0, int ia1, int ia2,
-                                                   float epsilon, uint8_t* __restrict__ flagged, Undecided u,
-                                                   int* err, long long max_visits) {
-    int x = top, side = 0;
-    for (long long visits = 0;; ++visits) {
-        if (visits >= 3 * max_visits || x < 0) {
-            walk_overrun(err);
-            return;
-        }
-        if (side == 2) {  // both children done
-            if (x == top) return;
-            const int up = slot[x];
-            x = up >> 1;
-            side = (up & 1) + 1;
-            continue;
-        }
-        const float4 lo = box[4 * (long long)x + 2 * side], hi = box[4 * (long long)x + 2 * side + 1];
-        if (!overlap(qlo, qhi, lo, hi)) {
-            ++side;
-            continue;
-        }
-        const int link = __float_as_int(lo.w);
-        if (link >= 0) {
-            x = link;
-            side = 0;
-        } else {
-            if (guard_candidate<kExact>(m, changed, a, ia0, ia1, ia2, ~link))
-                guard_eval<kExact>(m, a, ~link, epsilon, flagged, u);
-            ++side;
-        }
-    }
-}
-
 // Guard queries (self_intersect.cuh:151-392 restricted to changed faces):
 // every queried face a against every live face b whose box overlaps a's.
 //
@@ -1789,21 +1750,24 @@ __device__ __forceinline__ void guard_walk_subtree(Mesh m, const uint8_t* __rest
 // ones and appends the overlapping leaves to a pair queue, which the wave
 // evaluates 64 pairs at a time.  The critical path is then the wave's total
 // node count / 64 plus the tree depth, instead of the longest single walk.
-// (With node records and the children pushed untested, half of the pops found
-// no overlap; a launch still takes 60-64 us on average over a run from 2M to
-// 20k faces either way, and 37 us where it took 34-36 on 200k: what is gained
-// is the node records, which the box kernels no longer write.)
-// When the frontier is full, a lane walks the rest of its subtree by itself
-// (exact, only slower).  The flags are idempotent, so the visiting order does
-// not change the result.
+//
+// As many entries are popped as leave the pushes room in kStackCap, at least
+// one: popped one by one, the newest first, the frontier grows by no more than
+// the depth below an entry, kTreeDepth in all.  So it never overflows, and the
+// evaluation stands in one place: 112 registers, 4 waves per SIMD.  (A lane that
+// walked on by itself when the frontier was full, with two more copies of the
+// evaluation, took 137, or 128 and scratch memory: 60 us a launch over a run
+// from 2M to 20k faces, now 49; the first guard of 370k faces 124 -> 95 us.)
+// The flags are idempotent, so the visiting order does not change the result.
 template <int kStackCap, bool kExact>
-__device__ __forceinline__ void guard_query_body(Mesh m, const int* __restrict__ list, const int* __restrict__ cnt,
-                                                 const uint8_t* __restrict__ changed,
-                                                 const float4* __restrict__ box, const int* __restrict__ slot,
-                                                 float epsilon, uint8_t* __restrict__ flagged, Undecided u,
-                                                 int part_log, int* err, long long walk_cap) {
+__global__ void __launch_bounds__(kBlock) guard_query_k(Mesh m, const int* __restrict__ list,
+                                                        const int* __restrict__ cnt,
+                                                        const uint8_t* __restrict__ changed,
+                                                        const float4* __restrict__ box, float epsilon,
+                                                        uint8_t* __restrict__ flagged, Undecided u, int part_log,
+                                                        int* err, long long walk_cap) {
     constexpr int kW = kBlock / kWave;
-    __shared__ int2 stk[kW][kStackCap];
+    __shared__ int2 stk[kW][kStackCap + kTreeDepth];
     __shared__ int2 pq[kW][kQueue];
     __shared__ float4 qbox[kW][kGuardQ][2];
     __shared__ int4 qid[kW][kGuardQ];
@@ -1847,18 +1811,15 @@ __device__ __forceinline__ void guard_query_body(Mesh m, const int* __restrict__
     }
     wave_sync();
     // bounds of a valid tree; walk_cap > 0 lowers them (tests of the error path)
-    long long max_steps = (long long)nl * (2LL * n - 1), max_visits = 2LL * n;
-    if (walk_cap > 0) {
-        max_steps = min(max_steps, walk_cap);
-        max_visits = min(max_visits, walk_cap);
-    }
+    long long max_steps = (long long)nl * (2LL * n - 1);
+    if (walk_cap > 0) max_steps = min(max_steps, walk_cap);
     int batches = 0;
-    for (long long steps = 0; size > 0; ++steps) {
-        if (steps >= max_steps) {  // wave-uniform
+    for (long long steps = 0;; ++steps) {
+        if (steps > max_steps) {  // wave-uniform
             if (lane == 0) walk_overrun(err);
             return;
         }
-        const int take = size < kWave ? size : kWave;
+        const int take = min(min(size, kWave), max(kStackCap - size, 1));
         int l = 0, x = -1;
         if (lane < take) {
             const int2 e = stk[w][size - take + lane];
@@ -1892,57 +1853,30 @@ __device__ __forceinline__ void guard_query_body(Mesh m, const int* __restrict__
         qn += (int)__popcll(l1);
         const uint64_t m0 = __ballot(c0 >= 0), m1 = __ballot(c1 >= 0);
         const int p0 = size + lanes_below(m0), p1 = size + (int)__popcll(m0) + lanes_below(m1);
-        if (c0 >= 0 && p0 < kStackCap) stk[w][p0] = make_int2(l, c0);
-        if (c1 >= 0 && p1 < kStackCap) stk[w][p1] = make_int2(l, c1);
         const int full = size + (int)__popcll(m0) + (int)__popcll(m1);
-        if (full > kStackCap) {  // wave-uniform: pushes that fit form a prefix
-            const bool o0 = c0 >= 0 && p0 >= kStackCap, o1 = c1 >= 0 && p1 >= kStackCap;
-            for (int k = 0; k < 2; ++k) {
-                if (k == 0 ? o0 : o1) {
-                    const int4 id = qid[w][l];
-                    guard_walk_subtree<kExact>(m, changed, box, slot, k == 0 ? c0 : c1, qlo, qhi, id.x, id.y, id.z,
-                                               id.w, epsilon, flagged, u, err, max_visits);
-                }
-            }
+        if (full > kStackCap + kTreeDepth) {  // wave-uniform; a tree deeper than its keys allow
+            if (lane == 0) walk_overrun(err);
+            return;
         }
-        size = min(full, kStackCap);
+        if (c0 >= 0) stk[w][p0] = make_int2(l, c0);
+        if (c1 >= 0) stk[w][p1] = make_int2(l, c1);
+        size = full;
         wave_sync();
-        while (qn >= kWave) {
-            const int2 e = pq[w][qn - kWave + lane];
-            const int4 id = qid[w][e.x];
-            if (guard_candidate<kExact>(m, changed, id.x, id.y, id.z, id.w, e.y))
-                guard_eval<kExact>(m, id.x, e.y, epsilon, flagged, u, batches >= kInWave);
+        while (qn >= kWave || (size == 0 && qn > 0)) {
+            const int some = min(qn, kWave);
+            if (lane < some) {
+                const int2 e = pq[w][qn - some + lane];
+                const int4 id = qid[w][e.x];
+                if (guard_candidate<kExact>(m, changed, id.x, id.y, id.z, id.w, e.y))
+                    guard_eval<kExact>(m, id.x, e.y, epsilon, flagged, u, batches >= kInWave);
+            }
             ++batches;
-            qn -= kWave;
+            qn -= some;
             wave_sync();
         }
-    }
-    if (lane < qn) {
-        const int2 e = pq[w][lane];
-        const int4 id = qid[w][e.x];
-        if (guard_candidate<kExact>(m, changed, id.x, id.y, id.z, id.w, e.y))
-            guard_eval<kExact>(m, id.x, e.y, epsilon, flagged, u);
+        if (size == 0) return;
     }
 }
-
-#define PAMO_GUARD_PARAMS                                                                                  \
-    Mesh m, const int* __restrict__ list, const int* __restrict__ cnt, const uint8_t* __restrict__ changed,   \
-        const float4* __restrict__ box, const int* __restrict__ slot, float epsilon, uint8_t* __restrict__ flagged, Undecided u, int part_log, int* err, long long walk_cap
-#define PAMO_GUARD_ARGS m, list, cnt, changed, box, slot, epsilon, flagged, u, part_log, err, walk_cap
-
-template <int kStackCap, bool kExact>
-__global__ void __launch_bounds__(kBlock) guard_query_k(PAMO_GUARD_PARAMS) {
-    guard_query_body<kStackCap, kExact>(PAMO_GUARD_ARGS);
-}
-
-// The same guard with its registers capped for 4 waves per SIMD (the
-// compiler's own allocation is one register over); the results do not
-// change.
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) guard_query_w4_k(PAMO_GUARD_PARAMS) {
-    guard_query_body<kGuardStack, false>(PAMO_GUARD_ARGS);
-}
-#undef PAMO_GUARD_PARAMS
-#undef PAMO_GUARD_ARGS
 
 // ---------------------------------------------------------------- undo (A14)
 // What an undo leaves in a restored vertex's minimum key, which nothing reads
@@ -2142,7 +2076,7 @@ __global__ void __launch_bounds__(kCentThreads) centroid_seq_k(const float* __re
 // query raises it, and a face that is restored, or hangs on a vertex that
 // moves back, has such a vertex.  changed[f] is 1 for a query of this guard
 // and 3 for a changed face that is not one.  Blocks of 256 leaves without a
-// restored vertex keep their boxes.  (Runs on 120k faces with the exact guard
+// restored vertex keep their boxes.  (Runs on 200k faces with the exact guard
 // 118 -> 103 ms, from 2M to 20k faces with the other one 390 -> 385.)
 __global__ void __launch_bounds__(kBlock) guard_leaves_k(Mesh m, int nT, uint32_t* __restrict__ val, int carry,
                                                          const int* __restrict__ fpos, int nOld, int again,
