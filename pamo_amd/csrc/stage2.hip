@@ -14,6 +14,7 @@
 //   LBVH + guard ...... simp_cuda/src/bvh/{bvh,morton_code,query,self_intersect}.cuh
 //   round loop ........ simp_cuda/pamo/__init__.py:147-185
 #include <algorithm>
+#include <chrono>
 #include <cstring>
 #include <vector>
 
@@ -138,7 +139,9 @@ struct Ctx {
     int* ws = nullptr;
     LookbackScan lb;  // single-launch scans of the round loop
     int* dcnt = nullptr;
-    int* hcnt = nullptr;
+    int hcnt[C_COUNT] = {};              // the counters as last read
+    unsigned long long* pub = nullptr;  // pinned, where publish_k writes them
+    unsigned pub_seq = 0;
     // last round, host view
     int edge_bound = 0;  // edges that the round's launches cover
     int n_pts = 0, n_tris = 0, n_edges = 0, n_rec = 0, n_regular = 0, n_vertices_undo = 0;
@@ -354,7 +357,7 @@ static void free_all(Ctx& c) {
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
     lookback_free(c.lb);
-    if (c.hcnt) (void)hipHostFree(c.hcnt);
+    if (c.pub) (void)hipHostFree(c.pub);
 }
 
 static Feistel make_feistel(uint64_t m) {
@@ -396,9 +399,35 @@ static Orig orig_mesh(Ctx& c) { return Orig{c.op, c.oi, c.oj, c.ok}; }
 
 // Reads the device counters; reports (and clears) the error flags that
 // kernels set instead of reading out of bounds or walking a corrupted tree.
+//
+// A copy and a wait on the stream take some 20 us beside the work they wait
+// for, two or more times a round.  A one-wave kernel writes the counters to
+// pinned memory instead, and the host looks for this read's number for up to
+// kPollUs, after which (a long round, or an error) it waits on the stream
+// (1280 faces 4.6 -> 3.9 ms a run, 90k faces 43.4 -> 40; 40 us: 4.3 and 42.3).
+constexpr int kPollUs = 200;
 static int sync_counters(Ctx& c) {
-    PAMO_HIP(hipMemcpyAsync(c.hcnt, c.dcnt, sizeof(int) * C_COUNT, hipMemcpyDeviceToHost, c.stream));
-    PAMO_HIP(hipStreamSynchronize(c.stream));
+    const unsigned seq = ++c.pub_seq;
+    hipLaunchKernelGGL(publish_k, dim3(1), dim3(kWave), 0, c.stream, (const int*)c.dcnt, c.pub, seq);
+    PAMO_HIP(hipGetLastError());
+    const auto t0 = std::chrono::steady_clock::now();
+    int k = 0;  // counters read
+    auto read = [&]() {
+        for (; k < C_COUNT; ++k) {
+            const unsigned long long w = __atomic_load_n(c.pub + k, __ATOMIC_ACQUIRE);
+            if ((unsigned)(w >> 32) != seq) return false;
+            c.hcnt[k] = (int)(unsigned)w;
+        }
+        return true;
+    };
+    while (!read()) {
+        if (std::chrono::steady_clock::now() - t0 >= std::chrono::microseconds(kPollUs)) {
+            PAMO_HIP(hipStreamSynchronize(c.stream));
+            PAMO_CHECK(read(), "counters not written by a finished stream");
+            break;
+        }
+        for (int p = 0; p < 16; ++p) __builtin_ia32_pause();
+    }
     if (c.hcnt[C_WALK_ERR] || c.hcnt[C_BAD_UNDO]) {
         const bool walk = (c.hcnt[C_WALK_ERR] & 1) != 0, scan = (c.hcnt[C_WALK_ERR] & 2) != 0;
         c.hcnt[C_WALK_ERR] = c.hcnt[C_BAD_UNDO] = 0;
@@ -829,7 +858,9 @@ int pamo_ctx_create(pamo_ctx** out, int device) {
     c->stream = c->own_stream;
     if (e == hipSuccess) e = hipMalloc((void**)&c->dcnt, sizeof(int) * pamo::C_COUNT);
     if (e == hipSuccess) e = hipMemsetAsync(c->dcnt, 0, sizeof(int) * pamo::C_COUNT, c->stream);
-    if (e == hipSuccess) e = hipHostMalloc((void**)&c->hcnt, sizeof(int) * pamo::C_COUNT, 0);
+    if (e == hipSuccess) e = hipHostMalloc((void**)&c->pub, sizeof(unsigned long long) * pamo::C_COUNT,
+                                          hipHostMallocCoherent | hipHostMallocMapped);
+    if (e == hipSuccess) memset(c->pub, 0, sizeof(unsigned long long) * pamo::C_COUNT);
     if (e != hipSuccess) {
         pamo::set_error(std::string("pamo_ctx_create: ") + hipGetErrorString(e));
         pamo::free_all(*c);
@@ -1278,6 +1309,7 @@ int pamo_pasp_round(pamo_ctx* ctx, const float* d_pts, int n_pts, const int* d_t
     PAMO_HIP(hipMemcpyAsync(d_out_occ, c.occ, sizeof(int) * n_pts, hipMemcpyDeviceToDevice, c.stream));
     PAMO_HIP(hipMemcpyAsync(d_out_map, c.pts_map, sizeof(int) * n_pts, hipMemcpyDeviceToDevice, c.stream));
     PAMO_TRY(pamo::sync_counters(c));
+    PAMO_HIP(hipStreamSynchronize(c.stream));
     c.n_edges = c.hcnt[pamo::C_NEDGE];
     return 0;
 }

@@ -162,6 +162,17 @@ __global__ void invalid_set_k(const int* __restrict__ undo_in, int n, uint32_t* 
     if (v >= 0 && v < cap) invalid[v] = epoch;
 }
 
+// The counters to pinned host memory, each in one store with the number of
+// this read: a host that sees the number sees that counter, and no fence is
+// needed (one at system scope writes back the caches of kernels beside it).
+__global__ void __launch_bounds__(kWave) publish_k(const int* __restrict__ cnt, unsigned long long* pub, unsigned seq) {
+    static_assert(C_COUNT <= kWave, "one lane per counter");
+    const int k = threadIdx.x;
+    if (k < C_COUNT)
+        __hip_atomic_store(pub + k, ((unsigned long long)seq << 32) | (unsigned)cnt[k], __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ---------------------------------------------------------------- rings and edges (A4, A5)
 
 // One pass over the faces that counts, with the places that the counts leave:
