@@ -79,11 +79,11 @@ static double now_s() {
     return duration<double>(steady_clock::now().time_since_epoch()).count();
 }
 
-// HBM footprint of one job: the stage-2 context's arrays (about 231 B per
+// HBM footprint of one job: the stage-2 context's arrays (about 260 B per
 // face and 128 B per vertex over the round, with the LBVH) plus, with stage
 // 3, the input-surface tree and the CG state of the output mesh.
 static long long estimate_bytes(int nv, int nf, int stage3) {
-    long long b = 260LL * nf + 160LL * nv + (12LL * nv + 12LL * nf);
+    long long b = 290LL * nf + 160LL * nv + (12LL * nv + 12LL * nf);
     if (stage3) b += 160LL * nf + 64LL * nv + (long long)(0.01 * nf) * 4096;
     return b;
 }
