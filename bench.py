@@ -619,7 +619,7 @@ def main():
     traffic, tdetail = (None, "not measured (--no-traffic)")
     if not args.no_traffic:
         # the profiler's name is a fragment of every variant's kernel name
-        # (guard_query_k, guard_query_w4_k, edge_cost_group_k, ...)
+        # (guard_query_k, edge_cost_group_k, ...)
         traffic, tdetail = measure_traffic(dom["name"])
         print(f"[bench] traffic of {dom['name']}: {traffic} bytes per launch ({tdetail})", file=sys.stderr,
               flush=True)
