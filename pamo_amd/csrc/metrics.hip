@@ -170,9 +170,12 @@ __device__ __forceinline__ void near_store(const Near& q, long long i, double* _
     }
 }
 
-// A lower bound in 32 bits of a squared distance (0 where the relative
-// rounding does not hold).
-__device__ __forceinline__ float near_bound(double d) { return d > 1e-30 ? (float)(d * (1.0 - 1.2e-7)) : 0.0f; }
+// A lower bound in 32 bits of a squared distance: 0 where the relative rounding
+// does not hold, the largest number where 32 bits end (distances from 1.8e19
+// on, whose waiting nodes are then always opened).
+__device__ __forceinline__ float near_bound(double d) {
+    return d > 1e-30 ? fminf((float)(d * (1.0 - 1.2e-7)), 3.402823466e38f) : 0.0f;
+}
 
 // The whole tree by parent links, with the best so far: for a walk whose
 // stack ran out.

@@ -69,3 +69,22 @@ def test_points_without_a_distance():
     ok = np.setdiff1d(np.arange(len(P)), bad)
     so, _ = om.point_mesh_sqdist(P[ok], V, F)
     assert np.all(np.abs(sq[ok] - so) <= 1e-12 * so)
+
+
+@pytest.mark.parametrize("n", [300, 5000, 33000])
+@pytest.mark.parametrize("scale", [1e18, 1e20])
+def test_distances_beyond_single_precision(scale, n):
+    """Coordinates that 32-bit boxes hold, squared distances that 32 bits do
+    not (above 3.4e38 from 1.8e19 on): each point count takes another launch."""
+    print(f"case: scale {scale:g}, {n} points", flush=True)
+    V, F = synth.icosphere_sh(level=3, seed=2)
+    V = V.astype(np.float64) * scale
+    rng = np.random.default_rng(n)
+    _check(rng.uniform(-3.0, 3.0, (n, 3)) * scale, V, F)
+
+
+def test_hausdorff_beyond_single_precision():
+    print("case: Hausdorff at 1e20", flush=True)
+    (VA, FA), (VB, FB) = synth.icosphere_sh(level=3, seed=2), synth.icosphere_sh(level=2, seed=5)
+    VA, VB = VA.astype(np.float64) * 1e20, VB.astype(np.float64) * 3e20
+    assert metrics.hausdorff(VA, FA, VB, FB) == pytest.approx(om.hausdorff(VA, FA, VB, FB), rel=1e-12)
