@@ -568,8 +568,13 @@ __global__ void __launch_bounds__(kB) detect_k(const float4* __restrict__ x, int
         qbox[w][lane][0] = make_float4(lo.x, lo.y, lo.z, 0.0f);
         qbox[w][lane][1] = make_float4(hi.x, hi.y, hi.z, 0.0f);
         stk[w][lane] = make_int2(lane, -1);  // root
-        // a tree of one leaf has no pairs: the distance test alone decides
-        one = n_leaves == 1 && (kPT || (int)val[0] > q);
+        // a tree of one leaf has no pair records: its face's box is formed here
+        // (one edge is no pair with itself)
+        if (kPT && n_leaves == 1) {
+            const int4 t = tri[val[0]];
+            const V3 a = v3(x[t.x]), b = v3(x[t.y]), c = v3(x[t.z]);
+            one = box_hit(lo, hi, f4(vmin(a, vmin(b, c))), f4(vmax(a, vmax(b, c))));
+        }
     }
     if (n_leaves == 1) {
         size = 0;
