@@ -1162,11 +1162,11 @@ int pamo_round_debug(pamo_ctx* ctx, int what, void* d_out, long long cap, long l
             else {  // (2n-1) nodes x (lo4, hi4), gathered from the child pairs
                 n = h > 0 ? 8LL * (2 * h - 1) : 0;
                 PAMO_CHECK(n <= cap, "pamo_round_debug: cap too small");
-                if (h > 1)
+                if (h > 0)
                     hipLaunchKernelGGL(pamo::node_records_k, dim3(pamo::grid_for(2LL * h, pamo::kBlock)),
                                        dim3(pamo::kBlock), 0, c.stream, (const int*)c.bleft, (const int2*)c.brange,
                                        (const int*)c.dcnt, (const uint32_t*)c.bval, (const int*)c.bslot,
-                                       (const float4*)c.bbox, (float4*)d_out);
+                                       (const float4*)c.bbox, (const float4*)c.blk, (float4*)d_out);
                 PAMO_HIP(hipGetLastError());
                 PAMO_HIP(hipStreamSynchronize(c.stream));
                 if (n_out) *n_out = n;

@@ -1569,13 +1569,14 @@ __global__ void __launch_bounds__(kBlock) node_box_small_k(const int2* __restric
 // Node records for the tests' readback, in node order: lo.xyz with the left
 // child (a leaf: its item) in lo.w, hi.xyz with the escape node in hi.w (the
 // next node in depth-first order once the subtree is done, -1 past the end).
+// The box of a tree's one leaf is its block's (blk).
 __global__ void __launch_bounds__(kBlock) node_records_k(const int* __restrict__ left, const int2* __restrict__ range,
                                                          const int* __restrict__ cnt, const uint32_t* __restrict__ val,
                                                          const int* __restrict__ slot, const float4* __restrict__ box,
-                                                         float4* __restrict__ node) {
+                                                         const float4* __restrict__ blk, float4* __restrict__ node) {
     const int n = cnt[C_NLIVE];
     const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n <= 1 || x >= 2 * n - 1) return;
+    if (n <= 0 || x >= 2 * n - 1) return;
     // x's subtree ends at leaf b; the next node in depth-first order is the
     // right child of the node that splits between leaves b and b+1.  That
     // child is internal node b+1 when that node's range starts at b+1 (an
@@ -1590,7 +1591,10 @@ __global__ void __launch_bounds__(kBlock) node_records_k(const int* __restrict__
         esc = (c <= n - 2 && range[c].x == c) ? c : c + (n - 1);
     }
     float4 lo, hi;
-    if (x == 0) {
+    if (n == 1) {
+        lo = blk[0];
+        hi = blk[1];
+    } else if (x == 0) {
         const float4 a = box[0], c = box[1], d = box[2], e = box[3];
         lo = make_float4(fminf(a.x, d.x), fminf(a.y, d.y), fminf(a.z, d.z), 0.0f);
         hi = make_float4(fmaxf(c.x, e.x), fmaxf(c.y, e.y), fmaxf(c.z, e.z), 0.0f);

@@ -38,3 +38,36 @@ def test_rounds_of_changing_size_on_one_context(oracle_lib, levels):
             x = x.cpu().numpy()
             assert x.shape == y.shape and x.tobytes() == y.tobytes(), f"call {it}: {n}"
     assert undos > 0 or 3 not in levels, "the case undid nothing"
+
+
+@pytest.mark.parametrize("threshold", [1e-3, 1e-9])
+def test_records_of_a_one_leaf_tree(threshold):
+    """One face: the tree is one leaf, which no child pair holds; its record is
+    the face's box (an empty one where the round removed the face) with the
+    face and no escape, as any leaf's."""
+    import ctypes
+
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from pamo_amd import _hip
+    from pamo_amd.pamo import CUDSP_Free
+    print(f"case: one face, threshold {threshold}", flush=True)
+    V = np.array([[0.5, -0.25, 1.0], [-1.0, 0.125, 0.75], [0.25, 2.0, -0.5]], np.float32)
+    F = np.array([[0, 1, 2]], np.int32)
+    op = CUDSP_Free(0)
+    p, t, *_ = op.forward(torch.from_numpy(V).cuda(), torch.from_numpy(F).cuda(),
+                          torch.zeros(0, dtype=torch.int32, device="cuda"), 0, 3.0, threshold, 0, True)
+    p, t = p.cpu().numpy(), t.cpu().numpy()
+    assert op.debug(_hip.PAMO_DBG_BVH_N) == 1
+    buf = torch.full((8,), 7.0, dtype=torch.float32, device="cuda")
+    n = ctypes.c_longlong(0)
+    _hip.check(_hip.lib().pamo_round_debug(op.ctx.ptr, _hip.PAMO_DBG_BVH_BOXES, buf.data_ptr(), 8, ctypes.byref(n)),
+               "pamo_round_debug")
+    assert n.value == 8
+    box, at = buf.cpu().numpy(), p[t[0]]
+    if t[0, 0] < 0:
+        assert np.all(box[:3] == np.inf) and np.all(box[4:7] == -np.inf)
+    else:
+        assert np.array_equal(box[:3], at.min(0)) and np.array_equal(box[4:7], at.max(0))
+    assert box.view(np.int32)[[3, 7]].tolist() == [0, -1]
