@@ -441,8 +441,8 @@ struct Work {
     int* ws = nullptr;
     int* flags = nullptr;  // [3] device: bad faces, walk overrun, queries left over
     int* h_flags = nullptr;  // [2] host
-    // walk order of the queries (null: the points' own order): Morton keys,
-    // point numbers, and the sort's second pair of buffers
+    // walk order of up to kCallPoints queries (null: the points' own order):
+    // Morton keys, point numbers, and the sort's second pair of buffers
     uint32_t *qkey = nullptr, *qval = nullptr, *qkey2 = nullptr, *qval2 = nullptr;
     int* qws = nullptr;
     long long cap_q = 0;
@@ -489,10 +489,14 @@ static int build_tree(Work& w, hipStream_t st, const double* V, int nV, const in
 
 // Fewer points than this are walked in their own order.
 constexpr long long kSortPoints = 4096;
+// Points that are walked together: the order and leftover buffers that a
+// context keeps hold no more (24 bytes a point: 384 MiB, and the sort's
+// histograms).  20M points against 200k faces: 21.4 ms so, 20.9 in one turn,
+// 22.9 in turns of 2^22.
+constexpr long long kCallPoints = 1LL << 24;
 
-static int query(Work& w, hipStream_t st, const double* P, long long nP, const double* V, const int* F, double* sqd,
-                 int* I, double* C) {
-    if (nP <= 0) return 0;
+static int query_points(Work& w, hipStream_t st, const double* P, long long nP, const double* V, const int* F,
+                        double* sqd, int* I, double* C) {
     const uint32_t* order = nullptr;
     if (nP >= kSortPoints && nP <= w.cap_q && w.tree.n > 1) {
         const float* whole = w.tree.part + 6 * grid_for(w.tree.n, kBlock);
@@ -514,6 +518,14 @@ static int query(Work& w, hipStream_t st, const double* P, long long nP, const d
     return 0;
 }
 
+static int query(Work& w, hipStream_t st, const double* P, long long nP, const double* V, const int* F, double* sqd,
+                 int* I, double* C) {
+    for (long long k = 0; k < nP; k += kCallPoints)
+        PAMO_TRY(query_points(w, st, P + 3 * k, std::min(nP - k, kCallPoints), V, F, sqd + k, I ? I + k : nullptr,
+                              C ? C + 3 * k : nullptr));
+    return 0;
+}
+
 // Clears the walk flag at the start of a call.
 static int begin(Work& w, hipStream_t st) { return fill(w.flags + 1, 0, 1, st); }
 
@@ -526,15 +538,15 @@ static int finish(Work& w, hipStream_t st, const char* who) {
 }
 
 // Sizes the context's tree and workspace for nF faces, and the buffers of the
-// query order for nP points (none for few points, nor beyond the sort's range).
+// query order for nP points (none for few points).
 static int reserve(Ctx& c, int nF, long long nP) {
-    if (nP > c.w.cap_rest && nP < (1LL << 30)) {
+    const long long np = std::min(nP, kCallPoints), cap = std::min(np + np / 4, kCallPoints);
+    if (np > c.w.cap_rest) {
         c.w.cap_rest = 0;
-        PAMO_TRY(s3::dalloc(&c.w.rest, (size_t)(nP + nP / 4), c.stream));
-        c.w.cap_rest = nP + nP / 4;
+        PAMO_TRY(s3::dalloc(&c.w.rest, (size_t)cap, c.stream));
+        c.w.cap_rest = cap;
     }
-    if (nP >= kSortPoints && nP > c.w.cap_q && nP < (1LL << 30)) {
-        const long long cap = nP + nP / 4;
+    if (np >= kSortPoints && np > c.w.cap_q) {
         c.w.cap_q = 0;
         uint32_t** q[] = {&c.w.qkey, &c.w.qval, &c.w.qkey2, &c.w.qval2};
         for (uint32_t** x : q) PAMO_TRY(s3::dalloc(x, (size_t)cap, c.stream));

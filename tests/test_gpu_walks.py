@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from oracle import metrics as om
-from pamo_amd import metrics, synth
+from pamo_amd import _hip, metrics, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -88,3 +88,31 @@ def test_hausdorff_beyond_single_precision():
     (VA, FA), (VB, FB) = synth.icosphere_sh(level=3, seed=2), synth.icosphere_sh(level=2, seed=5)
     VA, VB = VA.astype(np.float64) * 1e20, VB.astype(np.float64) * 3e20
     assert metrics.hausdorff(VA, FA, VB, FB) == pytest.approx(om.hausdorff(VA, FA, VB, FB), rel=1e-12)
+
+
+def test_buffers_of_a_large_call_are_bounded():
+    """A context keeps order and leftover buffers for 2^24 points at most (24
+    bytes each, and the sort's histograms), and points past that number are
+    walked as in calls of their own."""
+    n, cut = 40_000_000, 1 << 24
+    print(f"case: {n} points", flush=True)
+    V, F = synth.icosphere_sh(level=2, seed=4)
+    m = metrics._Metrics(0)
+    Vd, Fd = torch.from_numpy(V.astype(np.float64)).cuda(), torch.from_numpy(F).cuda()
+    P = torch.rand((n, 3), dtype=torch.float64, device="cuda", generator=torch.Generator("cuda").manual_seed(1)) * 4 - 2
+
+    def call(P):
+        k = len(P)
+        out = (torch.empty(k, dtype=torch.float64, device="cuda"), torch.empty(k, dtype=torch.int32, device="cuda"),
+               torch.empty((k, 3), dtype=torch.float64, device="cuda"))
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        _hip.check(_hip.lib().pamo_point_mesh_sqdist(m.ptr, P.data_ptr(), k, Vd.data_ptr(), len(V), Fd.data_ptr(),
+                                                     len(F), *(t.data_ptr() for t in out)), "pamo_point_mesh_sqdist")
+        return out, free - torch.cuda.mem_get_info()[0]
+
+    whole, kept = call(P)
+    assert kept < 640 << 20, kept
+    for a, b in ((0, 5000), (cut - 3000, cut + 3000), (2 * cut - 70000, 2 * cut + 70000), (n - 100, n)):
+        part, _ = call(P[a:b].contiguous())
+        assert all(torch.equal(w[a:b], p) for w, p in zip(whole, part))
