@@ -282,21 +282,28 @@ __device__ __forceinline__ V3 tri_corner(const float4* __restrict__ tri, long lo
     return v3(tri[3 * f + k]);
 }
 
-// Rows of columns (a column is a sample line along the dominant axis, a row
-// the columns of one index of the second other axis) of each triangle's box.
-__global__ void __launch_bounds__(kB) columns_k(const float4* __restrict__ tri, int nF, int R, float band,
-                                                long long* __restrict__ rows) {
+// A column is a sample line along the dominant axis; a row holds the columns of
+// one index of the second other axis, and is worked on in segments of at most
+// 2^seg_log columns.
+__device__ __forceinline__ int row_segments(const Raster& r, int seg_log) {
+    const int d1 = r.axis == 0 ? 1 : 0;
+    return ((r.hi[d1] - r.lo[d1]) >> seg_log) + 1;
+}
+
+// Segments of each triangle's box.
+__global__ void __launch_bounds__(kB) columns_k(const float4* __restrict__ tri, int nF, int R, float band, int seg_log,
+                                                long long* __restrict__ segs) {
     const int f = blockIdx.x * blockDim.x + threadIdx.x;
     if (f > nF) return;
     if (f == nF) {
-        rows[nF] = 0;
+        segs[nF] = 0;
         return;
     }
     const Raster r = raster_of(tri_corner(tri, f, 0), tri_corner(tri, f, 1), tri_corner(tri, f, 2), R, band);
     const int d2 = r.axis == 2 ? 1 : 2;
     bool any = true;
     for (int d = 0; d < 3; ++d) any = any && r.hi[d] >= r.lo[d];
-    rows[f] = any ? r.hi[d2] - r.lo[d2] + 1 : 0;
+    segs[f] = any ? (long long)(r.hi[d2] - r.lo[d2] + 1) * row_segments(r, seg_log) : 0;
 }
 
 // Exclusive scan of 64-bit column counts in one workgroup per 2048 items
@@ -333,18 +340,29 @@ __global__ void __launch_bounds__(kB) scan64_add_k(long long* __restrict__ v, lo
     if (i < n) v[i] += offs[i / 2048];
 }
 
-// One work item per row of columns: the samples of each column within the band
-// of the triangle's plane, each given min(current, distance) (the distance's
+// One work item per segment of a row: the samples of each column within the
+// band of the triangle's plane, each given min(current, distance) (the distance's
 // bits order like the non-negative floats they encode).
-// A block finds its first and last row's triangles in `off` and the rows
+// A block finds its first and last item's triangles in `off` and the items
 // between search the offsets between, brought to LDS (in `off` where there are
-// more than kUdfRange, as triangles without rows can make it).  Bound by its
+// more than kUdfRange, as triangles without items can make it).  Bound by its
 // instructions: a column an item, each with its own search, box, plane and
 // region setup, took 1.16 ms on 370k faces at R = 256, a row an item 0.88.
+//
+// Segments: small triangles' rows have some ten columns, and a dense mesh has
+// items enough, so a row is one item (16 columns hold it); the rows of a few
+// large triangles have up to R columns and are too few for the chip.  Remeshing
+// in ms with 2 | 4 | 8 | 16 columns | whole rows: a cube (12 faces) at R = 64
+// .32 | .34 | .35 | .39 | .64, at R = 256 .92 | .93 | .95 | .98 | 2.28; a sphere
+// of 5120 faces at R = 256 .78 | .81 | .83 | .87 | .87; a union of 19k faces at
+// R = 64 .37 | .35 | .36 | .36 | .36, of 366k faces at R = 256 2.00 | 1.81 |
+// 1.75 | 1.74 | 1.75.
 constexpr int kUdfRange = 512;
+constexpr int kFewFaces = 16384;
+static int segment_log(int n_tris) { return n_tris <= kFewFaces ? 1 : 4; }
 
 __device__ __forceinline__ int udf_find(const long long* __restrict__ off, int lo, int hi, long long w) {
-    while (lo < hi) {  // the last triangle whose rows start at or before w
+    while (lo < hi) {  // the last triangle whose items start at or before w
         const int mid = (lo + hi + 1) >> 1;
         if (off[mid] <= w) lo = mid;
         else hi = mid - 1;
@@ -353,7 +371,8 @@ __device__ __forceinline__ int udf_find(const long long* __restrict__ off, int l
 }
 
 __global__ void __launch_bounds__(kB) udf_k(const float4* __restrict__ tri, int nF, const long long* __restrict__ off,
-                                            long long total, int R, float band, unsigned* __restrict__ grid) {
+                                            long long total, int R, float band, int seg_log,
+                                            unsigned* __restrict__ grid) {
     __shared__ long long loff[kUdfRange];
     __shared__ int ends[2];
     const long long w0 = (long long)blockIdx.x * kB, w = w0 + threadIdx.x;
@@ -369,7 +388,8 @@ __global__ void __launch_bounds__(kB) udf_k(const float4* __restrict__ tri, int 
     const V3 a = tri_corner(tri, f, 0), b = tri_corner(tri, f, 1), c = tri_corner(tri, f, 2);
     const Raster r = raster_of(a, b, c, R, band);
     const int ax = r.axis, d1 = ax == 0 ? 1 : 0, d2 = ax == 2 ? 1 : 2;
-    const int i2 = r.lo[d2] + (int)(w - off[f]);
+    const int ns = row_segments(r, seg_log), k = (int)(w - off[f]), i2 = r.lo[d2] + k / ns;
+    const int s0 = r.lo[d1] + ((k % ns) << seg_log), s1 = min(r.hi[d1], s0 + (1 << seg_log) - 1);
     const float inv = 1.0f / (float)R, x2 = ((float)i2 + 0.5f) * inv;
     // the triangle lies in the ball (mid, rad): a sample farther from mid than
     // rad plus the distance that its cell already holds (or the band) cannot
@@ -381,8 +401,8 @@ __global__ void __launch_bounds__(kB) udf_k(const float4* __restrict__ tri, int 
     const float e2 = x2 - comp(mid, d2), reach = band + rad, row2 = reach * reach - e2 * e2;
     if (row2 < 0.0f) return;
     const float half1 = sqrtf(row2) + slack, m1 = comp(mid, d1);
-    const int c0 = max(r.lo[d1], (int)ceilf((m1 - half1) * (float)R - 0.5f));
-    const int c1 = min(r.hi[d1], (int)floorf((m1 + half1) * (float)R - 0.5f));
+    const int c0 = max(s0, (int)ceilf((m1 - half1) * (float)R - 0.5f));
+    const int c1 = min(s1, (int)floorf((m1 + half1) * (float)R - 0.5f));
     const V3 n = s3::cross(b - a, c - a);
     const float na = comp(n, ax), nl = s3::len(n);
     const bool plane = fabsf(na) > 1e-30f && nl > 0.0f;
@@ -806,8 +826,9 @@ static int remesh(Ctx& c, const float* d_pts, const int* d_tris, int n_tris, con
     hipLaunchKernelGGL(fill_val_k<unsigned>, dim3(grid_for(ng, kB)), dim3(kB), 0, st, c.grid, 0x7F800000u, ng);
     PAMO_HIP(hipGetLastError());
     PAMO_TRY(ensure(&c.cols, c.cap_cols, (size_t)n_tris + 1, st));
+    const int seg_log = segment_log(n_tris);
     hipLaunchKernelGGL(columns_k, dim3(grid_for(n_tris + 1, kB)), dim3(kB), 0, st, (const float4*)c.tri, n_tris, R,
-                       c.band, c.cols);
+                       c.band, seg_log, c.cols);
     PAMO_HIP(hipGetLastError());
     const long long nc = n_tris + 1, ntile = (nc + 2047) / 2048;
     PAMO_TRY(ensure(&c.sums, c.cap_sums, (size_t)ntile, st));
@@ -827,7 +848,7 @@ static int remesh(Ctx& c, const float* d_pts, const int* d_tris, int n_tris, con
     PAMO_HIP(hipGetLastError());
     if (total > 0)
         hipLaunchKernelGGL(udf_k, dim3(grid_for(total, kB)), dim3(kB), 0, st, (const float4*)c.tri, n_tris,
-                           (const long long*)c.cols, total, R, c.band, c.grid);
+                           (const long long*)c.cols, total, R, c.band, seg_log, c.grid);
     PAMO_HIP(hipGetLastError());
     // sign: flood fill of the outside from the border
     const float wall = 0.55f / (float)R;

@@ -60,3 +60,53 @@ def test_smaller_grid_after_a_larger_one():
     v, f = used.remesh(Vd, Fd, mean, 20)
     v0, f0 = t1._remesher().remesh(Vd, Fd, mean, 20)
     assert torch.equal(v, v0) and torch.equal(f, f0)
+
+
+def _cube():
+    V = t1._box_tris((0.0, 0.0, 0.0), (1.0, 1.0, 1.0)).reshape(-1, 3).astype(np.float32)
+    return V, np.arange(36, dtype=np.int32).reshape(-1, 3)
+
+
+def _turned_cube():
+    V, F = _cube()
+    q, _ = np.linalg.qr(np.random.default_rng(1).standard_normal((3, 3)))
+    return (V @ q).astype(np.float32), F
+
+
+@pytest.mark.parametrize("times,R", [(1, 33), (1, 70), (1400, 70)])
+def test_field_of_large_triangles(times, R):
+    """Triangles whose rows have up to R columns, more than a work item takes
+    (rows of every remainder among them), against the oracle's field; the same
+    faces many times over take the dense meshes' longer segments."""
+    from oracle import stage1 as o
+    V, F = _turned_cube()
+    print(f"case: field of {len(F)} large triangles, {times} times, R {R}", flush=True)
+    r = t1._remesher()
+    r.remesh(*t1._dev(V, np.tile(F, (times, 1))), t1._mean(V, F), R)
+    tris = r.debug(_hip.PAMO_S1_DBG_NORMALIZED, np.float32, 12 * len(F) * times).reshape(-1, 3, 4)[:len(F), :, :3]
+    field = r.debug(_hip.PAMO_S1_DBG_FIELD, np.uint32, R ** 3).view(np.float32).reshape(R, R, R)
+    ref = o.udf(tris, R, 3.0 / R)
+    assert np.array_equal(np.isfinite(field), np.isfinite(ref))
+    fin = np.isfinite(ref)
+    assert np.abs(field[fin] - ref[fin]).max() <= 2e-7
+
+
+def test_few_large_triangles_spread_over_the_chip():
+    """12 triangles across the grid are no more work than 5120 small ones on a
+    surface of that size (their samples are the same): the call takes no
+    longer, with room for noise (2.5 times as long with a row of columns a
+    lane, 0.7 with a column a lane)."""
+    import time
+    print("case: remesh 12 and 5120 triangles, R 128", flush=True)
+    r = t1._remesher()
+    meshes = [t1._dev(*m) for m in (_cube(), synth.icosphere_sh(4, 3))]
+    times = [[], []]
+    for _ in range(25):
+        for k, (V, F) in enumerate(meshes):
+            t = time.perf_counter()
+            r.remesh(V, F, (0.0, 0.0, 0.0), 128)
+            torch.cuda.synchronize()
+            times[k].append(time.perf_counter() - t)
+    few, many = (float(np.median(t[5:])) for t in times)
+    print(f"few {few * 1e3:.3f} ms, many {many * 1e3:.3f} ms", flush=True)
+    assert few < 1.7 * many, (few, many)
