@@ -576,8 +576,12 @@ __global__ void __launch_bounds__(kB) cross_bits_k(const unsigned* __restrict__ 
 // The crossing vertices, direction by direction in sample order: a scan over
 // the words' counts; the vertices of a word by linear interpolation, in
 // sample index units.  wpos[k] (k <= 3 words): vertices before word k.
+// A lane writes its words' vertices one by one, up to 64 a word where a flat
+// face lies along the grid: two words a lane (a cube at R = 64 0.32 -> 0.275 ms
+// a call, at R = 256 0.92 -> 0.78, against four; a union of 366k faces at R = 256
+// 1.76 either way; one word: 0.30, 0.73 and 1.76, but at R = 512 3 % slower).
 struct CrossVertsOp {
-    static constexpr int kIpt = 4;
+    static constexpr int kIpt = 2;
     const uint64_t* cross;
     const unsigned* grid;
     const uint8_t* out;
