@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from oracle import metrics as om
-from pamo_amd import _hip, metrics, synth
+from pamo_amd import _hip, metrics, stage3, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -44,7 +44,9 @@ def test_smallest_trees(faces):
 
 def test_tree_deeper_than_the_stack():
     """30 places whose Morton codes differ bit by bit, 64 equal triangles at
-    each: from near the origin a walk passes 36 levels before its first face."""
+    each: from near the origin a walk passes 36 levels before its first face, so a
+    lane meets none within its steps and leaves the query to a wave, whose stack
+    holds it (the walks that run out of stack: below)."""
     print("case: deep tree", flush=True)
     at = [np.eye(3)[d] * 2.0 ** -k for k in range(10) for d in range(3)]
     tri = np.array([[0, 0, 0], [1e-5, 0, 0], [0, 1e-5, 0]])
@@ -116,3 +118,92 @@ def test_buffers_of_a_large_call_are_bounded():
     for a, b in ((0, 5000), (cut - 3000, cut + 3000), (2 * cut - 70000, 2 * cut + 70000), (n - 100, n)):
         part, _ = call(P[a:b].contiguous())
         assert all(torch.equal(w[a:b], p) for w, p in zip(whole, part))
+
+
+def _deep_mesh():
+    """The mesh of test_tree_deeper_than_the_stack, and points near its
+    origin: the way down to their first face leaves 30 places behind, all of
+    them still to visit, on a stack of 24."""
+    at = [np.eye(3)[d] * 2.0 ** -k for k in range(10) for d in range(3)]
+    tri = np.array([[0, 0, 0], [1e-5, 0, 0], [0, 1e-5, 0]])
+    V = np.concatenate([a + tri for a in at for _ in range(64)])
+    P = 1e-4 * np.random.default_rng(1).standard_normal((100, 3))
+    return P, V, np.arange(len(V), dtype=np.int32).reshape(-1, 3)
+
+
+def test_lane_finishes_by_links_when_its_stack_ran_out():
+    """The allocation-free form has no buffer for leftover queries, so every
+    lane finishes its own: here with nodes that found no place on its stack."""
+    print("case: deep tree, no leftovers", flush=True)
+    P, V, F = _deep_mesh()
+    Pd, Vd, Fd = (torch.from_numpy(a).cuda() for a in (P, V, F))
+    sq = torch.empty(len(P), dtype=torch.float64, device="cuda")
+    idx = torch.empty(len(P), dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    _hip.check(_hip.lib().pamo_point_mesh_sqdist_noalloc(Pd.data_ptr(), len(P), Vd.data_ptr(), len(V), Fd.data_ptr(),
+                                                         len(F), sq.data_ptr(), idx.data_ptr(), None,
+                                                         torch.cuda.current_stream().cuda_stream), "noalloc")
+    torch.cuda.synchronize()
+    so, io = om.point_mesh_sqdist(P, V, F)
+    assert np.all(np.abs(sq.cpu().numpy() - so) <= 1e-12 * so)
+    assert np.array_equal(idx.cpu().numpy(), io)  # the places' 64 equal triangles: the smallest number
+
+
+def test_stage3_targets_when_the_stack_ran_out():
+    """Stage 3's closest points over the same tree (its lanes have the same
+    stack and no second kernel)."""
+    print("case: deep tree as a stage-3 target", flush=True)
+    _, gV, gF = _deep_mesh()
+    V, F = synth.icosphere(1)
+    V = (V * 1e-4).astype(np.float32)
+    s = stage3.Stage3System()
+    s.register_mesh(gV.astype(np.float32), gF, V, F)
+    got = s.debug(_hip.PAMO_S3_DBG_TARGET).reshape(-1, 3)
+    P = V.astype(np.float64)
+    so, _ = om.point_mesh_sqdist(P, gV.astype(np.float32).astype(np.float64), gF)
+    # 32-bit coordinates below 1: a distance's error is below 1e-6
+    assert np.abs(np.sqrt(((got - P) ** 2).sum(1)) - np.sqrt(so)).max() < 1e-6
+    on, _ = om.point_mesh_sqdist(got, gV.astype(np.float32).astype(np.float64), gF)
+    assert np.sqrt(on).max() < 1e-6
+
+
+def _expand(v):
+    out = np.zeros_like(v)
+    for b in range(10):
+        out |= ((v >> b) & 1) << (3 * b)
+    return out
+
+
+def test_wave_walk_beyond_its_stack(oracle_lib):
+    """64 cells, each with a chain of 24 places that split off one by one from
+    the corner where most triangles are: a wave's walk goes down all chains at
+    once (the right children, last pushed) and leaves 64 nodes behind a step, more
+    than 1024 before its first face; a lane meets no face within its 32 steps,
+    so nothing is pruned."""
+    print("case: wide frontier", flush=True)
+    cells = np.stack(np.meshgrid(*[np.arange(4)] * 3, indexing="ij"), -1).reshape(-1, 3) * 256
+    ones = np.array([255, 255, 255])
+    places = [ones - np.eye(3, dtype=int)[d] * (1 << b) for b in range(8) for d in range(3)]
+    at = np.concatenate([np.repeat([c + p for p in places], 2, 0) for c in cells] +
+                        [np.repeat([c + ones], 64, 0) for c in cells] + [[[0, 0, 0]]])
+    centre = at / 1023.0  # place x of 1024 along an axis of the whole box, which is the unit cube
+    tri = np.array([[1, 0, 0], [-1, 0, 0], [0, 0, 0]]) * 1e-6
+    V = (centre[:, None] + tri).reshape(-1, 3)
+    F = np.arange(len(V), dtype=np.int32).reshape(-1, 3)
+    # the frontier, over the same hierarchy
+    code = (_expand(at[:, 0]) * 4 + _expand(at[:, 1]) * 2 + _expand(at[:, 2])).astype(np.uint32)
+    by = np.argsort(code, kind="stable")
+    left, right = oracle_lib.karras(code[by], by.astype(np.int32))
+    inner, stack, faces = len(F) - 1, [0], False
+    while not faces:
+        top, stack = stack[-64:], stack[:-64]
+        kids = [left[x] for x in top] + [right[x] for x in top]
+        faces = any(k >= inner for k in kids)
+        stack += [k for k in kids if k < inner]
+    assert len(stack) > 1024, len(stack)
+    depth, x = 0, 0  # a lane's way down to the corner that is nearest to (2, 2, 2)
+    while x < inner:
+        x, depth = right[x], depth + 1
+    assert depth > 32, depth
+    P = 2.0 + 1e-3 * np.random.default_rng(2).standard_normal((40, 3))
+    _check(P, V, F)
