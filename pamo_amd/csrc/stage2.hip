@@ -646,12 +646,13 @@ static int pasp_round_device(Ctx& c, int nP, int nT, float scale, float thr) {
            c.eord_cnt, (unsigned long long*)c.vmin, (uint8_t*)nullptr);
     PAMO_TRY(topology_and_quadrics(c, m, nP, nT));
     const int nE = c.edge_bound;  // launches cover this bound
+    const double mE = 1.5 * nT;   // the bytes of their models: a closed mesh's edges
     const int* cnt = c.dcnt;
-    LAUNCHP(K_EDGE_COST, 12.0 * nE + 4.0 * nP + 48.0 * nT + 16.0 * nP + 48.0 * nP + 4.0 * nE, pasp_cost_k, nE, m,
+    LAUNCHP(K_EDGE_COST, 12.0 * mE + 4.0 * nP + 48.0 * nT + 16.0 * nP + 48.0 * nP + 4.0 * mE, pasp_cost_k, nE, m,
             c.ring_off, c.rv, c.eu, c.ev, c.eord, cnt, c.Q, scale, thr, c.edge_cost);
-    LAUNCHP(K_PROPAGATE, 12.0 * nE + 16.0 * nP, propagate_k, nE, c.eu, c.ev, cnt, c.edge_cost,
+    LAUNCHP(K_PROPAGATE, 12.0 * mE + 16.0 * nP, propagate_k, nE, c.eu, c.ev, cnt, c.edge_cost,
             (unsigned long long*)c.vmin);
-    LAUNCHP(K_SELECT_COLLAPSE, 16.0 * nE + 4.0 * nP + 48.0 * nT + 8.0 * nP, pasp_collapse_k, nE, m, c.occ,
+    LAUNCHP(K_SELECT_COLLAPSE, 16.0 * mE + 4.0 * nP + 48.0 * nT + 8.0 * nP, pasp_collapse_k, nE, m, c.occ,
             c.ring_off, c.ring, (const int4*)c.rv, c.eu, c.ev, cnt, c.edge_cost, (const unsigned long long*)c.vmin,
             collapse_t);
     PAMO_TRY(scan_exclusive_lb(c.occ, c.pts_map, nP + 1, c.lb, c.stream));
@@ -669,10 +670,11 @@ static int round_device(Ctx& c, int nP, int nT, float scale, float thr, bool is_
            c.eord_cnt, (unsigned long long*)c.vmin, c.changed);
     PAMO_TRY(topology_and_quadrics(c, m, nP, nT));
     const int nE = c.edge_bound;  // launches cover this bound
+    const double mE = 1.5 * nT;   // the bytes of their models: a closed mesh's edges
     const int* cnt = c.dcnt;
     CostParams cp{edge_s, tres, is_stuck ? 1 : 0, c.inv_epoch};
     // (+ 16 B per vertex: the minimum keys the fused propagation lowers)
-    const double cost_bytes = 12.0 * nE + 4.0 * nP + 48.0 * nT + 16.0 * nP + 48.0 * nP + 1.0 * nP + 4.0 * nE + 16.0 * nP;
+    const double cost_bytes = 12.0 * mE + 4.0 * nP + 48.0 * nT + 16.0 * nP + 48.0 * nP + 1.0 * nP + 4.0 * mE + 16.0 * nP;
 #define PAMO_EDGE_COST(K, lanes)                                                                              \
     LAUNCHP(K_EDGE_COST, cost_bytes, K, (long long)nE * (lanes), m, c.ring_off, c.rv, c.eu, c.ev, c.eord, cnt,    \
             c.invalid, c.Q, cp, c.edge_cost, (unsigned long long*)c.vmin)
@@ -689,7 +691,7 @@ static int round_device(Ctx& c, int nP, int nT, float scale, float thr, bool is_
 #undef PAMO_EDGE_COST
     // independent set + collapse (the cost kernels have lowered the
     // per-vertex minimum keys)
-    const double sel_bytes = 16.0 * nE + 4.0 * nP + 48.0 * nT + 8.0 * nP;
+    const double sel_bytes = 16.0 * mE + 4.0 * nP + 48.0 * nT + 8.0 * nP;
 #define PAMO_SELECT(K, lanes)                                                                                 \
     LAUNCHP(K_SELECT_COLLAPSE, sel_bytes, K, (long long)nE * (lanes), m, orig_mesh(c), c.occ, c.ring_off,         \
             c.ring, (const int4*)c.rv, c.eu, c.ev, cnt, c.edge_cost, (const unsigned long long*)c.vmin, collapse_t,  \
@@ -708,7 +710,7 @@ static int round_device(Ctx& c, int nP, int nT, float scale, float thr, bool is_
     // the records, and the cleanup with the line collapses, in one launch
     PAMO_TRY(scan_pair(CollapseListOp{c.esel, c.recs, c.dcnt}, nE, CleanupOp{m, c.eu, c.ev, nT, c.lines, c.dcnt},
                        (long long)std::max(nE, nT), c.lb, c.stream, K_LINE_FLAG,
-                       8.0 * nE + 16.0 * nP + 4.0 * nE + 12.0 * nT));
+                       8.0 * mE + 16.0 * nP + 4.0 * mE + 12.0 * nT));
     hipLaunchKernelGGL(line_apply_k, dim3(1), dim3(1), 0, c.stream, m, c.occ, c.ring_off, c.ring, c.eu, c.ev,
                        (const int*)c.lines, c.dcnt, c.changed);
     PAMO_HIP(hipGetLastError());

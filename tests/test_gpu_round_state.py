@@ -71,3 +71,28 @@ def test_records_of_a_one_leaf_tree(threshold):
     else:
         assert np.array_equal(box[:3], at.min(0)) and np.array_equal(box[4:7], at.max(0))
     assert box.view(np.int32)[[3, 7]].tolist() == [0, -1]
+
+
+def test_byte_models_count_a_closed_meshs_edges():
+    """The launch profiler's bytes: launches over the edges cover a bound (two
+    a face), their compulsory traffic is that of the edges (1.5 a face)."""
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from pamo_amd import _hip, synth
+    from pamo_amd.pamo import CUDSP_Free
+    V, F = synth.icosphere_sh(3, 3)
+    V = centred(V, F)
+    print(f"case: byte models, {len(F)} faces", flush=True)
+    op = CUDSP_Free(0)
+    prof = _hip.Profiler(op.ctx)
+    prof.enable()
+    op.forward(torch.from_numpy(V).cuda(), torch.from_numpy(F).cuda(), torch.zeros(0, dtype=torch.int32, device="cuda"),
+               0, float((V.max(0) - V.min(0)).max()), 1e-3, 0, True)
+    by = {s["name"]: s["bytes"] for s in prof.stats()}
+    nP, nT = len(V), len(F)
+    nE = op.debug(_hip.PAMO_DBG_EDGES).numel() // 2
+    assert nE == 1.5 * nT
+    assert by["edge_cost"] == 16 * nE + 85 * nP + 48 * nT
+    assert by["select_collapse"] == 16 * nE + 12 * nP + 48 * nT
+    assert by["line_flag"] == 12 * nE + 16 * nP + 12 * nT
