@@ -95,6 +95,12 @@ int pamo_ctx_set_stream(pamo_ctx* ctx, void* stream, int own);
  * selection-and-collapse and undo kernels, or 4 / 8 (default) lanes
  * splitting the one-ring faces (float sums kept in the single-lane order). */
 #define PAMO_OPT_RING_LANES 10
+/* Microseconds (0 to 1000000, default 200) for which a host thread looks for
+ * the counters a round publishes before it waits on the stream (no
+ * counterpart in the reference; results do not change).  Looking holds a
+ * core: the batched and served forms set 0 when they run more slots than
+ * there are cores. */
+#define PAMO_OPT_COUNTER_POLL 11
 int pamo_ctx_set_option(pamo_ctx* ctx, int option, long long value);
 
 /* Last error message of the calling thread ("" if none).

@@ -286,8 +286,12 @@ static int create(Engine** out, int device, int n_slots, long long budget, const
         destroy(e);
         PAMO_CHECK(false, "pamo serve/batch: stream creation failed");
     }
+    // a worker that looks for its counters holds a core (0: the cores are unknown)
+    const unsigned cores = std::thread::hardware_concurrency();
+    const bool crowded = cores > 0 && (unsigned)n_slots > cores;
     for (Slot& s : e->slots) {
         int rc = pamo_ctx_create(&s.c2, device);
+        if (rc == 0 && crowded) rc = pamo_ctx_set_option(s.c2, PAMO_OPT_COUNTER_POLL, 0);
         if (rc == 0 && exact_guard) rc = pamo_ctx_set_option(s.c2, PAMO_OPT_EXACT_GUARD, exact_guard);
         if (rc == 0 && e->has_s3) rc = pamo_s3_create(&s.c3, device, &e->s3p);
         if (rc == 0 && hipStreamCreateWithFlags(&s.st, hipStreamNonBlocking) != hipSuccess) rc = 1;

@@ -142,6 +142,7 @@ struct Ctx {
     int hcnt[C_COUNT] = {};              // the counters as last read
     unsigned long long* pub = nullptr;  // pinned, where publish_k writes them
     unsigned pub_seq = 0;
+    int poll_us = 200;  // how long sync_counters looks before it waits
     // last round, host view
     int edge_bound = 0;  // edges that the round's launches cover
     int n_pts = 0, n_tris = 0, n_edges = 0, n_rec = 0, n_regular = 0, n_vertices_undo = 0;
@@ -403,9 +404,13 @@ static Orig orig_mesh(Ctx& c) { return Orig{c.op, c.oi, c.oj, c.ok}; }
 // A copy and a wait on the stream take some 20 us beside the work they wait
 // for, two or more times a round.  A one-wave kernel writes the counters to
 // pinned memory instead, and the host looks for this read's number for up to
-// kPollUs, after which (a long round, or an error) it waits on the stream
+// poll_us, after which (a long round, or an error) it waits on the stream
 // (1280 faces 4.6 -> 3.9 ms a run, 90k faces 43.4 -> 40; 40 us: 4.3 and 42.3).
-constexpr int kPollUs = 200;
+// Looking holds a core, so that it pays only where every waiting thread has
+// one: 96 meshes of 5k and 20k faces on 4 | 8 | 16 | 32 | 64 slots and 16 cores
+// took 256 | 278 | 324 | 733 | 1064 ms, with the wait at once 283 | 296 | 348 |
+// 723 | 936; 32 meshes of 60k with stage 3 on 32 slots 2464 and 2178 (the engine
+// sets poll_us to 0 for more slots than cores).
 static int sync_counters(Ctx& c) {
     const unsigned seq = ++c.pub_seq;
     hipLaunchKernelGGL(publish_k, dim3(1), dim3(kWave), 0, c.stream, (const int*)c.dcnt, c.pub, seq);
@@ -421,7 +426,7 @@ static int sync_counters(Ctx& c) {
         return true;
     };
     while (!read()) {
-        if (std::chrono::steady_clock::now() - t0 >= std::chrono::microseconds(kPollUs)) {
+        if (std::chrono::steady_clock::now() - t0 >= std::chrono::microseconds(c.poll_us)) {
             PAMO_HIP(hipStreamSynchronize(c.stream));
             PAMO_CHECK(read(), "counters not written by a finished stream");
             break;
@@ -956,6 +961,11 @@ int pamo_ctx_set_option(pamo_ctx* ctx, int option, long long value) {
     if (option == PAMO_OPT_WALK_LIMIT) {
         PAMO_CHECK(value >= 0, "pamo_ctx_set_option: walk limit must be >= 0");
         c.walk_cap = value;
+        return 0;
+    }
+    if (option == PAMO_OPT_COUNTER_POLL) {
+        PAMO_CHECK(value >= 0 && value <= 1000000, "pamo_ctx_set_option: counter poll must be in [0, 1000000] us");
+        c.poll_us = (int)value;
         return 0;
     }
     PAMO_CHECK(option == PAMO_OPT_EXACT_GUARD, "pamo_ctx_set_option: unknown option");

@@ -124,3 +124,34 @@ def test_many_slots_first_allocations_concurrent():
     out, secs = simplify_batch(meshes, ratios, stage3, n_slots=6)
     for (V, F), r, s3, got in zip(meshes, ratios, stage3, out):
         _same(got, _alone(V, F, r, s3), V, s3)
+
+
+@pytest.mark.parametrize("us", [0, 1, 1000000])
+def test_counter_poll_changes_no_result(us):
+    """The wait for a round's counters: at once on the stream, after a look, and
+    by looking alone; refused outside its range."""
+    print(f"case: counter poll {us} us", flush=True)
+    V, F = synth.icosphere_sh(4, 3)
+    V = V - V[F].mean(axis=1).mean(axis=0)
+    Vd, Fd = torch.from_numpy(V).cuda(), torch.from_numpy(F).cuda()
+    want = simplify_device(_hip.Context(0), Vd, Fd, 0.1, min_verts=0)
+    ctx = _hip.Context(0)
+    _hip.check(_hip.lib().pamo_ctx_set_option(ctx.ptr, _hip.PAMO_OPT_COUNTER_POLL, us), "set_option")
+    got = simplify_device(ctx, Vd, Fd, 0.1, min_verts=0)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]) and np.array_equal(got[2], want[2])
+    for bad in (-1, 1000001):
+        with pytest.raises(_hip.PamoError):
+            _hip.check(_hip.lib().pamo_ctx_set_option(ctx.ptr, _hip.PAMO_OPT_COUNTER_POLL, bad), "set_option")
+
+
+def test_more_slots_than_cores():
+    """The engine's workers then wait on their streams at once; each mesh's
+    result is its own, as with few slots."""
+    import os
+    n = min(64, (os.cpu_count() or 1) + 1)
+    print(f"case: {n} slots", flush=True)
+    meshes = [synth.icosphere_sh(3, i) for i in range(n)]
+    many, _ = simplify_batch(meshes, 0.1, n_slots=n)
+    few, _ = simplify_batch(meshes, 0.1, n_slots=1)
+    for (va, fa), (vb, fb) in zip(many, few):
+        assert np.array_equal(va.view(np.uint32), vb.view(np.uint32)) and np.array_equal(fa, fb)
