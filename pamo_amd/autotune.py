@@ -10,7 +10,7 @@ faces and vertices, bit for bit):
 - PAMO_OPT_GUARD_SPLIT_FACES / PAMO_OPT_GUARD_SPLIT_LOG: below this face count
   each group of guard queries is spread over 2^log waves, one per subtree.
 - PAMO_OPT_GUARD_WAVES: without effect since the guard kernel has one variant
-  (4 waves per SIMD); still accepted in settings.
+  (4 waves per SIMD); still accepted in settings, no longer timed.
 - PAMO_OPT_EDGE_LANES: 1, 4 or 8 lanes per edge in the edge-cost kernel.
 - PAMO_OPT_RING_LANES: 1, 4 or 8 lanes per item in the quadric, selection
   and undo kernels.
@@ -37,7 +37,6 @@ CANDIDATES = {
     "tree_keep": [50, 65, 80, 90, 100],
     "guard_split_faces": [1 << 16, 1 << 18, 1 << 20],
     "guard_split_log": [2, 3, 4],
-    "guard_waves": [4],
     "edge_lanes": [1, 4, 8],
     "ring_lanes": [1, 4, 8],
 }

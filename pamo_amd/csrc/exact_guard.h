@@ -372,10 +372,11 @@ __device__ bool x_faces_intersect(const int* ia, const XP3* pa, const int* ib, c
 // at run time: kApart or kMeet, or kUnsure for x_faces_intersect.  Orientations
 // change sign with every exchange of two points, which the signs below use.
 // Most candidates share a vertex or an edge and end here after one to five
-// determinants, in 104 registers and no scratch memory; with the whole decision
-// in the query kernel it took 248 registers and 208 B of scratch a lane.  A run
-// on 200k faces with slivers: 118 us a query launch (336 before), 42 us for
-// the open pairs (115 before, with expansions in scratch memory).
+// determinants, in a query kernel of 84 registers and no scratch memory; with
+// the whole decision in that kernel it took 248 registers and 208 B of scratch a
+// lane.  A run on 200k faces with slivers: 118 us a query launch (336 before), 42
+// us for the open pairs (115 before, with every expansion in scratch memory;
+// now those of o3_raw and o2_raw alone are).
 enum { kApart = 0, kMeet = 1, kUnsure = 2 };
 
 __device__ __forceinline__ int x_o3(const XP3& a, const XP3& b, const XP3& c, const XP3& d) {

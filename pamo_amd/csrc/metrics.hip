@@ -126,8 +126,8 @@ __global__ void __launch_bounds__(kB) point_keys_k(const double* __restrict__ P,
 constexpr int kWaveStack = 1024;  // nodes waiting in a wave's walk of one query (8 KiB)
 
 // Steps after which a lane leaves its query to a whole wave.  Up to
-// kWavePoints queries a wave each fits the chip at once (256 compute units of
-// 20 such waves and more), so a lane only finds a first bound (32 steps: about
+// kWavePoints queries take a wave each in a few turns of the chip (some 5000
+// such waves are resident), so a lane only finds a first bound (32 steps: about
 // the depth of the tree, twice); beyond that the lanes finish the ordinary
 // queries by themselves (128 steps) and leave the long ones.  Measured on
 // surface samples against a 200k-face union (ms a call, tree build included),

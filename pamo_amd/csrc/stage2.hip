@@ -164,7 +164,6 @@ struct Ctx {
     // each query group with 2^guard_split_log waves, one per subtree
     int guard_split_faces = 1 << 16;
     int guard_split_log = 3;
-    int guard_waves = 4;        // accepted, no effect: the guard's own registers allow 4 waves per SIMD
     int edge_lanes = 4;         // lanes per edge in the edge-cost kernel (1, 4 or 8)
     int ring_lanes = 8;         // lanes per item in the quadric, selection and undo kernels (1, 4 or 8)
     float* cent_out = nullptr;  // pamo_centroid's result (3 floats)
@@ -945,8 +944,7 @@ int pamo_ctx_set_option(pamo_ctx* ctx, int option, long long value) {
     }
     if (option == PAMO_OPT_GUARD_WAVES) {
         PAMO_CHECK(value == 0 || value == 4, "pamo_ctx_set_option: guard waves must be 0 (compiler's choice) or 4");
-        c.guard_waves = (int)value;
-        return 0;
+        return 0;  // the guard kernel has one variant
     }
     if (option == PAMO_OPT_TREE_KEEP) {
         PAMO_CHECK(value >= 1 && value <= 100, "pamo_ctx_set_option: tree keep percentage must be in [1, 100]");

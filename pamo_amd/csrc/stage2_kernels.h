@@ -1333,11 +1333,12 @@ __global__ void karras_k(const uint32_t* __restrict__ key, const uint32_t* __res
 // LDS: level k holds the union of entries [t, t + 2^k), so any range of the
 // block is the union of two table entries (min / max are exact and
 // idempotent, so overlapping halves give the same box).  One launch writes
-// the sorted leaf boxes (level 0: node n-1+s of `node`, lo.w = item id,
-// hi.w left as it is), the in-block prefix and suffix boxes, each block's
-// box, and (given `range`) the box of every internal node whose leaf range
-// lies inside the block: internal node i covers [i, j] or [j, i], so those
-// nodes are exactly the ones numbered inside the block.  Level 1 runs the
+// the sorted leaves' boxes into their parents' pairs (level 0: leaf s at
+// slot[n-1+s], lo.w = ~item, hi.w left as it is), the in-block prefix and
+// suffix boxes, each block's box, and (given `range`) the box of every
+// internal node but the root whose leaf range lies inside the block, at the
+// node's slot: internal node i covers [i, j] or [j, i], so those nodes are
+// exactly the ones numbered inside the block.  Level 1 runs the
 // same kernel over the block boxes and also stores its table (`tab`, level
 // k at tab + 2 k stride) for the nodes that span blocks.
 constexpr int kTabLevels = 8;  // 2^0 .. 2^7 entries
@@ -1668,11 +1669,12 @@ constexpr int kQueue = 192;   // per-wave pair queue (< 64 pending + one append 
 constexpr int kGuardQ = 8;    // guard queries per wave
 // A launch covers a group of kGuardQ queries for every kGuardQ faces; where
 // few faces are queries, the idle waves take finer subtrees: the split is
-// doubled while all waves at work stay within kSplitWaves (half of the 16384
-// that can be resident), to at most 2^kMaxSplit subtrees.  A face that is long
-// and thin overlaps thousands of boxes, and such faces come in groups: 200k
-// faces with the exact guard 148 -> 122 ms a run, from 2M to 20k faces 304.5 ->
-// 301 (16384 waves: 307, to 2^6 subtrees: 133 and 303).
+// doubled while all waves at work stay within kSplitWaves, to at most
+// 2^kMaxSplit subtrees.  A face that is long and thin overlaps thousands of
+// boxes, and such faces come in groups: 200k faces with the exact guard 148 ->
+// 122 ms a run, from 2M to 20k faces 304.5 -> 301.  Both limits as measured
+// (16384 waves: 307, to 2^6 subtrees: 133 and 303); 4096 waves are resident at
+// once, so the 8192 go in two turns of shorter walks.
 constexpr int kMaxSplit = 8, kSplitWaves = 8192;
 // Exact mode: a wave decides its first kInWave batches of 64 pairs, and hands
 // further full batches to exact_pairs_k, which spreads them over the chip
