@@ -352,7 +352,8 @@ __global__ void __launch_bounds__(kB) scan64_add_k(long long* __restrict__ v, lo
 // Segments: small triangles' rows have some ten columns, and a dense mesh has
 // items enough, so a row is one item (16 columns hold it); the rows of a few
 // large triangles have up to R columns and are too few for the chip.  Remeshing
-// in ms with 2 | 4 | 8 | 16 columns | whole rows: a cube (12 faces) at R = 64
+// in ms (with four words of crossings a lane, see CrossVertsOp) with 2 | 4 | 8 |
+// 16 columns | whole rows: a cube (12 faces) at R = 64
 // .32 | .34 | .35 | .39 | .64, at R = 256 .92 | .93 | .95 | .98 | 2.28; a sphere
 // of 5120 faces at R = 256 .78 | .81 | .83 | .87 | .87; a union of 19k faces at
 // R = 64 .37 | .35 | .36 | .36 | .36, of 366k faces at R = 256 2.00 | 1.81 |
@@ -576,12 +577,15 @@ __global__ void __launch_bounds__(kB) cross_bits_k(const unsigned* __restrict__ 
 // The crossing vertices, direction by direction in sample order: a scan over
 // the words' counts; the vertices of a word by linear interpolation, in
 // sample index units.  wpos[k] (k <= 3 words): vertices before word k.
-// A lane writes its words' vertices one by one, up to 64 a word where a flat
-// face lies along the grid: two words a lane (a cube at R = 64 0.32 -> 0.275 ms
-// a call, at R = 256 0.92 -> 0.78, against four; a union of 366k faces at R = 256
-// 1.76 either way; one word: 0.30, 0.73 and 1.76, but at R = 512 3 % slower).
+// A lane writes its words' few vertices one by one; a word of more than kWide,
+// up to 64 where a flat face lies along the grid, is written by its wave, a
+// sample a lane, which reads the samples in whole lines.  Remeshing in ms, with
+// four words a lane and no wave | two and no wave | four and the wave | two and
+// the wave: a cube (12 faces) at R = 64 .32 | .28 | .24 | .24, at R = 128 .41 | .42
+// | .43 | .35, at R = 256 .92 | .78 | .80 | .71 (a lane a grid edge: .26, .42 and
+// 1.35); a union of 366k faces at R = 256 1.76 | 1.76 | 1.74 | 1.72.
 struct CrossVertsOp {
-    static constexpr int kIpt = 2;
+    static constexpr int kIpt = 2, kWide = 12;
     const uint64_t* cross;
     const unsigned* grid;
     const uint8_t* out;
@@ -593,21 +597,34 @@ struct CrossVertsOp {
     long long cap;   // room in verts (a first guess; the launch is repeated when it was too small)
     int* total;
     __device__ int count(long long k) const { return __popcll(cross[k]); }
-    __device__ void emit(long long k, int v, int pos) const {
-        wpos[k] = pos;
-        if (!v) return;
+    // the vertex of sample `bit` of word k, at place p of verts
+    __device__ void put(long long k, int bit, long long p) const {
+        if (p >= cap) return;
         const int dir = (int)(k / words);
         const long long step = dir == 0 ? 1 : (dir == 1 ? R : (long long)R * R);
-        uint64_t m = cross[k];
-        for (int j = 0; m; ++j, m &= m - 1) {
-            if (pos + j >= cap) return;
-            const long long s = (k - dir * words) * 64 + (__ffsll((unsigned long long)m) - 1);
-            const float d0 = sdf_at(grid, out, s), d1 = sdf_at(grid, out, s + step);
-            const float t = (iso - d0) / (d1 - d0);
-            float p[3] = {(float)(s % R), (float)((s / R) % R), (float)(s / ((long long)R * R))};
-            p[dir] += t;
-            verts[pos + j] = make_float4(p[0], p[1], p[2], 0.0f);
+        const long long s = (k - dir * words) * 64 + bit;
+        const float d0 = sdf_at(grid, out, s), d1 = sdf_at(grid, out, s + step);
+        const float t = (iso - d0) / (d1 - d0);
+        float q[3] = {(float)(s % R), (float)((s / R) % R), (float)(s / ((long long)R * R))};
+        q[dir] += t;
+        verts[p] = make_float4(q[0], q[1], q[2], 0.0f);
+    }
+    __device__ void emit(long long k, int v, int pos) const {
+        wpos[k] = pos;
+        uint64_t m = v ? cross[k] : 0;
+        uint64_t wide = __ballot(v > kWide);
+        if (wide && __ballot(true) == ~0ull) {  // (the last tile's last wave may hold fewer lanes)
+            const int lane = threadIdx.x & (kWave - 1);
+            if (v > kWide) m = 0;
+            for (; wide; wide &= wide - 1) {
+                const int src = __ffsll((unsigned long long)wide) - 1;
+                const long long wk = __shfl(k, src);
+                const int at = __shfl(pos, src);
+                const uint64_t w = cross[wk];
+                if ((w >> lane) & 1) put(wk, lane, (long long)at + lanes_below(w));
+            }
         }
+        for (int j = 0; m; ++j, m &= m - 1) put(k, __ffsll((unsigned long long)m) - 1, (long long)pos + j);
     }
     __device__ void done(int n) const { *total = n; }
 };

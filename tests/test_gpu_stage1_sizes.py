@@ -50,6 +50,13 @@ def test_steps_after_the_field(case, R):
     t1._check_closed_manifold(f.cpu().numpy(), len(v))
 
 
+@pytest.mark.parametrize("R", [64, 72, 128])
+def test_faces_along_the_grid(R):
+    """Flat faces along the grid: words whose 64 samples all cross, and (R = 72)
+    words that end inside a row."""
+    test_steps_after_the_field("boxes", R)
+
+
 def test_smaller_grid_after_a_larger_one():
     print("case: remesh R 72 then 20 on one context", flush=True)
     V, F = t1._boxes()
@@ -95,7 +102,7 @@ def test_few_large_triangles_spread_over_the_chip():
     """12 triangles across the grid are no more work than 5120 small ones on a
     surface of that size (their samples are the same): the call takes no
     longer, with room for noise (2.5 times as long with a row of columns a
-    lane, 0.7 with a column a lane)."""
+    lane, 0.7 with a column a lane, 0.9 now)."""
     import time
     print("case: remesh 12 and 5120 triangles, R 128", flush=True)
     r = t1._remesher()
