@@ -38,9 +38,9 @@ int pamo_ctx_reset(pamo_ctx* ctx);
 int pamo_ctx_set_stream(pamo_ctx* ctx, void* stream, int own);
 
 /* Test option (no counterpart in the reference): with value 1 the guard
- * query runs with a 32-entry frontier per wave, so the exact overflow walk
- * of the frontier traversal is exercised; 0 restores the default.  The
- * result is identical either way. */
+ * query runs with a 32-entry frontier per wave, so that it fills and few
+ * entries are popped a step; 0 restores the default.  The result is identical
+ * either way. */
 #define PAMO_OPT_GUARD_SMALL_STACK 1
 /* Guard predicate (no counterpart in the reference, whose guard predicate
  * is not exact): 0 (default) the reference's predicate and skip rules,

@@ -126,8 +126,8 @@ def test_fused_loop_matches_oracle(torch_cuda, oracle_lib, level):
 @pytest.mark.parametrize("small_stack", [0, 1])
 def test_guard_frontier_matches_oracle(torch_cuda, oracle_lib, small_stack):
     """Undo-heavy input (offset sheets) through the fused loop.  With the
-    32-entry guard frontier almost every wave overflows and walks subtrees
-    by escape links; both frontier sizes give the oracle's result."""
+    32-entry guard frontier almost every wave fills it and pops few entries a
+    step, down to one; both frontier sizes give the oracle's result."""
     from pamo_amd import synth, _hip
     from pamo_amd.pamo import simplify_device
     torch = torch_cuda
